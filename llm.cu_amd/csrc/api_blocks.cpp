@@ -205,7 +205,7 @@ static int head_ce_packed(hipStream_t st, const _Float16* hidden, const _Float16
   gemm_finalize_segments(d);
   d.M = T;
   d.K = V;
-  d.split = gemm_pick_split(T, H, V, 64);
+  d.split = gemm_pick_split(T, H, V, 64, false);
   TRY_ARG((size_t)d.split * T * H <= part_elems, "head_ce: partial workspace");
   d.C = part;
   d.ldc = H;
@@ -261,7 +261,7 @@ int llmt_lm_head_ce(const void* hidden, const void* W, const int* targets, int T
   float2* stats = tmp.get<float2>((size_t)T * ce_stats_per_row(V));
   float* rows = tmp.get<float>(T);
   float* lse = tmp.get<float>(T);
-  const size_t pe = (size_t)gemm_pick_split(T, H, V, 64) * T * H;
+  const size_t pe = (size_t)gemm_pick_split(T, H, V, 64, false) * T * H;
   float* part = tmp.get<float>(pe);
   TRY_ARG(E && ET && logits && g16 && stats && rows && lse && part,
           "llmt_lm_head_ce: out of memory");

@@ -173,14 +173,16 @@ int Ctx::init() {
   TRY_HIP(hipMemset(tgt_buf, 0, T * sizeof(int)));
 
   // split-K partials: the largest split * M * N over every GEMM of the step
-  const int shapes[9][2] = {{NT + 3 * kRank, H}, {H + kRank, Q}, {2 * I, H}, {H, I},
-                            {H, V},              {I, H},         {H, 2 * I}, {Q + kRank, H},
-                            {H + 3 * kRank, NT}};
+  // (the gate/up GEMM runs unsplit; the head's dX is fp16 whatever the layers are)
+  const int shapes[8][2] = {{NT + 3 * kRank, H}, {H + kRank, Q}, {H, I},         {H, V},
+                            {I, H},              {H, 2 * I},     {Q + kRank, H}, {H + 3 * kRank, NT}};
   part_elems = 0;
   for (int b = 1; b <= maxB; ++b) {
     const int M = rows(b);
     for (auto& sh : shapes) {
-      const int split = gemm_split_col(M, sh[0], sh[1]) ? 2 : gemm_pick_split(M, sh[0], sh[1], 64);
+      const bool i8 = wfmt == LLMT_WEIGHTS_I8 && &sh != &shapes[3];
+      const int split =
+          gemm_split_col(M, sh[0], sh[1], i8) ? 2 : gemm_pick_split(M, sh[0], sh[1], 64, i8);
       const size_t e = (size_t)split * M * sh[0];
       if (e > part_elems) part_elems = e;
     }

@@ -214,9 +214,8 @@ struct Ctx {
   // C = A B^T over the segments.  direct: split 1 into `direct` (ld ldc).
   // Otherwise the fp32 split-K partials land in `part` and *out describes
   // them; the consuming row epilogue sums them in split order.  glu16: the
-  // fused SwiGLU epilogue (split 1, gemm_glu_ok shapes only) writes [gate |
-  // up] fp16 [M, N] to gu16 and fp16(silu(gate) * up) [M, N / 2] to glu16
-  // (direct and ldc unused).
+  // fused SwiGLU epilogue (split 1) writes [gate | up] fp16 [M, N] to gu16
+  // and fp16(silu(gate) * up) [M, N / 2] to glu16 (direct and ldc unused).
   // rowstats (direct only): also the per-(row, column tile) softmax pairs
   // (GemmArgs::rowstats); *tiles gets their row width.  last_wave_split:
   // the consumer reads the partials through load_row, so an unsplit

@@ -11,24 +11,19 @@
 // kernels (src/kernels/matmul.cu:8-138): matmul_forward (NT), matmul_nn
 // (dX) and, for LoRA, matmul_tn.
 //
-// Work decomposition.  The step's activations have few rows (T = 128 at the
-// headline shape), so every weight element is used T times: the kernel is
-// HBM-bound on the weight stream.  B operands are stored fragment-packed
-// (packed_index in common.h): each wave streams its NF*16 weight rows as
-// contiguous 1 KB loads straight into MFMA operand registers through a
-// register ring (RING - 1 k-steps of 32 ahead).  The A tile of all MF*16 rows
-// is staged through LDS in 64-wide K chunks (double-buffered, in MFMA
-// fragment order so every ds_read_b128 is a contiguous conflict-free 1 KB)
-// and shared by the NW waves; the next chunk's A loads are issued a chunk of
-// MFMA work before they are stored.  K is split across workgroups (split-K)
-// so a launch fills the CUs; the fp32 split partials are summed in split
-// order by the consuming row epilogue (deterministic), and the standalone
-// GEMM entry points reduce them with reduce_lora.  Measured on MI355X
-// (per-workgroup timestamps): the in-loop weight stream runs at 2.6-3.8 TB/s,
-// and each launch pays ~5 us of fixed latency (launch, the first A/B round
-// trip, the partial stores), which four-wave 128-column tiles at about 3/4 of
-// a workgroup per CU balance best against the partial traffic; deeper B
-// rings and A prefetch distances measured no faster.
+// Kernels.  B operands are stored fragment-packed (packed_index in common.h),
+// so an MFMA fragment of B is one contiguous 1 KB (int8: 512 B) wherever it
+// is read from.
+//   gemm_ring_kernel  M up to about a thousand rows, any M % 16 == 0: 16 MR x
+//                     16 NB tiles fed by LDS DMA, K split over workgroups so
+//                     that a launch fills the CUs; the fp32 split partials
+//                     are summed in split order by the consuming row
+//                     epilogue (deterministic), and the standalone GEMM entry
+//                     points reduce them with reduce_lora
+//   gemm_dma_kernel   many rows: 256 x 256 tiles
+//   gemm_nt_kernel    what the two do not take (K % 64 != 0, several int8
+//                     segments): B streamed into registers, A through LDS
+// gemm_plan picks the kernel, the tile and the split from a cost model.
 #include <math.h>
 #include <stdlib.h>
 #include <type_traits>
@@ -69,14 +64,14 @@ __device__ __forceinline__ half8 i8x8_to_h8(u32x2 raw) {
   return h - (_Float16)1152.0f;
 }
 
-// One workgroup: output tile (MF*16) x (NW*NF*16) over k-steps [s0, s1) of
-// its split.  The A tile goes through LDS in chunks of CHS k-steps (two LDS
-// buffers); chunk c + ADIST is loaded into registers while chunk c is
-// multiplied, so an A load has ADIST chunks of MFMA work to land.  B
-// fragments stream through a RING-slot register ring, RING - 1 k-steps
-// ahead.  The main loop body covers UC chunks so that every LDS buffer,
-// A register set and ring slot index is a compile-time constant.  Chunks
-// and k-steps past the end are clamped loads multiplied by zeroed B
+// Register-staged kernel.  One workgroup: output tile (MF*16) x (NW*NF*16)
+// over k-steps [s0, s1) of its split.  The A tile goes through LDS in chunks
+// of CHS k-steps (two LDS buffers); chunk c + ADIST is loaded into registers
+// while chunk c is multiplied, so an A load has ADIST chunks of MFMA work to
+// land.  B fragments stream through a RING-slot register ring, RING - 1
+// k-steps ahead.  The main loop body covers UC chunks so that every LDS
+// buffer, A register set and ring slot index is a compile-time constant.
+// Chunks and k-steps past the end are clamped loads multiplied by zeroed B
 // fragments (branch-free: the compiler then keeps the newer loads in flight
 // across every wait).  With I8 a segment may be int8 (dequantised in
 // registers at MFMA time, optionally times a per-k scale loaded alongside).
@@ -289,7 +284,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(const GemmArgs g) {
   }
 }
 
-constexpr int BM = 256, BCH = 2;  // large-tile rows; k-steps per big_tiles() K quantum
+constexpr int BM = 256;  // large-tile rows
 
 // LDS-DMA kernel for the large-M GEMMs: the operands go from global memory
 // straight into LDS (global_load_lds: lane l's 16 bytes land at offset 16 l
@@ -345,7 +340,7 @@ __global__ __launch_bounds__(WNN * 128) void gemm_dma_kernel(const GemmArgs g, i
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WNN, wn = wave % WNN;
-  const int ntn = (g.N + 255) / 256, ntm = g.M / 256;
+  const int ntn = (g.N + 255) / 256, ntm = (g.M + 255) / 256;
   int t = blockIdx.x, sidx = blockIdx.y, nsp = g.split, tn0 = 0, ntn_r = ntn;
   if (g.split_col > 0) {
     // column tiles [0, ntc) unsplit (workgroups 0 .. ntc ntm - 1), then the
@@ -379,9 +374,13 @@ __global__ __launch_bounds__(WNN * 128) void gemm_dma_kernel(const GemmArgs g, i
 
   // issue pointers: wave w moves A fragments FPW w .. and B fragments FPW w ..
   // of every chunk (plus, with KS, k-scales through lane 0 of waves 0-3)
-  const _Float16* asrc =
-      g.A + (long long)(m0 + wave * FPW * 16 + (lane & 15)) * g.lda + (lane >> 4) * 8;
-  const long long astep = 16LL * g.lda;
+  // (A fragments past M re-read the last one; their rows are not stored)
+  const int mfr = (g.M - m0) >> 4;  // 16-row fragments with rows of A
+  const _Float16* asrc[FPW];
+#pragma unroll
+  for (int j = 0; j < FPW; ++j)
+    asrc[j] = g.A + (long long)(m0 + min(wave * FPW + j, mfr - 1) * 16 + (lane & 15)) * g.lda +
+              (lane >> 4) * 8;
   const BSeg& sg = g.seg[0];
   constexpr int ES = I8 ? 1 : 2;
   const char* bsrc = (const char*)sg.ptr + (long long)lane * 16;  // lanes < 32 for int8
@@ -408,7 +407,7 @@ __global__ __launch_bounds__(WNN * 128) void gemm_dma_kernel(const GemmArgs g, i
     char* st = smem + (c % S) * SBYTES;
 #pragma unroll
     for (int j = 0; j < FPW; ++j)
-      dma16(asrc + j * astep + cc * KSTEP, reinterpret_cast<_Float16*>(st + (wave * FPW + j) * 1024));
+      dma16(asrc[j] + cc * KSTEP, reinterpret_cast<_Float16*>(st + (wave * FPW + j) * 1024));
 #pragma unroll
     for (int j = 0; j < FPW; ++j) {
       const char* src = bsrc + boff[j] + (long long)cc * 512 * ES;
@@ -549,7 +548,8 @@ __global__ __launch_bounds__(WNN * 128) void gemm_dma_kernel(const GemmArgs g, i
     }
     const int col0 = (tn * 8 + ((wn * NFR) >> 1)) * 16 + (lane & 15);
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 8; ++i) {
+      if (wm * 8 + i >= mfr) break;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const long long row = m0 + wm * 128 + i * 16 + (lane >> 4) * 4 + v;
@@ -563,18 +563,21 @@ __global__ __launch_bounds__(WNN * 128) void gemm_dma_kernel(const GemmArgs g, i
           arow[16 * jj] = (_Float16)(gt * sigmoid_rcp(gt) * up);
         }
       }
+    }
     return;
   }
   if constexpr (TL) {
     if (has_tail) {
       const int col = tail_c0 + tn * 16 + (lane & 15);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 2; ++j) {
+        if (wm * 8 + 2 * wn + j >= mfr) continue;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int row = m0 + wm * 128 + (2 * wn + j) * 16 + (lane >> 4) * 4 + v;
           C[(long long)row * g.ldc + col] = acc_t[j][v];
         }
+      }
     }
   }
   float scj[NFR];
@@ -594,12 +597,14 @@ __global__ __launch_bounds__(WNN * 128) void gemm_dma_kernel(const GemmArgs g, i
   for (int j = 0; j < NFR; ++j) {
     if (n0 + wn * WC + j * 16 >= g.N) continue;  // N % 16 == 0: whole fragments
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 8; ++i) {
+      if (wm * 8 + i >= mfr) break;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         float* const Cr = Cw + (long long)(i * 16 + v) * g.ldc + j * 16;
         Cr[lo] = acc[i][j][v] * scj[j];
       }
+    }
   }
   if (g.rowstats) {
     // each row's (max, sum exp) over the tile's 256 columns: a wave's pair
@@ -621,7 +626,7 @@ __global__ __launch_bounds__(WNN * 128) void gemm_dma_kernel(const GemmArgs g, i
         if ((lane & 15) == 0) sh[(wm * 128 + i * 16 + (lane >> 4) * 4 + v) * WNN + wn] = p;
       }
     __syncthreads();
-    for (int r = tid; r < 256; r += WNN * 128) {
+    for (int r = tid; r < 256 && r < 16 * mfr; r += WNN * 128) {
       float m = -INFINITY, s = 0.f;
 #pragma unroll
       for (int w = 0; w < WNN; ++w) softmax_merge(m, s, sh[r * WNN + w].x, sh[r * WNN + w].y);
@@ -630,27 +635,39 @@ __global__ __launch_bounds__(WNN * 128) void gemm_dma_kernel(const GemmArgs g, i
   }
 }
 
-// Skinny fp16 kernel fed by DMA (the T = 128 training step): a 128 x BN
-// output tile (BN = 16 NB) per workgroup of eight waves, K split over
-// blockIdx.x (the fastest grid index) in 64-wide stages.  Wave w = 4 kg + wr computes rows
-// 32 wr .. 32 wr + 31 x all BN columns over k half kg (32 of the 64) of
-// every stage, so each SIMD runs two waves whose LDS reads and MFMAs
-// interleave; the two halves' sums meet in LDS at the end (kg 1 hands its
-// accumulators to kg 0, which stores).  Both operands move global -> LDS with
-// buffer loads that have an LDS destination, 16 bytes a lane: A as 128-byte
-// row pieces (8 lanes a row, so each stage touches every A cache line once;
-// the 16-byte pieces are XOR-swizzled by row so the fragment reads are
-// bank-conflict free; wave w moves rows 16 w .. 16 w + 15), B as the 1 KB
-// fragment of k half kg of each fragment-packed row block (row blocks wr,
-// wr + 4, ..; one wave-uniform descriptor per row block, the stage offset a
-// scalar).  An S-stage ring (A 16 KB + B 2 NB KB a stage) keeps S - 1 stages
-// in flight; stage c is waited for with an explicit vmcnt (the loads of later
-// stages stay in flight) and a plain barrier, the last S - 1 stages wait for
-// all.  A wave reads all fragments of its stage half before its MFMAs.
-// Measured on MI355X (C2 shapes, back to back): 5-15% below the four-wave
-// form with the same tiles; the partial tiles and the first round trip set
-// the rest of the cost at this M.  Columns past N load row block 0 of the
-// first segment (in bounds) and are not stored.
+// Stage-ring kernel: M up to about a thousand rows (a training step of one to
+// a few sequences), fp16 or int8 weights, any M % 16 == 0.  A workgroup of
+// eight waves owns 16 MR rows x 16 NB columns, K split over workgroups.
+//
+// What bounds it: up to M = 128 the weight stream and the fixed costs of a
+// launch (about 5 us: the first round trip, the partial stores), above that
+// the LDS: a 64-wide stage of a 128 x 128 tile is 512 cycles of MFMA a SIMD
+// but 96 KB of LDS traffic (64 KB of fragment reads, 32 KB of DMA), 768
+// cycles at 128 B/clk; with the operands re-read from L2 (no fresh memory
+// traffic) a stage takes 0.41 us, with them 0.58.  Hence the wave layout: two
+// groups of four waves take one k half of every stage each (their sums meet
+// in LDS at the end), so a wave covers 64 x (8 NB) with half the fragment
+// reads per MFMA that eight waves over the whole tile would need, and the
+// fragments are read one stage ahead into registers (an A register is
+// refilled right after its last MFMA), so the reads run beside the MFMAs.
+//
+// Both operands move global -> LDS with buffer loads that have an LDS
+// destination, 16 bytes a lane: A as 128-byte row pieces (the 16-byte pieces
+// XOR-swizzled by row so the fragment reads are bank-conflict free; rows past
+// M lie outside the descriptor and arrive as zeros), B as whole fragments
+// (one wave-uniform descriptor per row block, the stage offset a scalar).
+// int8 rows stay bytes in LDS and are dequantised after the fragment read.
+// An S-stage ring keeps S - 1 stages in flight; a stage is waited for with an
+// explicit vmcnt (younger stages stay in flight) and a plain barrier.
+//
+// Measured on MI355X (cold operands, replayed in a graph) against the
+// register-staged kernel, which streams all weights once per 16 rows where M
+// is not a multiple of 32: M = 624 fp16 gate/up 180 -> 44 us, gate/up dX 196
+// -> 43 us; M = 128 int8 (which that kernel also took) gate/up 111 -> 20 us,
+// Q/K/V 60 -> 11 us; M = 512 fp16 against the 128 x 64 tiles this kernel
+// replaced: gate/up 45 -> 36 us, its dX 43 -> 38 us, O 15 -> 14 us; the
+// logits of M = 128 (128 x 256 tiles, 622 MB of weights) 172 -> 162 us, their
+// dX 135 -> 130 us.
 constexpr int kRsrcWord3 = 0x00020000;  // raw buffer, 32-bit data format
 typedef __attribute__((address_space(3))) void lds_void_t;
 
@@ -664,175 +681,364 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, unsig
 // slot of 16-byte piece p (0..7) of A row r in a stage
 __device__ __forceinline__ int a_slot(int r, int p) { return p ^ ((r >> 1) & 7); }
 
-// GLU: fragment f of the tile is the gate (f even) or up (f odd) row block of
-// the same 16 columns (split 1, one segment, N = 2 glu); the epilogue writes
-// [gate | up] and fp16(silu(gate) * up) as the large-tile kernel's.
-template <int S, int NB, bool GLU = false>
-__global__ __launch_bounds__(512) void gemm_skinny_kernel(const GemmArgs g) {
-  constexpr int AB = 16384;                  // A bytes per stage
-  constexpr int SB = AB + NB * 2048;         // bytes per stage
-  constexpr int BPW = (NB + 3) / 4;          // B row blocks a wave moves at most (wr, wr + 4, ..)
-  static_assert(4 * 2 * NB * 64 * 16 <= S * SB, "k-half exchange fits in the ring");
-  __shared__ __attribute__((aligned(1024))) char smem[S * SB];
+// vmcnt(rem * OPS): the rem youngest stages (OPS DMA issues of this wave
+// each) may still be in flight, everything older has landed.
+template <int OPS, int MAXREM>
+__device__ __forceinline__ void wait_stages(int rem) {
+  [&]<int... R>(std::integer_sequence<int, R...>) LLMT_INLINE {
+    (void)((rem == R ? (wait_vm<R * OPS>(), true) : false) || ...);
+  }(std::make_integer_sequence<int, MAXREM + 1>{});
+}
+
+// Shape of a stage-ring tile: S stages, MR x NB fragments (16 rows / columns
+// each) a workgroup, WR x (4 / WR) waves over them and two groups of four
+// waves over the k halves of a stage.
+template <int S_, int MR_, int NB_, int WR_, bool I8_>
+struct RingCfg {
+  static constexpr int S = S_, MR = MR_, NB = NB_, WR = WR_, WC = 4 / WR_;
+  static constexpr bool I8 = I8_;
+  static constexpr int FR = MR / WR, FC = NB / WC;  // fragments a wave
+  // Fragments one stage ahead in registers, where a wave has enough MFMAs a
+  // stage to cover the reads; the 32-row waves of the narrow 128-row tiles
+  // (8 MFMAs a stage, HBM-bound) read a stage when it lands instead: at
+  // M = 128 the O GEMM 7.5 -> 7.2 us, gate/up dX 17.6 -> 17.2.
+  static constexpr bool AHEAD = WR < 4;
+  static constexpr int AB = MR * 2048;              // A bytes a stage
+  static constexpr int BB = NB * (I8 ? 1024 : 2048);
+  static constexpr int KSB = I8 ? 256 : 0;          // per-k scales of a stage (int8)
+  static constexpr int SB = AB + BB + KSB;
+  static constexpr int XCH = 8 * (FR / 2) * FC * 1024;  // k-half exchange
+  static constexpr int LDS = S * SB > XCH ? S * SB : XCH;
+  static_assert(MR % WR == 0 && NB % WC == 0 && FR % 2 == 0, "whole fragments a wave");
+  static_assert(LDS <= 160 * 1024, "ring fits the LDS");
+};
+
+// One output tile over stages [c0, c1) of 64 k.  B8: this tile's B rows are
+// int8 (a GEMM with int8 weights has its fp16 LoRA rows in tiles of their
+// own, half as many fragments wide so that they take the same LDS).
+template <class C, bool B8, bool KS, bool GLU>
+__device__ __forceinline__ void ring_tile(const GemmArgs& g, char* smem, int seg, int f0, int ct,
+                                          int rb, int sp, int ntn) {
+  constexpr int S = C::S, MR = C::MR, FR = C::FR;
+  constexpr bool HALF = C::I8 && !B8;              // an fp16 tile of an int8 GEMM
+  constexpr int NB = HALF ? C::NB / 2 : C::NB;
+  constexpr int FC = HALF ? (C::FC + 1) / 2 : C::FC;
+  constexpr int BK = B8 ? 512 : 1024;              // bytes of a B fragment (32 k)
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wr = wave & 3, kg = wave >> 2;
-  // grid = (split, column tile, row tile): the split is the fastest index,
-  // so workgroup b (on XCD b % 8) of split s reads A's K slice s, and that
-  // slice reaches only the XCDs running split s (one of eight at split 8 or
-  // 16) instead of every XCD's L2 -- the lm_head dX at C2 had fetched its
-  // 39 MB A operand eight times over
-  const int ct = blockIdx.y, sp = blockIdx.x;
-  const int n0 = ct * (NB * 16), m0 = blockIdx.z * 128;
-  const int ksteps = g.K / KSTEP;
-  const int nst = g.K / 64;
+  const int kg = wave >> 2, wq = wave & 3, wr = wq % C::WR, wc = wq / C::WR;
+  const int m0 = rb * MR * 16;
+  const int ksteps = g.K / KSTEP, nst = g.K / 64;
   const int c0 = (int)((long long)sp * nst / g.split);
   const int c1 = (int)((long long)(sp + 1) * nst / g.split);
+  const BSeg& sg = g.seg[seg];
 
-  // A: wave w moves rows 16 w .. 16 w + 15 (two 1 KB pieces of 8 rows)
+  // A: 2 MR pieces of 8 rows x 128 bytes a stage, wave w moves pieces
+  // APW w ..; rows past M lie outside the descriptor and arrive as zeros
+  constexpr int APW = (2 * MR + 7) / 8;
+  const int naw = 2 * MR >= 8 ? APW : (wave < 2 * MR ? 1 : 0);
   const __amdgpu_buffer_rsrc_t ars =
-      make_rsrc(g.A + (long long)m0 * g.lda, (unsigned)(128u * g.lda * 2u));
-  unsigned aoff[2];
+      make_rsrc(g.A + (long long)m0 * g.lda, (unsigned)min(MR * 16, g.M - m0) * (unsigned)g.lda * 2u);
+  unsigned aoff[APW];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = 8 * (2 * wave + i) + (lane >> 3);
+  for (int i = 0; i < APW; ++i) {
+    const int r = 8 * (APW * wave + i) + (lane >> 3);
     aoff[i] = (unsigned)((r * g.lda + a_slot(r, lane & 7) * 8) * 2);
   }
-  const int nbw = (NB - wr + 3) / 4;  // row blocks this wave moves
+  // B: fp16 row blocks as two 1 KB fragments (k halves), wave w moves half
+  // w / 4 of row blocks w % 4, w % 4 + 4, ..; int8 row blocks as one 1 KB
+  // piece, wave w moves row blocks w, w + 8, ..
+  constexpr int BST = B8 ? 8 : 4;
+  constexpr int BPW = (NB + BST - 1) / BST;
+  const int bw = B8 ? wave : wq;
+  const int nbw = (NB - bw + BST - 1) / BST;
   __amdgpu_buffer_rsrc_t brs[BPW];
 #pragma unroll
   for (int i = 0; i < BPW; ++i) {
+    const int f = min(bw + BST * i, NB - 1);
+    long long rbk;
     if constexpr (GLU) {
-      const int f = min(wr + 4 * i, NB - 1);
-      const long long rb = (f & 1) * (g.glu >> 4) + (long long)ct * (NB / 2) + (f >> 1);
-      brs[i] = make_rsrc((const _Float16*)g.seg[0].ptr + rb * ksteps * 512, (unsigned)(ksteps * 1024u));
-      continue;
+      const int pr = ct * (NB / 2) + (f >> 1);
+      rbk = (f & 1) * (g.glu >> 4) + (pr < (g.glu >> 4) ? pr : 0);
+      brs[i] = make_rsrc((const char*)sg.ptr + rbk * ksteps * BK, (unsigned)(ksteps * BK));
+    } else if constexpr (C::I8) {
+      rbk = f0 + f < (sg.rows >> 4) ? f0 + f : 0;
+      brs[i] = make_rsrc((const char*)sg.ptr + rbk * ksteps * BK, (unsigned)(ksteps * BK));
+    } else {  // fp16 tiles may straddle segments
+      const int nn = 16 * (f0 + f);
+      int s = 0;
+#pragma unroll
+      for (int q = 1; q < 4; ++q)
+        if (q < g.nseg && nn >= g.seg_start[q]) s = q;
+      rbk = nn < g.N ? (nn - g.seg_start[s]) >> 4 : 0;
+      brs[i] = make_rsrc((const char*)g.seg[s].ptr + rbk * ksteps * BK, (unsigned)(ksteps * BK));
     }
-    const int nn = n0 + 16 * min(wr + 4 * i, NB - 1);
-    int s = 0;
-#pragma unroll
-    for (int q = 1; q < 4; ++q)
-      if (q < g.nseg && nn >= g.seg_start[q]) s = q;
-    const long long rb16 = nn < g.N ? (nn - g.seg_start[s]) >> 4 : 0;
-    brs[i] = make_rsrc((const _Float16*)g.seg[s].ptr + rb16 * ksteps * 512, (unsigned)(ksteps * 1024u));
   }
+  const bool ksw = KS && B8 && wave == 7;  // wave 7 also moves the stage's 64 k scales
+  const __amdgpu_buffer_rsrc_t krs = make_rsrc(KS && B8 ? sg.kscale : nullptr,
+                                               KS && B8 ? (unsigned)(g.K * 2) : 0u);
   auto issue = [&](int c) LLMT_INLINE {
-    char* st = smem + (c % S) * SB;
+    char* st = smem + (c % S) * C::SB;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) buffer_lds16(ars, st + (2 * wave + i) * 1024, aoff[i], c * 128u);
+    for (int i = 0; i < APW; ++i)
+      if (i < naw) buffer_lds16(ars, st + (APW * wave + i) * 1024, aoff[i], c * 128u);
 #pragma unroll
     for (int i = 0; i < BPW; ++i)
-      if (i < nbw)
-        buffer_lds16(brs[i], st + AB + ((wr + 4 * i) * 2 + kg) * 1024, lane * 16u + kg * 1024u,
-                     c * 2048u);
-  };
-  // stage c complete: only the later stages' loads (2 + nbw a stage) may be pending
-  auto wait_stage = [&]() LLMT_INLINE {
-    switch (nbw) {
-      case 0: wait_vm<(S - 2) * 2>(); break;
-      case 1: wait_vm<(S - 2) * 3>(); break;
-      default: wait_vm<(S - 2) * 4>(); break;
+      if (i < nbw) {
+        if constexpr (B8)
+          buffer_lds16(brs[i], st + C::AB + (bw + 8 * i) * 1024, lane * 16u, c * 1024u);
+        else
+          buffer_lds16(brs[i], st + C::AB + ((bw + 4 * i) * 2 + kg) * 1024, lane * 16u + kg * 1024u,
+                       c * 2048u);
+      }
+    if constexpr (KS && B8) {
+      if (ksw && lane < 8) buffer_lds16(krs, st + C::AB + C::BB, lane * 16u, c * 128u);
     }
   };
-  // A fragment reads: row 16 (2 wr + i) + c of the stage, k half kg, halves 8 g..
-  const int arow0 = 16 * (2 * wr) + (lane & 15);
-  int aread[2];
+  // DMA issues a stage of this wave: OMIN .. OMAX
+  constexpr int OMIN = (2 * MR >= 8 ? APW : 0) + NB / BST;
+  constexpr int OMAX = APW + BPW + (KS && B8 ? 1 : 0);
+  const int nops = naw + nbw + (ksw ? 1 : 0);
+  auto wait_rem = [&](int rem) LLMT_INLINE {
+    [&]<int... O>(std::integer_sequence<int, O...>) LLMT_INLINE {
+      (void)((OMIN == OMAX || nops == OMIN + O ? (wait_stages<OMIN + O, S - 1>(rem), true) : false) || ...);
+    }(std::make_integer_sequence<int, OMAX - OMIN + 1>{});
+  };
+
+  int aread[FR];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = arow0 + 16 * i;
+  for (int i = 0; i < FR; ++i) {
+    const int r = 16 * (wr * FR + i) + (lane & 15);
     aread[i] = r * 128 + a_slot(r, 4 * kg + (lane >> 4)) * 16;
   }
-
-  floatx4 acc[2][NB];
+  floatx4 acc[FR][FC];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < FR; ++i)
 #pragma unroll
-    for (int j = 0; j < NB; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  for (int c = c0; c < c1 && c < c0 + S - 1; ++c) issue(c);
-  for (int c = c0; c < c1; ++c) {
-    if (c + S - 1 < c1) {
-      wait_stage();
-      __builtin_amdgcn_s_barrier();
-      issue(c + S - 1);
-    } else {
-      wait_vm<0>();
-      __builtin_amdgcn_s_barrier();
+    for (int j = 0; j < FC; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  half8 a[FR], b[FC], bn[FC], ksn;
+  u32x2 b8[FC];
+  auto read_a = [&](const char* st, int i) LLMT_INLINE {
+    a[i] = *reinterpret_cast<const half8*>(st + aread[i]);
+  };
+  auto read_b = [&](const char* st) LLMT_INLINE {
+    if constexpr (KS && B8)
+      ksn = *reinterpret_cast<const half8*>(st + C::AB + C::BB + kg * 64 + (lane >> 4) * 16);
+#pragma unroll
+    for (int j = 0; j < FC; ++j) {
+      const int f = min(wc * FC + j, NB - 1);
+      if constexpr (B8)
+        b8[j] = *reinterpret_cast<const u32x2*>(st + C::AB + f * 1024 + kg * 512 + lane * 8);
+      else
+        bn[j] = *reinterpret_cast<const half8*>(st + C::AB + (f * 2 + kg) * 1024 + lane * 16);
     }
+  };
+  auto take_b = [&]() LLMT_INLINE {
+#pragma unroll
+    for (int j = 0; j < FC; ++j) {
+      if constexpr (B8) {
+        b[j] = i8x8_to_h8(b8[j]);
+        if constexpr (KS) b[j] = b[j] * ksn;
+      } else {
+        b[j] = bn[j];
+      }
+    }
+  };
+
+  if constexpr (C::AHEAD) {
+    for (int c = c0; c < c1 && c < c0 + S; ++c) issue(c);
+    wait_rem(min(S, c1 - c0) - 1);
+    __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    const char* st = smem + (c % S) * SB;
-    half8 a[2], b[NB];
+    {
+      const char* st = smem + (c0 % S) * C::SB;
+      read_b(st);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) a[i] = *reinterpret_cast<const half8*>(st + aread[i]);
+      for (int i = 0; i < FR; ++i) read_a(st, i);
+      take_b();
+    }
+    for (int c = c0; c < c1 - 1; ++c) {
+      // stage c + 1 landed, and this wave's reads of stage c returned: after
+      // the barrier slot c % S takes stage c + S
+      wait_rem(min(S - 2, c1 - 2 - c));
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (c + S < c1) issue(c + S);
+      const char* st = smem + ((c + 1) % S) * C::SB;
+      read_b(st);
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
-      b[j] = *reinterpret_cast<const half8*>(st + AB + (j * 2 + kg) * 1024 + lane * 16);
+      for (int i = 0; i < FR; ++i) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
+        for (int j = 0; j < FC; ++j) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
+        read_a(st, i);
+      }
+      // B reads first, then each row's MFMAs and the read that refills its A
+      // register
+      __builtin_amdgcn_sched_group_barrier(0x100, FC + (KS && B8 ? 1 : 0), 0);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
-    asm volatile("" ::: "memory");
+      for (int i = 0; i < FR; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, FC, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      take_b();
+      asm volatile("" ::: "memory");
+    }
+#pragma unroll
+    for (int i = 0; i < FR; ++i)
+#pragma unroll
+      for (int j = 0; j < FC; ++j) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
+  } else {
+    for (int c = c0; c < c1 && c < c0 + S - 1; ++c) issue(c);
+    for (int c = c0; c < c1; ++c) {
+      // stage c landed for every wave, and every wave is past its reads of
+      // stage c - 1, whose slot takes stage c + S - 1
+      wait_rem(min(S - 2, c1 - 1 - c));
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (c + S - 1 < c1) issue(c + S - 1);
+      const char* st = smem + (c % S) * C::SB;
+      read_b(st);
+#pragma unroll
+      for (int i = 0; i < FR; ++i) read_a(st, i);
+      take_b();
+#pragma unroll
+      for (int j = 0; j < FC; ++j)
+#pragma unroll
+        for (int i = 0; i < FR; ++i) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
+      asm volatile("" ::: "memory");
+    }
   }
 
-  // k half 1 hands its sums to k half 0 (the ring is free: every load has
-  // landed and every wave is past its last fragment read)
+  // the two k halves meet: each wave hands the other group's half of its row
+  // fragments over through the (now free) ring, adds what it gets to its own
+  // half and stores it
+  constexpr int FH = FR / 2;
   wait_vm<0>();
   __syncthreads();
-  floatx4* xch = reinterpret_cast<floatx4*>(smem) + wr * (2 * NB * 64);
-  if (kg == 1) {
+  floatx4* xch = reinterpret_cast<floatx4*>(smem) + (size_t)wq * (2 * FH * FC * 64);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+  for (int h = 0; h < FH; ++h)
 #pragma unroll
-      for (int j = 0; j < NB; ++j) xch[(i * NB + j) * 64 + lane] = acc[i][j];
-  }
+    for (int j = 0; j < FC; ++j)
+      xch[(((1 - kg) * FH + h) * FC + j) * 64 + lane] = kg ? acc[h][j] : acc[FH + h][j];
   __syncthreads();
-  if (kg == 1) return;
+  floatx4 o[FH][FC];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int h = 0; h < FH; ++h)
 #pragma unroll
-    for (int j = 0; j < NB; ++j) acc[i][j] += xch[(i * NB + j) * 64 + lane];
+    for (int j = 0; j < FC; ++j)
+      o[h][j] = (kg ? acc[FH + h][j] : acc[h][j]) + xch[((kg * FH + h) * FC + j) * 64 + lane];
+  const int row0 = m0 + (wr * FR + kg * FH) * 16;  // first row of this wave's half
 
-  float* C = g.C + (long long)sp * g.split_stride;
   if constexpr (GLU) {
-    const _Float16* cs = g.seg[0].colscale;
+    const _Float16* cs = sg.colscale;
 #pragma unroll
-    for (int jj = 0; jj < NB / 2; ++jj) {
-      const int col = (ct * (NB / 2) + jj) * 16 + (lane & 15);
-      const float sg = cs ? (float)cs[col] : 1.0f, su = cs ? (float)cs[g.glu + col] : 1.0f;
+    for (int jj = 0; jj < FC / 2; ++jj) {
+      const int pr = ct * (NB / 2) + wc * (FC / 2) + jj;
+      if (pr >= (g.glu >> 4)) continue;
+      const int col = pr * 16 + (lane & 15);
+      const float sgt = cs ? (float)cs[col] : 1.0f, su = cs ? (float)cs[g.glu + col] : 1.0f;
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int h = 0; h < FH; ++h) {
+        if (row0 + 16 * h >= g.M) continue;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const long long row = m0 + (2 * wr + i) * 16 + (lane >> 4) * 4 + v;
-          const float gt = acc[i][2 * jj][v] * sg, up = acc[i][2 * jj + 1][v] * su;
+          const long long row = row0 + 16 * h + (lane >> 4) * 4 + v;
+          const float gt = o[h][2 * jj][v] * sgt, up = o[h][2 * jj + 1][v] * su;
           g.gu16[row * (2LL * g.glu) + col] = (_Float16)gt;
           g.gu16[row * (2LL * g.glu) + g.glu + col] = (_Float16)up;
           g.glu16[row * g.ldglu + col] = (_Float16)(gt * sigmoid_rcp(gt) * up);
         }
+      }
     }
     return;
   }
+  float* Cp = g.C + (long long)sp * g.split_stride;
+  const int n0 = (C::I8 ? g.seg_start[seg] : 0) + 16 * f0;  // first column of the tile
+  const int nend = C::I8 ? g.seg_start[seg] + sg.rows : g.N;
   // a wave-uniform row base plus one 32-bit lane offset for every store
   const int lo = (lane >> 4) * 4 * g.ldc + (lane & 15);
-  float* const Cw = C + (long long)(m0 + 2 * wr * 16) * g.ldc + n0;
+  float* const Cw = Cp + (long long)row0 * g.ldc;
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
-    const int nn = n0 + 16 * j;
-    if (nn >= g.N) continue;
-    int s = 0;
+  for (int j = 0; j < FC; ++j) {
+    const int nn = n0 + 16 * (wc * FC + j);
+    if (nn >= nend || wc * FC + j >= NB) continue;
+    if constexpr (B8) {
+      const _Float16* cs = sg.colscale;
+      const float sc = cs ? (float)cs[nn - g.seg_start[seg] + (lane & 15)] : 1.0f;
 #pragma unroll
-    for (int q = 1; q < 4; ++q)
-      if (q < g.nseg && nn >= g.seg_start[q]) s = q;
-    const _Float16* cs = g.seg[s].colscale;
-    const int col = nn + (lane & 15);
-    const float sc = cs ? (float)cs[col - g.seg_start[s]] : 1.0f;
+      for (int h = 0; h < FH; ++h) o[h][j] *= sc;
+    }
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int h = 0; h < FH; ++h) {
+      if (row0 + 16 * h >= g.M) continue;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        float* const Cr = Cw + (long long)(i * 16 + v) * g.ldc + 16 * j;
-        Cr[lo] = acc[i][j][v] * sc;
+        float* const Cr = Cw + (long long)(16 * h + v) * g.ldc + nn;
+        Cr[lo] = o[h][j][v];
       }
+    }
+  }
+  if constexpr (!C::I8) {
+    if (g.rowstats) {
+      // each row's (max, sum exp) over the tile: a wave's pair over its
+      // columns from its 16-lane groups, the column waves merged in order
+      constexpr int WC = C::WC;
+      float2* sh = reinterpret_cast<float2*>(smem);  // [16 MR][WC]
+      __syncthreads();  // the exchange has been read
+#pragma unroll
+      for (int h = 0; h < FH; ++h)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          float x[FC];
+#pragma unroll
+          for (int j = 0; j < FC; ++j)
+            x[j] = n0 + 16 * (wc * FC + j) < nend ? o[h][j][v] : -INFINITY;
+          const float2 p = softmax_pair16<FC>(x);
+          if ((lane & 15) == 0)
+            sh[((wr * FR + kg * FH + h) * 16 + (lane >> 4) * 4 + v) * WC + wc] = p;
+        }
+      __syncthreads();
+      for (int r = threadIdx.x; r < MR * 16 && m0 + r < g.M; r += 512) {
+        float m = -INFINITY, s = 0.f;
+#pragma unroll
+        for (int w = 0; w < WC; ++w) softmax_merge(m, s, sh[r * WC + w].x, sh[r * WC + w].y);
+        g.rowstats[(long long)(m0 + r) * ntn + ct] = make_float2(m, s);
+      }
+    }
+  }
+}
+
+// Tile (row block, column tile, split) of linear workgroup id t.  One row
+// block: the split is fastest, so the K slices of a column tile spread over
+// the XCDs (workgroup t runs on XCD t % 8) while each XCD reads only the A
+// columns of its splits.  More: each XCD gets a contiguous run of tiles with
+// the row block fastest, so a B tile is fetched into one XCD's L2 and read
+// there by every row block.
+template <class C, bool KS, bool GLU>
+__global__ __launch_bounds__(512) void gemm_ring_kernel(const GemmArgs g, int nrb, int nct) {
+  __shared__ __attribute__((aligned(1024))) char smem[C::LDS];
+  int rb = 0, ct = blockIdx.y, sp = blockIdx.x;  // one row block: grid (split, column tile)
+  if (nrb > 1) {
+    int t = blockIdx.x;
+    const int n = gridDim.x, x = t & 7, q = n >> 3, r = n & 7;
+    t = x * q + min(x, r) + (t >> 3);
+    rb = t % nrb;
+    t /= nrb;
+    ct = t % nct;
+    sp = t / nct;
+  }
+  if constexpr (C::I8) {
+    const int nm = GLU ? nct : (g.seg[0].rows + C::NB * 16 - 1) / (C::NB * 16);
+    if (ct < nm) {
+      ring_tile<C, true, KS, GLU>(g, smem, 0, ct * C::NB, ct, rb, sp, nct);
+    } else if constexpr (!GLU) {
+      ring_tile<C, false, false, false>(g, smem, 1, (ct - nm) * (C::NB / 2), ct, rb, sp, nct);
+    }
+  } else {
+    ring_tile<C, false, false, GLU>(g, smem, 0, ct * C::NB, ct, rb, sp, nct);
   }
 }
 
@@ -1109,197 +1315,316 @@ void gemm_finalize_segments(GemmArgs& g) {
   g.N = s;
 }
 
-// Split-K factor: enough (column tiles x splits) workgroups for about one
-// per CU, without splits shorter than 4 k-steps of 32.  Fewer splits means
-// fewer fp32 partials to reduce.
-// DMA skinny kernel (fp16 weights, M % 128 == 0; LLMT_GEMM_SKINNY_STAGES = 0
-// selects the register-staged kernel).  Plan: 64-column tiles (48 when that
-// fills more of the GPU) and the most splits that keep the grid within one
-// wave of the 256 CUs (a second, partial wave costs more than the extra
-// partials); at least two 64-wide stages a split.  Wider tiles at the same
-// grid size write proportionally more fp32 partials and measured slower.  Very wide outputs with no split (the lm_head logits) keep the
-// register-staged kernel, measured faster there.  LLMT_GEMM_SKINNY_NB forces
-// the width for tuning.
+// Depth of the register-staged fallback: LLMT_GEMM_SKINNY_STAGES = 0 selects
+// it for fp16 M % 128 == 0; 3, 5 or 6 with LLMT_GEMM_SKINNY_NB (2, 3, 4, 6 or
+// 8 column fragments) force that ring for tests and tuning.
 static int skinny_stages() { return env_int("LLMT_GEMM_SKINNY_STAGES", 4); }
-struct SkinnyPlan {
-  int nb, split;
+
+// ------------------------------------------------------------------ plan
+// Every tile the library launches, with the modelled time of a launch in us:
+//   launch + waves (wave + stages (stage + fill f)) + part split M N / 1e6
+// waves: rounds of the 256 CUs that the workgroups take, f: how full they
+// are (a fuller chip shares L2 and HBM), stages: 64-wide K stages of a
+// workgroup.  Fitted on MI355X to 4,800 timings of the layer GEMMs of
+// Qwen3-1.7B (M = 16 .. 4096, cold random operands): mean error 4%, and the
+// tile and split picked from the model cost 0.6% over the best measured ones
+// on average, 7% at worst.
+enum { GK_NT = 0, GK_RING = 1, GK_BIG = 2 };
+struct TileCost {
+  int kind, i8, mr, nb;
+  float launch, wave, stage, fill, part;
 };
-static SkinnyPlan skinny_plan(int M, int N, int K) {
-  const int frags = (N + 15) / 16, mt = M / 128;
-  const int forced = env_int("LLMT_GEMM_SKINNY_NB", 0);
-  // Workgroups aimed for: one per CU, except that short reductions
-  // (K <= 4096) aim for 192, i.e. fewer K splits.  Each split is an fp32
-  // [M, N] partial that the row pass after the GEMM reads back, and at these
-  // K those partials come close to the weight bytes (7 splits of K = 2048:
-  // 0.9x); measured on the whole M = 128 training step, 5.23 -> 5.19 ms, with
-  // the GEMMs alone 0-8% slower.
-  const int target = K <= 4096 ? 192 : 256;
-  SkinnyPlan best{0, 0};
-  int best_w = 0;
-  // Very long reductions (the logits' dX, K = V): every column tile re-reads
-  // its K range of A, so 128-column tiles halve that traffic (163 -> 141 us
-  // at M = 128, N = 2048, K = 151936); elsewhere 64/48-column tiles.
-  const bool wide = K >= 32768;
-  for (int nb : {4, 3, 2, 6, 8}) {
-    if (!forced && (wide ? nb != 8 : (nb != 4 && nb != 3))) continue;
-    if (forced && nb != forced) continue;
-    const int tiles = (frags + nb - 1) / nb * mt;
-    int split = target / tiles;
-    if (split > K / 128) split = K / 128;
-    if (split < 1) split = 1;
-    const int w = tiles * split;
-    if (w <= target && w > best_w) {
-      best = {nb, split};
-      best_w = w;
+static const TileCost kTiles[] = {
+    {GK_RING, 0, 2, 4, 3.607f, 0.219f, 0.200f, 0.069f, 0.815f},
+    {GK_RING, 0, 2, 8, 2.544f, 1.642f, 0.275f, 0.162f, 0.633f},
+    {GK_RING, 0, 4, 4, 4.288f, 0.002f, 0.178f, 0.089f, 0.814f},
+    {GK_RING, 0, 4, 8, 2.784f, 1.773f, 0.292f, 0.166f, 0.579f},
+    {GK_RING, 0, 8, 3, 2.839f, 1.055f, 0.323f, 0.034f, 1.122f},
+    {GK_RING, 0, 8, 4, 3.067f, 0.888f, 0.342f, 0.062f, 1.058f},
+    {GK_RING, 0, 8, 8, 3.380f, 1.277f, 0.403f, 0.206f, 0.814f},
+    {GK_RING, 0, 8, 12, 4.222f, 1.775f, 0.520f, 0.270f, 0.679f},
+    {GK_RING, 0, 8, 16, 4.392f, 2.099f, 0.720f, 0.278f, 0.600f},
+    {GK_BIG, 0, 16, 16, 4.626f, 0.000f, 1.213f, 0.541f, 0.854f},
+    {GK_RING, 1, 2, 4, 3.686f, 0.000f, 0.249f, 0.000f, 0.748f},
+    {GK_RING, 1, 2, 8, 2.031f, 1.299f, 0.312f, 0.111f, 0.912f},
+    {GK_RING, 1, 4, 4, 2.147f, 1.397f, 0.349f, 0.021f, 0.924f},
+    {GK_RING, 1, 4, 8, 2.668f, 1.546f, 0.392f, 0.081f, 0.778f},
+    {GK_RING, 1, 8, 8, 3.108f, 1.488f, 0.470f, 0.113f, 0.695f},
+    {GK_RING, 1, 8, 12, 3.362f, 2.829f, 0.570f, 0.215f, 0.492f},
+    {GK_RING, 1, 8, 16, 3.915f, 2.049f, 0.759f, 0.179f, 0.599f},
+    {GK_BIG, 1, 16, 16, 4.076f, 1.263f, 1.343f, 0.403f, 0.791f},
+};
+struct GemmPlan {
+  int kind, mr, nb, split;
+};
+// What the GEMM asks of its tile besides the product.
+enum { GN_PLAIN = 0, GN_GLU = 1, GN_STATS = 2 };
+
+// The cheapest tile and split (fixed > 0: with that split) of a GEMM.  A
+// consumer reads every partial back (at 5.5 TB/s), and the row epilogues
+// issue 2, 4 or 8 partials as one round trip, other counts as several.
+// N counts a trailing LoRA segment (N % 64 rows); on 256 x 256 tiles it
+// rides along, with int8 weights it has column tiles of its own.
+static GemmPlan gemm_plan(int M, int N, int K, bool i8, int need, int fixed, int max_split) {
+  GemmPlan best{GK_NT, 0, 0, 0};
+  if (K % 64) return best;
+  double best_t = 1e300;
+  const int nst = K / 64, tail = N % 64, nmain = N - tail;
+  for (const TileCost& c : kTiles) {
+    if (c.i8 != (i8 ? 1 : 0)) continue;
+    // SwiGLU: whole (gate, up) fragment pairs a wave (RingCfg::FC even)
+    if (need == GN_GLU && c.kind == GK_RING && (c.nb % 2 || (c.mr == 2 && c.nb == 4))) continue;
+    // the softmax pairs' array has room for tiles of 128 columns or more
+    if (need == GN_STATS && c.nb < 8) continue;
+    // 256-row tiles below 512 rows leave most of a tile empty
+    if (c.kind == GK_BIG && (M < 512 || (need == GN_GLU && N % 256))) continue;
+    const int rows = 16 * c.mr, cols = 16 * c.nb;
+    int nct;
+    if (c.kind == GK_BIG) nct = ((nmain ? nmain : N) + cols - 1) / cols;
+    else if (i8) nct = (nmain + cols - 1) / cols + (tail + cols / 2 - 1) / (cols / 2);
+    else nct = (N + cols - 1) / cols;
+    const int tiles = nct * ((M + rows - 1) / rows);
+    auto consider = [&](int split) {
+      if (split < 1 || split > max_split || split > nst) return;
+      const int wg = tiles * split, waves = (wg + 255) / 256, st = (nst + split - 1) / split;
+      const double pm = (double)split * M * N * 1e-6, fill = wg / (256.0 * waves);
+      double t = c.launch + waves * (c.wave + st * (c.stage + c.fill * fill)) + c.part * pm;
+      t += pm * (4 / 5.5) + (split == 1 || split == 2 || split == 4 || split == 8 ? 0.0 : 0.8);
+      if (t < best_t) {
+        best_t = t;
+        best = {c.kind, c.mr, c.nb, split};
+      }
+    };
+    if (fixed > 0) {
+      consider(fixed);
+    } else {
+      // at most two rounds of the CUs, at least two stages a workgroup
+      const int most = nst / 2 > 1 ? nst / 2 : 1;
+      const int s1 = 256 / tiles, s2 = 512 / tiles;
+      consider(1);
+      consider(s1 < most ? s1 : most);
+      consider(s2 < most ? s2 : most);
+      for (int s = 2; s <= 8; s *= 2)
+        if (s <= s2 && s <= most) consider(s);
     }
   }
-  if (!best.nb) best = {forced ? forced : 4, 1};
-  return best;
-}
-static bool skinny_ok(int M, int N, int K) {
-  return M % 128 == 0 && K % 64 == 0 && skinny_stages() != 0 && (N + 15) / 16 < 2048;
-}
-
-// The 256 x 256 tile kernel takes GEMMs with many rows; the skinny kernels
-// everything else.
-static bool big_tiles(int M, int K) { return M >= 1024 && M % BM == 0 && K % (BCH * KSTEP) == 0; }
-static bool use_big_tiles(const GemmArgs& g) {
-  return big_tiles(g.M, g.K) && g.N >= 16 && g.split <= (g.K / (BCH * KSTEP));
-}
-// Large-tile split-K: the one of 1, 2, 4 with the least modelled time.  A
-// wave of tiles costs (0.54 + K / split / 1024) units, one unit being a
-// 256 x 256 tile's 1024-deep K slice; each split past the first adds an fp32
-// [M, N] partial that the GEMM writes and its consumer reads back, M N / 3.15e7
-// units.  (Fitted on MI355X at M = 4096: int8 tiles of K = 1024 and 2048 took
-// 49 and 81 us, and the SwiGLU backward read 100 MB of extra partial in
-// 25 us; so N = 6144, K = 2048 runs unsplit in 1.5 waves, 384 tiles, while the
-// 128-tile GEMMs split in two.)
-// A trailing LoRA segment of <= 64 columns rides in the main launch (its
-// fragments on the first column tiles' workgroups), so it adds no tiles.
-static int big_split(int M, int N, int K, int max_split) {
-  const int nmain = (N % 256 != 0 && N % 64 != 0) ? N - N % 64 : N;
-  const int tiles = (nmain + 255) / 256 * (M / BM);
-  const double partial = (double)M * N / 3.15e7;
-  int best = 1;
-  double best_t = 1e300;
-  for (int split = 1; split <= 4 && split <= max_split && split <= K / (BCH * KSTEP) / 4;
-       split *= 2) {
-    const double t = ceil(tiles * split / 256.0) * (0.54 + K / (1024.0 * split)) +
-                     (split - 1) * partial;
-    if (t < best_t) best_t = t, best = split;
-  }
   return best;
 }
 
-// The DMA large-tile kernel carries the SwiGLU epilogue: 256-wide tiles over
-// 8 waves, gate/up fragment pairs per wave.
+// 256 x 256 tiles take one B segment plus at most one fp16 LoRA segment whose
+// fragments fit on the column tiles (fragment f rides with tile f).
+static bool big_segments(const GemmArgs& g) {
+  if (g.nseg == 1) return true;
+  return g.nseg == 2 && !g.seg[1].is_i8 && g.seg[1].rows <= 64 && g.seg_start[1] % 64 == 0 &&
+         g.seg[1].rows / 16 <= (g.seg[0].rows + 255) / 256;
+}
+static bool ring_segments(const GemmArgs& g) {
+  if (g.seg[0].is_i8) return g.nseg == 1 || (g.nseg == 2 && !g.seg[1].is_i8);
+  for (int i = 1; i < g.nseg; ++i)
+    if (g.seg[i].is_i8) return false;
+  return true;
+}
+
+// The plan gemm_nt launches for g (g.split fixed by the caller).
+static GemmPlan plan_of(const GemmArgs& g) {
+  const GemmPlan nt{GK_NT, 0, 0, g.split};
+  if (g.K % 64 || g.split > g.K / 64) return nt;
+  const bool i8 = g.seg[0].is_i8;
+  if (!i8 && g.M % 128 == 0 && skinny_stages() == 0 && !g.glu) return nt;
+  const int need = g.glu ? GN_GLU : g.rowstats ? GN_STATS : GN_PLAIN;
+  GemmPlan p = gemm_plan(g.M, g.N, g.K, i8, need, g.split, g.split);
+  if (g.split_col) p = {GK_BIG, 16, 16, g.split};  // planned as 256 x 256 tiles, unsplit
+  if (p.kind == GK_BIG && !big_segments(g)) p = {GK_RING, 8, 8, g.split};
+  if (p.kind == GK_RING && !ring_segments(g)) return nt;
+  return p;
+}
+
 int gemm_rowstats_tiles(const GemmArgs& g) {
-  if (g.split != 1 || g.nseg != 1 || g.glu || g.N < 16) return 0;
-  if (use_big_tiles(g)) return (g.N + 255) / 256;  // gemm_dma_kernel tiles
-  return (g.N + kNW * kNF * 16 - 1) / (kNW * kNF * 16);  // gemm_nt_kernel workgroups
+  if (g.split != 1 || g.nseg != 1 || g.glu || g.N < 16 || g.seg[0].is_i8) return 0;
+  GemmArgs q = g;
+  static float2 any;
+  q.rowstats = &any;  // planned with the statistics, as it will be launched
+  const GemmPlan p = plan_of(q);
+  const int cols = p.kind == GK_NT ? kNW * kNF * 16 : 16 * p.nb;
+  return (g.N + cols - 1) / cols;
 }
 
-bool gemm_glu_ok(int M, int I, int K, bool i8) {
-  if (big_tiles(M, K))
-    return I % 128 == 0 && big_split(M, 2 * I, K, 64) == 1;
-  // the skinny kernel, 32 gate + 32 up columns a workgroup, split 1
-  return !i8 && skinny_ok(M, 2 * I, K) && I % 32 == 0;
-}
-
-// The last wave of an unsplit large-tile GEMM: with tiles = full waves of
+// The last wave of an unsplit 256 x 256-tile GEMM: with tiles = full waves of
 // the 256 CUs plus r more (r <= 128, whole column tiles), the last r tiles
 // run as 2 r half-K workgroups, so the launch takes 1 + 1/2 wave-times of a
-// tile instead of 2 (C4's down-projection dX: 384 tiles).  Their partial
-// is an extra fp32 [M, r/ntm x 256] the consumer reads back.
-int gemm_split_col(int M, int N, int K) {
-  if (!big_tiles(M, K) || N % 256 || big_split(M, N, K, 64) != 1 ||
-      K / (BCH * KSTEP) < 8)
-    return 0;
-  const int ntm = M / BM, ntn = N / 256, tiles = ntm * ntn;
+// tile instead of 2 (the down-projection dX of 4096 rows: 384 tiles).  Their
+// partial is an extra fp32 [M, r/ntm x 256] the consumer reads back.
+int gemm_split_col(int M, int N, int K, bool i8) {
+  if (N % 256 || K % 64 || K / 64 < 8) return 0;
+  const GemmPlan p = gemm_plan(M, N, K, i8, GN_PLAIN, 0, 64);
+  if (p.kind != GK_BIG || p.split != 1) return 0;
+  const int ntm = (M + BM - 1) / BM, ntn = N / 256, tiles = ntm * ntn;
   const int rest = tiles % 256;
   if (tiles < 256 || rest == 0 || rest > 128 || rest % ntm) return 0;
   return (ntn - rest / ntm) * 256;
 }
 
-int gemm_pick_split(int M, int N, int K, int max_split) {
-  if (big_tiles(M, K)) return big_split(M, N, K, max_split);
-  if (skinny_ok(M, N, K)) {
-    const int split = skinny_plan(M, N, K).split;
-    return split > max_split ? max_split : split;
+// Forced ring widths (tests, tuning): the splits that keep the grid near one
+// workgroup per CU.
+static int forced_split(int M, int N, int K, int nb) {
+  const int tiles = ((N + 15) / 16 + nb - 1) / nb * (M / 128);
+  int split = (K <= 4096 ? 192 : 256) / tiles;
+  if (split > K / 128) split = K / 128;
+  return split < 1 ? 1 : split;
+}
+static int forced_nb(int M, int K, bool i8) {
+  if (i8 || M % 128 || K % 64) return 0;
+  return env_int("LLMT_GEMM_SKINNY_NB", 0);
+}
+
+int gemm_pick_split(int M, int N, int K, int max_split, bool i8) {
+  if (const int nb = forced_nb(M, K, i8)) {
+    const int s = forced_split(M, N, K, nb);
+    return s > max_split ? max_split : s;
   }
-  // Partials grow with the workgroup count: about 3/4 of the CUs for the
-  // layer GEMMs, two waves of CUs for the very long lm_head dX reduction.
-  const int target = K > 16384 ? 512 : 192;
-  constexpr int min_steps = 4;
+  const GemmPlan p = gemm_plan(M, N, K, i8, GN_PLAIN, 0, max_split);
+  if (p.kind != GK_NT) return p.split;
+  // the register-staged kernel: about 3/4 of the CUs, four k-steps or more a
+  // split
   const int mt = (M % 128 == 0) ? M / 128 : 1;
   constexpr int tn = kNW * kNF * 16;
   const int ntiles = (N + tn - 1) / tn * mt;
-  int split = (target + ntiles / 2) / ntiles;
-  const int kmax = (K / KSTEP) / min_steps;
+  int split = ((K > 16384 ? 512 : 192) + ntiles / 2) / ntiles;
+  const int kmax = (K / KSTEP) / 4;
   if (split > kmax) split = kmax;
   if (split > max_split) split = max_split;
   if (split < 1) split = 1;
   return split;
 }
 
-// M % 128 == 0 with fp16 weights: the DMA-fed skinny kernel, 128 x BN tiles.
-// LDS of an S-stage ring of NB-fragment tiles within the 160 KB of a CU
-template <int S, int NB>
-constexpr bool skinny_fits = S * (16384 + NB * 2048) <= 160 * 1024;
-
-template <int S>
-static void launch_skinny(const GemmArgs& g, int nb, hipStream_t st) {
-  const dim3 grid(g.split, (g.N + nb * 16 - 1) / (nb * 16), g.M / 128);
-  switch (nb) {
-    case 2: hipLaunchKernelGGL((gemm_skinny_kernel<S, 2>), grid, dim3(512), 0, st, g); break;
-    case 3: hipLaunchKernelGGL((gemm_skinny_kernel<S, 3>), grid, dim3(512), 0, st, g); break;
-    case 6:
-      if constexpr (skinny_fits<S, 6>)
-        hipLaunchKernelGGL((gemm_skinny_kernel<S, 6>), grid, dim3(512), 0, st, g);
-      break;
-    case 8:
-      if constexpr (skinny_fits<S, 8>)
-        hipLaunchKernelGGL((gemm_skinny_kernel<S, 8>), grid, dim3(512), 0, st, g);
-      break;
-    default: hipLaunchKernelGGL((gemm_skinny_kernel<S, 4>), grid, dim3(512), 0, st, g); break;
+template <class C>
+static hipError_t launch_ring(const GemmArgs& g, hipStream_t st) {
+  const int nrb = (g.M + C::MR * 16 - 1) / (C::MR * 16);
+  int nct;
+  if (g.glu) {
+    nct = (g.glu / 16 + C::NB / 2 - 1) / (C::NB / 2);
+  } else if (C::I8) {
+    nct = (g.seg[0].rows / 16 + C::NB - 1) / C::NB;
+    if (g.nseg > 1) nct += (g.seg[1].rows / 16 + C::NB / 2 - 1) / (C::NB / 2);
+  } else {
+    nct = (g.N / 16 + C::NB - 1) / C::NB;
   }
-}
-static hipError_t launch_m128(const GemmArgs& g, hipStream_t st) {
-  bool i8 = false;
-  for (int i = 0; i < g.nseg; ++i) i8 = i8 || g.seg[i].is_i8;
-  if (i8 || g.rowstats || !skinny_ok(g.M, g.N, g.K) || g.split > g.K / 64)
-    return launch_mf<8>(g, st);
-  const int nb = skinny_plan(g.M, g.N, g.K).nb;
-  const int stages = skinny_stages();
-  if (stages == 6 && nb > 4) {
-    set_error("gemm_nt: %d-stage skinny ring of %d fragments exceeds the LDS", stages, nb);
+  const dim3 grid = nrb == 1 ? dim3(g.split, nct) : dim3(nrb * nct * g.split);
+  if (g.glu) {
+    if constexpr (C::FC % 2 == 0) {
+      hipLaunchKernelGGL((gemm_ring_kernel<C, false, true>), grid, dim3(512), 0, st, g, nrb, nct);
+      return hipGetLastError();
+    }
+    set_error("gemm_nt: no SwiGLU epilogue on tiles of %d fragments", C::NB);
     return hipErrorInvalidValue;
   }
-  switch (stages) {
-    case 3: launch_skinny<3>(g, nb, st); break;
-    case 5: launch_skinny<5>(g, nb, st); break;
-    case 6: launch_skinny<6>(g, nb, st); break;
-    default: launch_skinny<4>(g, nb, st); break;
+  if constexpr (C::I8) {
+    if (g.seg[0].kscale) {
+      hipLaunchKernelGGL((gemm_ring_kernel<C, true, false>), grid, dim3(512), 0, st, g, nrb, nct);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((gemm_ring_kernel<C, false, false>), grid, dim3(512), 0, st, g, nrb, nct);
+  return hipGetLastError();
+}
+
+// Ring depths: what keeps enough weight bytes in flight (about 24 KB a CU)
+// and fits the LDS.
+static hipError_t launch_plan(const GemmArgs& g, const GemmPlan& p, hipStream_t st) {
+  const bool i8 = g.seg[0].is_i8;
+  const int key = p.mr * 100 + p.nb;
+  if (i8) {
+    switch (key) {
+      case 204: return launch_ring<RingCfg<8, 2, 4, 1, true>>(g, st);
+      case 208: return launch_ring<RingCfg<8, 2, 8, 1, true>>(g, st);
+      case 404: return launch_ring<RingCfg<8, 4, 4, 2, true>>(g, st);
+      case 408: return launch_ring<RingCfg<7, 4, 8, 2, true>>(g, st);
+      case 812: return launch_ring<RingCfg<5, 8, 12, 2, true>>(g, st);
+      case 816: return launch_ring<RingCfg<4, 8, 16, 2, true>>(g, st);
+      default: return launch_ring<RingCfg<5, 8, 8, 2, true>>(g, st);
+    }
+  } else {
+    switch (key) {
+      case 204: return launch_ring<RingCfg<6, 2, 4, 1, false>>(g, st);
+      case 208: return launch_ring<RingCfg<5, 2, 8, 1, false>>(g, st);
+      case 404: return launch_ring<RingCfg<4, 4, 4, 2, false>>(g, st);
+      case 408: return launch_ring<RingCfg<4, 4, 8, 2, false>>(g, st);
+      case 803: return launch_ring<RingCfg<4, 8, 3, 4, false>>(g, st);
+      case 804: return launch_ring<RingCfg<4, 8, 4, 4, false>>(g, st);
+      case 812: return launch_ring<RingCfg<4, 8, 12, 2, false>>(g, st);
+      case 816: return launch_ring<RingCfg<3, 8, 16, 2, false>>(g, st);
+      default: return launch_ring<RingCfg<4, 8, 8, 2, false>>(g, st);
+    }
+  }
+}
+template <int S>
+static hipError_t launch_forced(const GemmArgs& g, int nb, hipStream_t st) {
+  switch (nb) {
+    case 2: return launch_ring<RingCfg<S, 8, 2, 4, false>>(g, st);
+    case 3: return launch_ring<RingCfg<S, 8, 3, 4, false>>(g, st);
+    case 4: return launch_ring<RingCfg<S, 8, 4, 4, false>>(g, st);
+  }
+  if constexpr (S <= 5) {
+    if (nb == 6) return launch_ring<RingCfg<S, 8, 6, 4, false>>(g, st);
+    if (nb == 8) return launch_ring<RingCfg<S, 8, 8, 4, false>>(g, st);
+  }
+  set_error("gemm_nt: no %d-stage ring of %d fragments", S, nb);
+  return hipErrorInvalidValue;
+}
+
+static hipError_t launch_big(const GemmArgs& g, hipStream_t st) {
+  GemmArgs gm = g;
+  const bool fold = g.nseg > 1;  // the LoRA rows ride along (fragment f with column tile f)
+  const BSeg tl = fold ? g.seg[1] : BSeg{};
+  const int tc0 = fold ? g.seg_start[1] : 0;
+  gm.nseg = 1;
+  gemm_finalize_segments(gm);
+  const int ntm = (gm.M + BM - 1) / BM;
+  // XCD-contiguous tile runs: workgroup b goes to XCD b % 8, and the tiles
+  // sharing an A row block then share that XCD's L2 (+0.7% step rate at 4096
+  // rows)
+  const int order = 1;
+  const bool i8 = gm.seg[0].is_i8, ks = gm.seg[0].kscale != nullptr;
+  if (gm.split_col > 0 &&
+      (gm.split != 2 || gm.split_col % 256 || gm.split_col >= gm.N || gm.N % 256 || gm.glu ||
+       gm.rowstats || fold)) {
+    set_error("gemm_nt: split_col %d needs split 2 and whole 256-column tiles (N = %d)",
+              gm.split_col, gm.N);
+    return hipErrorInvalidValue;
+  }
+  const dim3 gr = gm.split_col > 0
+                      ? dim3(gm.split_col / 256 * ntm + 2 * (gm.N - gm.split_col) / 256 * ntm, 1)
+                      : dim3((gm.N + 255) / 256 * ntm, gm.split);
+  // ring depth 5 (int8) / 4 (fp16): 4 measured the same, 6 slower
+  auto go = [&](auto i8c, auto ksc, auto gluc, auto tlc) {
+    constexpr bool I8 = decltype(i8c)::value, KS = decltype(ksc)::value;
+    constexpr bool GL = decltype(gluc)::value, TLc = decltype(tlc)::value;
+    constexpr int SD = I8 ? 5 : 4;
+    hipLaunchKernelGGL((gemm_dma_kernel<I8, KS, SD, 4, GL, TLc>), gr, dim3(512), 0, st, gm, order,
+                       tl, tc0);
+  };
+  using BT = std::integral_constant<bool, true>;
+  using BF = std::integral_constant<bool, false>;
+  if (gm.glu) {
+    if (!i8) go(BF(), BF(), BT(), BF());
+    else if (ks) go(BT(), BT(), BT(), BF());
+    else go(BT(), BF(), BT(), BF());
+  } else if (fold) {
+    if (!i8) go(BF(), BF(), BF(), BT());
+    else if (ks) go(BT(), BT(), BF(), BT());
+    else go(BT(), BF(), BF(), BT());
+  } else {
+    if (!i8) go(BF(), BF(), BF(), BF());
+    else if (ks) go(BT(), BT(), BF(), BF());
+    else go(BT(), BF(), BF(), BF());
   }
   return hipGetLastError();
 }
 
 const char* gemm_kernel_name(const GemmArgs& g) {
-  if (use_big_tiles(g)) {
-    const int last = g.nseg - 1;
-    if (g.glu) return "gemm_dma_glu";
-    if (g.nseg > 1 && g.seg[last].rows <= 64 && g.seg_start[last] % 64 == 0)
-      return g.seg[last].is_i8 || g.seg[last].rows / 16 > (g.N - g.seg[last].rows + 255) / 256
-                 ? "gemm_dma+lora_skinny"
-                 : "gemm_dma+lora";
-    return "gemm_dma";
-  }
-  if (g.glu) return "gemm_skinny_glu";
-  bool i8 = false;
-  for (int i = 0; i < g.nseg; ++i) i8 = i8 || g.seg[i].is_i8;
-  if ((g.M / 16) % 8 == 0 && !i8 && !g.rowstats && skinny_ok(g.M, g.N, g.K) &&
-      g.split <= g.K / 64)
-    return "gemm_skinny";
+  const GemmPlan p = plan_of(g);
+  if (p.kind == GK_BIG) return g.glu ? "gemm_dma_glu" : g.nseg > 1 ? "gemm_dma+lora" : "gemm_dma";
+  if (p.kind == GK_RING) return g.glu ? "gemm_ring_glu" : "gemm_ring";
   return "gemm_nt";
 }
 
@@ -1314,98 +1639,42 @@ hipError_t gemm_nt(const GemmArgs& g, hipStream_t st) {
       set_error("gemm_nt: segment rows must be a multiple of 16 (%d)", g.seg[i].rows);
       return hipErrorInvalidValue;
     }
-  if (g.glu && !(g.N == 2 * g.glu && g.nseg == 1 && g.split == 1 && g.glu16 && g.gu16 &&
-                 gemm_glu_ok(g.M, g.glu, g.K, g.seg[0].is_i8))) {
-    set_error("gemm_nt: SwiGLU epilogue needs split 1, one segment, N = 2 x %d", g.glu);
+  const GemmPlan p = plan_of(g);
+  if (g.glu && !(g.N == 2 * g.glu && g.glu % 16 == 0 && g.nseg == 1 && g.split == 1 && g.glu16 &&
+                 g.gu16 && p.kind != GK_NT)) {
+    set_error("gemm_nt: SwiGLU epilogue needs K %% 64 == 0, split 1, one segment, N = 2 x %d", g.glu);
     return hipErrorInvalidValue;
   }
-  if (g.split_col && !use_big_tiles(g)) {
+  if (!g.glu && !g.C) {
+    set_error("gemm_nt: no output");
+    return hipErrorInvalidValue;
+  }
+  if (g.split_col && p.kind != GK_BIG) {
     set_error("gemm_nt: split_col needs the large-tile kernel");
     return hipErrorInvalidValue;
   }
   if (g.rowstats && gemm_rowstats_tiles(g) == 0) {
-    set_error("gemm_nt: row statistics need split 1, one segment and no SwiGLU epilogue");
+    set_error("gemm_nt: row statistics need split 1, one fp16 segment and no SwiGLU epilogue");
     return hipErrorInvalidValue;
-  }
-  if (g.glu && !use_big_tiles(g)) {
-    hipLaunchKernelGGL((gemm_skinny_kernel<4, 4, true>), dim3(1, g.glu / 32, g.M / 128), dim3(512),
-                       0, st, g);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) set_error("gemm_nt launch: %s", hipGetErrorString(e));
-    return e;
   }
   hipError_t e;
   const int m16 = g.M / 16;
-  if (use_big_tiles(g)) {
-    GemmArgs gm = g;
-    const int last = g.nseg - 1;
-    const bool lora_tail = g.nseg > 1 && g.seg[last].rows <= 64 && g.seg_start[last] % 64 == 0;
-    if (lora_tail) {  // the main segments on big tiles, the LoRA rows skinny
-      gm.nseg = last;
-      gemm_finalize_segments(gm);
+  const int nb = g.glu || g.rowstats ? 0 : forced_nb(g.M, g.K, g.seg[0].is_i8);
+  if (p.kind == GK_RING && nb) {
+    switch (skinny_stages()) {
+      case 3: e = launch_forced<3>(g, nb, st); break;
+      case 5: e = launch_forced<5>(g, nb, st); break;
+      case 6: e = launch_forced<6>(g, nb, st); break;
+      default: e = launch_forced<4>(g, nb, st); break;
     }
-    const int nwg = (gm.N + 255) / 256 * (gm.M / BM);
-    // XCD-contiguous tile runs: workgroup b goes to XCD b % 8, and the tiles
-    // sharing an A row block then share that XCD's L2 (C4: +0.7% step rate)
-    const int order = 1;
-    const bool i8 = gm.seg[0].is_i8, ks = gm.seg[0].kscale != nullptr;
-    if (gm.nseg != 1 || gm.N % 16 != 0) {
-      set_error("gemm_nt: large tiles take one B segment with N %% 16 == 0 (N = %d, %d segments)",
-                gm.N, gm.nseg);
-      return hipErrorInvalidValue;
-    }
-    if (gm.split_col > 0 &&
-        (gm.split != 2 || gm.split_col % 256 || gm.split_col >= gm.N || gm.N % 256 || gm.glu ||
-         gm.rowstats || lora_tail)) {
-      set_error("gemm_nt: split_col %d needs split 2 and whole 256-column tiles (N = %d)",
-                gm.split_col, gm.N);
-      return hipErrorInvalidValue;
-    }
-    const dim3 gr = gm.split_col > 0
-                        ? dim3(gm.split_col / 256 * (gm.M / BM) + 2 * (gm.N - gm.split_col) / 256 * (gm.M / BM), 1)
-                        : dim3(nwg, gm.split);
-    // the LoRA rows fold into the main launch (fragment f with column tile f)
-    // when they are fp16 and no more fragments than column tiles
-    const BSeg tl = lora_tail ? g.seg[last] : BSeg{};
-    const bool fold = lora_tail && !tl.is_i8 && tl.rows / 16 <= (gm.N + 255) / 256;
-    const int tc0 = lora_tail ? g.seg_start[last] : 0;
-    // ring depth 5 (int8) / 4 (fp16): 4 measured the same, 6 slower
-    auto go = [&](auto i8c, auto ksc, auto gluc, auto tlc) {
-      constexpr bool I8 = decltype(i8c)::value, KS = decltype(ksc)::value;
-      constexpr bool GL = decltype(gluc)::value, TLc = decltype(tlc)::value;
-      constexpr int SD = I8 ? 5 : 4;
-      hipLaunchKernelGGL((gemm_dma_kernel<I8, KS, SD, 4, GL, TLc>), gr, dim3(512), 0, st, gm, order,
-                         tl, tc0);
-    };
-    using BT = std::integral_constant<bool, true>;
-    using BF = std::integral_constant<bool, false>;
-    if (gm.glu) {
-      if (!i8) go(BF(), BF(), BT(), BF());
-      else if (ks) go(BT(), BT(), BT(), BF());
-      else go(BT(), BF(), BT(), BF());
-    } else if (fold) {
-      if (!i8) go(BF(), BF(), BF(), BT());
-      else if (ks) go(BT(), BT(), BF(), BT());
-      else go(BT(), BF(), BF(), BT());
-    } else {
-      if (!i8) go(BF(), BF(), BF(), BF());
-      else if (ks) go(BT(), BT(), BF(), BF());
-      else go(BT(), BF(), BF(), BF());
-    }
-    e = hipGetLastError();
-    if (e == hipSuccess && lora_tail && !fold) {
-      GemmArgs gl = g;
-      gl.nseg = 1;
-      gl.seg[0] = g.seg[last];
-      gemm_finalize_segments(gl);
-      gl.C = g.C + g.seg_start[last];
-      e = launch_m128(gl, st);
-    }
-  } else if (m16 % 8 == 0) e = launch_m128(g, st);
+  }
+  else if (p.kind == GK_RING) e = launch_plan(g, p, st);
+  else if (p.kind == GK_BIG) e = launch_big(g, st);
+  else if (m16 % 8 == 0) e = launch_mf<8>(g, st);
   else if (m16 % 4 == 0) e = launch_mf<4>(g, st);
   else if (m16 % 2 == 0) e = launch_mf<2>(g, st);
   else e = launch_mf<1>(g, st);
-  if (e != hipSuccess) set_error("gemm_nt launch: %s", hipGetErrorString(e));
+  if (e != hipSuccess && e != hipErrorInvalidValue) set_error("gemm_nt launch: %s", hipGetErrorString(e));
   return e;
 }
 

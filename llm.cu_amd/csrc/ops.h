@@ -51,8 +51,6 @@ struct GemmArgs {
   // statistics of the lm_head logits, so the logits are read only once).
   float2* rowstats;
 };
-// The fused SwiGLU epilogue exists for this GEMM shape and weight type.
-bool gemm_glu_ok(int M, int I, int K, bool i8);
 // Column tiles per row whose statistics gemm_nt writes for g.rowstats (the
 // row width of the rowstats array), 0 if this GEMM cannot write them.
 int gemm_rowstats_tiles(const GemmArgs& g);
@@ -61,15 +59,16 @@ int gemm_rowstats_tiles(const GemmArgs& g);
 // length K; rows a multiple of 16.  A is row-major fp16 [M, lda], K % 32 == 0.
 // Fills seg_start/N from seg[0..nseg).
 void gemm_finalize_segments(GemmArgs& g);
-// Split factor for a GEMM of this shape on this device (>=1, bounded by K).
-int gemm_pick_split(int M, int N, int K, int max_split);
+// Split factor for a GEMM of this shape and weight type on this device (>=1,
+// bounded by K); N counts a trailing LoRA segment.
+int gemm_pick_split(int M, int N, int K, int max_split, bool i8);
 // For a large-tile GEMM planned unsplit whose 256 x 256 tiles end in a
 // partial wave of the CUs: the column where tiles start to be split in two
 // so that the last wave is full (GemmArgs::split_col, with split 2); 0 when
 // the tiles fill whole waves or the shape does not allow it.
-int gemm_split_col(int M, int N, int K);
+int gemm_split_col(int M, int N, int K, bool i8);
 hipError_t gemm_nt(const GemmArgs& g, hipStream_t st);
-// Name of the kernel gemm_nt launches for g ("gemm_skinny", "gemm_dma", ...).
+// Name of the kernel gemm_nt launches for g ("gemm_ring", "gemm_dma", ...).
 const char* gemm_kernel_name(const GemmArgs& g);
 // out[m][n] = sum_s part[s][m][n] in split order, plus for output columns
 // [c0, c0 + n) of each LoRA adapter lscale * sum_r part-sum[m][hcol + r] *
@@ -218,7 +217,6 @@ hipError_t embed_norm(const int* tok, const _Float16* E, int V, int H, const flo
 hipError_t qkv_post(const QkvPostArgs& a, int T, hipStream_t st);
 hipError_t o_post(const RowIn& in, const float* x_in, const float* w, float eps, int H, int T,
                   float* hbuf, float* x_mid, _Float16* xn2, hipStream_t st);
-hipError_t gu_post(const RowIn& in, int I, int T, _Float16* gu, _Float16* a16, hipStream_t st);
 hipError_t resid_norm(const RowIn& in, const float* x_res, const float* w, float eps, int H, int T,
                       float* x_out, _Float16* xn, hipStream_t st);
 // cos / sin tables of the half-split RoPE, [S, 64] fp32 each, on the device.

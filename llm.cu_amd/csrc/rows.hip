@@ -71,21 +71,6 @@ __device__ __forceinline__ float amax4(float4 v) {
   return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
 }
 
-// Split-K partial sums in split order (deterministic), every load of a
-// batch issued before the first add.
-__device__ __forceinline__ float4 sum_splits4(const float* p, int split, long long ss) {
-  constexpr int SB = 16;
-  float4 v = ld4(p);
-  for (int k = 1; k < split; k += SB) {
-    float4 x[SB];
-#pragma unroll
-    for (int i = 0; i < SB; ++i) x[i] = ld4(p + (long long)min(k + i, split - 1) * ss);
-#pragma unroll
-    for (int i = 0; i < SB; ++i) v = k + i < split ? add4(v, x[i]) : v;
-  }
-  return v;
-}
-
 // This thread's pieces of row t of a split-K GEMM output: piece p is columns
 // 4 (tid + p RT) .. + 3 (live when < n; dead pieces hold column 0's values),
 // plus (HH) this thread's four raw h columns when tid < nh / 4 (others hold
@@ -289,8 +274,6 @@ __device__ __forceinline__ void lora_apply_rows(const RowIn& in, const float (*h
 #pragma unroll
   for (int i = 0; i < NR; ++i) v[i] = add4(v[i], mul4(acc[i], in.lscale));
 }
-
-__device__ __forceinline__ float silu(float g) { return g * sigmoid_rcp(g); }
 
 // Two block sums at once (one barrier pair).
 __device__ __forceinline__ float2 block_sum2(float a, float b, float* red) {
@@ -760,30 +743,6 @@ __global__ __launch_bounds__(RT) void resid_norm_rows_kernel(const RowIn in,
   }
 }
 
-// After the fused gate/up GEMM: stash g, u (fp16, for the backward) and
-// a = silu(g) * u (src/kernels/activation.cu:5-18) from the fp32 sums as the
-// fp16 operand of the down GEMM.
-__global__ __launch_bounds__(RT) void gu_post_kernel(const RowIn in, int I, long long n4,
-                                                     _Float16* __restrict__ gu,
-                                                     _Float16* __restrict__ a16) {
-  for (long long i = (long long)blockIdx.x * RT + threadIdx.x; i < n4;
-       i += (long long)gridDim.x * RT) {
-    const long long t = i / (I / 4);
-    const int c = (int)(i - t * (I / 4)) * 4;
-    const float* p = in.part + t * in.ldp + c;
-    const float4 g = sum_splits4(p, in.split, in.ss);
-    const float4 u = sum_splits4(p + I, in.split, in.ss);
-    st_h4(gu + t * 2 * I + c, g);
-    st_h4(gu + t * 2 * I + I + c, u);
-    half4 o;
-    o[0] = (_Float16)(silu(g.x) * u.x);
-    o[1] = (_Float16)(silu(g.y) * u.y);
-    o[2] = (_Float16)(silu(g.z) * u.z);
-    o[3] = (_Float16)(silu(g.w) * u.w);
-    *reinterpret_cast<half4*>(a16 + t * I + c) = o;
-  }
-}
-
 // After the down GEMM: x_out = x_mid + aW_down^T, then the next RMSNorm
 // (the next layer's attention norm, or the final norm) -> fp16.
 template <int P>
@@ -1122,7 +1081,9 @@ __global__ __launch_bounds__(RT) void norm_bwd_rows_kernel(const NormBwdArgs a, 
 // dX of the down projection -> SwiGLU backward (src/kernels/activation.cu:
 // 26-43 with d_up = dy * silu(g), i.e. without the reference's aliasing of
 // d_gate and d_swiglu at src/kernels/lora_backward.cu:287) -> [dg | du] fp16.
-template <int P, bool SC = false, bool NTG = false>
+// NS = 1: exactly one partial (the general form keeps 8 partials of a piece
+// in registers, 24 float4 a thread: at 4096 rows 70 us against 50).
+template <int P, bool SC = false, bool NTG = false, int NS = 0>
 __global__ __launch_bounds__(RT) void swiglu_bwd_kernel(const RowIn in,
                                                         const float* __restrict__ rinv_in,
                                                         const _Float16* __restrict__ gu, int I,
@@ -1148,7 +1109,12 @@ __global__ __launch_bounds__(RT) void swiglu_bwd_kernel(const RowIn in,
   }
   const float rs = rinv_in[t];
   float4 v[P];
-  load_partials<P, SC>(in, t, I, v);
+  if constexpr (NS > 0) {
+    float4 none;
+    load_row_ns<P, NS, false>(in, t, I, v, none, []() {});
+  } else {
+    load_partials<P, SC>(in, t, I, v);
+  }
   float4 dg[P], du[P];
   float amax = 0.f;
 #pragma unroll
@@ -1661,14 +1627,6 @@ hipError_t o_post(const RowIn& in, const float* x_in, const float* w, float eps,
   return hipSuccess;
 }
 
-hipError_t gu_post(const RowIn& in, int I, int T, _Float16* gu, _Float16* a16, hipStream_t st) {
-  if (!row_in_ok(in, I, "gu_post") || in.nterm) return hipErrorInvalidValue;
-  const long long n4 = (long long)T * (I / 4);
-  hipLaunchKernelGGL(gu_post_kernel, dim3(grid_elems(n4)), dim3(RT), 0, st, in, I, n4, gu, a16);
-  LLMT_LAUNCH_CHECK();
-  return hipSuccess;
-}
-
 hipError_t resid_norm(const RowIn& in, const float* x_res, const float* w, float eps, int H, int T,
                       float* x_out, _Float16* xn, hipStream_t st) {
   if (!row_in_ok(in, H, "resid_norm")) return hipErrorInvalidValue;
@@ -1831,7 +1789,12 @@ hipError_t swiglu_bwd(const RowIn& in, const float* rinv_in, const _Float16* gu,
   auto pick = [&](auto p, auto s) {
     constexpr int PP = decltype(p)::value;
     constexpr bool SS = decltype(s)::value;
-    if (nt)
+    constexpr int one = SS ? 0 : 1;  // a split_col input has two partials
+    if (nt && in.split == 1)
+      go(swiglu_bwd_kernel<PP, SS, true, one>);
+    else if (in.split == 1)
+      go(swiglu_bwd_kernel<PP, SS, false, one>);
+    else if (nt)
       go(swiglu_bwd_kernel<PP, SS, true>);
     else
       go(swiglu_bwd_kernel<PP, SS, false>);

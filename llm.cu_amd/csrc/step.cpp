@@ -110,9 +110,9 @@ hipError_t Ctx::gemm(int cat, const _Float16* A, int lda, const BSeg* segs, int 
       if (tiles) *tiles = nt;
     }
   } else {
-    g.split = gemm_pick_split(M, g.N, K, 64);
+    g.split = gemm_pick_split(M, g.N, K, 64, segs[0].is_i8);
     if (last_wave_split && nseg == 1 && g.split == 1) {
-      g.split_col = gemm_split_col(M, g.N, K);
+      g.split_col = gemm_split_col(M, g.N, K, segs[0].is_i8);
       if (g.split_col) g.split = 2;
     }
     g.C = part;
@@ -269,19 +269,9 @@ hipError_t Ctx::layer_fwd(int l, int B, const float* next_w, float* x_out, _Floa
       return o_post(ri, x_in, fw, eps, Hh, T, hb, x_mid, xn2, q);
     }, 0, part_bytes(ri, T, H) + (double)T * (H * 4 + H * 4 + H * 2 + 16 * 4)));
   }
-  // gate/up, SwiGLU (in the GEMM epilogue where the large-tile kernel runs)
+  // gate/up with the SwiGLU in the GEMM's epilogue
   BSeg sg[1] = {wseg(w.wgu)};
-  if (gemm_glu_ok(T, I, H, sg[0].is_i8)) {
-    LLMT_HIP_TRY(gemm(CAT_GEMM_FWD, s.xn2, H, sg, 1, T, H, nullptr, 0, nullptr, a16, s.gu));
-  } else {
-    LLMT_HIP_TRY(gemm(CAT_GEMM_FWD, s.xn2, H, sg, 1, T, H, nullptr, 0, &go));
-    const RowIn ri = row_in(go);
-    _Float16* gu = s.gu;
-    _Float16* a = a16;
-    const int Ii = I;
-    LLMT_HIP_TRY(run(CAT_ROWS, "gu_post", [=](hipStream_t q) { return gu_post(ri, Ii, T, gu, a, q); },
-                     0, part_bytes(ri, T, 2 * I) + (double)T * (2 * I * 2 + I * 2)));
-  }
+  LLMT_HIP_TRY(gemm(CAT_GEMM_FWD, s.xn2, H, sg, 1, T, H, nullptr, 0, nullptr, a16, s.gu));
   // down, residual, next norm
   BSeg sd[1] = {wseg(w.wd)};
   LLMT_HIP_TRY(gemm(CAT_GEMM_FWD, a16, I, sd, 1, T, I, nullptr, 0, &go));

@@ -1,0 +1,107 @@
+"""GPU: the GEMM tiles at the row counts where they change (edges of the 32-,
+64-, 128- and 256-row tiles, remainders of all of them), with fp16 and int8
+weights: the standalone products, one full-width decoder layer (the Q/K/V and
+O GEMMs' LoRA rows, the SwiGLU epilogue, the per-k scales of int8 dX GEMMs)
+against the fp32 oracle, and the head with its softmax statistics."""
+import numpy as np
+import pytest
+import torch
+
+import llmt
+from helpers import grad_errors, rel_l2
+from oracle import lora_step as ref
+from oracle.configs import make_adapters, make_layer
+from oracle.quant import quantize_rows
+
+pytestmark = pytest.mark.gpu
+
+GRAD_TOL = 1e-2
+
+
+@pytest.mark.parametrize("i8", [False, True])
+@pytest.mark.parametrize("M", [16, 48, 80, 144, 336, 528, 1040])
+@pytest.mark.parametrize("N,K", [(16, 64), (176, 192), (2064, 2048), (4096, 320)])
+def test_gemm_row_tiles(dev, L, i8, M, N, K):
+    # fp16 operands (int8 ones are exact in fp16), fp32 sums of K products in
+    # another order: 1e-5 is the bar of the other GEMM tests
+    print(f"case: gemm i8={i8} M{M} N{N} K{K}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g).half()
+    w = torch.randn(N, K, generator=g) * 0.02
+    if i8:
+        q, sc = quantize_rows(w.numpy())
+        sc16 = torch.from_numpy(sc.astype(np.float16))
+        qt = torch.from_numpy(q)
+        want = (A.float() @ qt.float().t()) * sc16.float()[None, :]
+        got = llmt.gemm_i8(A.to(dev), qt.to(dev), sc16.to(dev)).cpu()
+    else:
+        B = w.half()
+        want = A.float() @ B.float().t()
+        got = llmt.gemm_f16(A.to(dev), B.to(dev)).cpu()
+    assert rel_l2(got, want) < 1e-5
+    assert torch.isfinite(got).all()
+
+
+@pytest.mark.parametrize("int8,B,S", [(False, 1, 16), (False, 1, 80), (False, 3, 208),
+                                      (False, 5, 400), (True, 1, 48), (True, 1, 208),
+                                      (True, 1, 336), (True, 5, 400)])
+def test_layer_row_tiles_match_oracle(dev, int8, B, S):
+    print(f"case: full-width layer int8={int8} B{B} S{S}", flush=True)
+    d = ref.Dims(**{**ref.QWEN3_1_7B.__dict__, "n_layers": 1, "vocab": 256})
+    g = torch.Generator().manual_seed(B * 1000 + S)
+    lw = make_layer(g, d)
+    ad = make_adapters(g, d)[0]
+    x, dy = torch.randn(B * S, d.hidden, generator=g), torch.randn(B * S, d.hidden, generator=g)
+    names = ("wq", "wk", "wv", "wo", "w_gate", "w_up", "w_down")
+    f = lambda t: t.to(torch.float32).to(dev).contiguous()
+    norms = [f(t) for t in (lw.attn_norm, lw.ffn_norm, lw.q_norm, lw.k_norm)]
+    ctx = llmt.Context(llmt.make_dims(d), B, S, int8=int8)
+    try:
+        if int8:
+            qs, ss = [], []
+            for n in names:
+                q, sc = quantize_rows(getattr(lw, n).float().numpy())
+                sc16 = sc.astype(np.float16)
+                qs.append(torch.from_numpy(q).to(dev))
+                ss.append(torch.from_numpy(sc16).to(dev))
+                setattr(lw, n, torch.from_numpy(q.astype(np.float32) *
+                                                sc16.astype(np.float32)[:, None]))
+            ctx.set_layer_i8(0, qs, ss, *norms)
+        else:
+            ctx.set_layer_f16(0, *(getattr(lw, n).half().to(dev).contiguous() for n in names), *norms)
+        cos, sin = ref.rope_tables(S, d.head_dim, d.theta)
+        y_ref, st = ref.layer_forward(x, lw, ad, d, B, S, cos, sin)
+        dx_ref, grads_ref = ref.layer_backward(dy, st, lw, ad, d, B, S, cos, sin)
+        ctx.lora_set("param", llmt.flatten_adapters([ad]).to(dev))
+        y = ctx.layer_forward(0, x.to(dev), B)
+        assert rel_l2(y.cpu(), y_ref) < GRAD_TOL
+        dx = ctx.layer_backward(0, dy.to(dev), B)
+        assert rel_l2(dx.cpu(), dx_ref) < GRAD_TOL
+        errs = grad_errors(ctx.lora_get("grad"), [grads_ref], d)
+        print("worst", max(errs.items(), key=lambda kv: kv[1]), flush=True)
+        assert max(errs.values()) < GRAD_TOL
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("T", [16, 48, 112, 336, 528, 1040])
+def test_head_row_tiles(dev, T):
+    print(f"case: head T{T}", flush=True)
+    H, V = 512, 9984  # 78 tiles of 128 columns, 39 of 256, 52 of 192
+    g = torch.Generator().manual_seed(T)
+    E = (torch.randn(V, H, generator=g) * 0.05).half()
+    x = torch.randn(T, H, generator=g).half()
+    tgt = torch.randint(0, V, (T,), generator=g, dtype=torch.int32)
+    logits = x.float() @ E.float().t()
+    loss_ref, dl_ref, _ = ref.cross_entropy(logits, tgt, ref.valid_rows(1, T))
+    d = ref.Dims(**{**ref.QWEN3_1_7B.__dict__, "n_layers": 1, "vocab": V, "hidden": H,
+                    "intermediate": 512, "n_heads": 2, "n_kv_heads": 1})
+    ctx = llmt.Context(llmt.make_dims(d), 1, T)
+    try:
+        ctx.set_embed_f16(E.to(dev), torch.ones(H, device=dev))
+        loss, dl, dx = ctx.head_ce(x.to(dev), tgt.view(1, T).to(dev), want_dlogits=True)
+        assert abs(loss - float(loss_ref)) < 1e-3
+        assert rel_l2(dl.cpu(), dl_ref) < 1e-4
+        assert rel_l2(dx.cpu(), dl_ref @ E.float()) < 1e-3
+    finally:
+        ctx.close()
