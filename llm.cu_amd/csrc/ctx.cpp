@@ -220,14 +220,14 @@ int Ctx::init() {
         return lora_g + (size_t)l * lora_per_layer + seg_off[2 * proj + is_b];
       };
       const LoraGradJob js[kLoraJobs] = {
-          {s.xn, 1, H, nullptr, H, dhl + 0, 64, g(0, 0), 0},
-          {s.xn, 1, H, nullptr, H, dhl + 16, 64, g(1, 0), 0},
-          {s.xn, 1, H, nullptr, H, dhl + 32, 64, g(2, 0), 0},
-          {s.o16, 1, Q, nullptr, Q, dhl + 48, 64, g(3, 0), 0},
-          {gql, 1, NT, rq(l), Q, s.h + 0, 64, g(0, 1), 1},
-          {gql + Q, 1, NT, rq(l), KV, s.h + 16, 64, g(1, 1), 1},
-          {gql + Q + KV, 1, NT, rq(l), KV, s.h + 32, 64, g(2, 1), 1},
-          {go16(l), 1, H, ro(l), H, s.h + 48, 64, g(3, 1), 1},
+          {s.xn, H, nullptr, H, dhl + 0, 64, g(0, 0), 0},
+          {s.xn, H, nullptr, H, dhl + 16, 64, g(1, 0), 0},
+          {s.xn, H, nullptr, H, dhl + 32, 64, g(2, 0), 0},
+          {s.o16, Q, nullptr, Q, dhl + 48, 64, g(3, 0), 0},
+          {gql, NT, rq(l), Q, s.h + 0, 64, g(0, 1), 1},
+          {gql + Q, NT, rq(l), KV, s.h + 16, 64, g(1, 1), 1},
+          {gql + Q + KV, NT, rq(l), KV, s.h + 32, 64, g(2, 1), 1},
+          {go16(l), H, ro(l), H, s.h + 48, 64, g(3, 1), 1},
       };
       for (int j = 0; j < kLoraJobs; ++j) jobs[(size_t)l * kLoraJobs + j] = js[j];
       if (l == 0)

@@ -9,6 +9,7 @@
 // src/kernels/lora.cu:32-62 (cuRAND, not reproduced: this library draws its
 // own seeded normals).
 #include <algorithm>
+#include <type_traits>
 
 #include "ops.h"
 
@@ -24,76 +25,75 @@ constexpr int NTH = 256;
 //   dA [16, d_in]:  X = adapter input (xn or o, fp16), G = dh  -> out[r][c]
 //   dB [d_out, 16]: X = upstream grad dy,              G = h   -> out[c][r]
 // (dy as the fp16 GEMM operand, row t scaled by the power of two 1 / xs[t],
-// which the G row takes back exactly).  A workgroup owns GC columns of one
-// job.
-constexpr int GC = 256;
-
+// which the G row takes back exactly).
 struct LoraGradGrid {
   int block_start[kLoraJobs + 1];  // column blocks of each job within a layer
 };
 
 // The reduction on the matrix cores in fp32 (v_mfma_f32_16x16x4_f32:
 // out[r][c] = sum over 4 tokens k of G[k][r] X[k][c], so no operand needs a
-// transposition): a workgroup of four waves owns GC columns, wave w the 64
-// columns cb + 64 w .., every wave all T tokens (no cross-wave sum).  Lane
-// l reads G[t + l / 16][l % 16] (times the row factor) as its A value and
-// four consecutive fp16 columns cb + 64 w + 4 (l % 16) .. of X[t + l / 16]
-// as its B values of the four MFMA column tiles (tile nb, MFMA column n
-// stands for column 4 n + nb), so both loads are contiguous rows and each
-// output lane ends up with four consecutive columns or ranks to store.
-template <bool F16>
-__device__ __forceinline__ float4 load_x4s(const void* X, long long off);
-template <>
-__device__ __forceinline__ float4 load_x4s<true>(const void* X, long long off) {
-  const half4 h = *reinterpret_cast<const half4*>((const _Float16*)X + off);
-  return make_float4((float)h[0], (float)h[1], (float)h[2], (float)h[3]);
-}
-template <>
-__device__ __forceinline__ float4 load_x4s<false>(const void* X, long long off) {
-  return *reinterpret_cast<const float4*>((const float*)X + off);
-}
-
+// transposition).  Lane l reads G[t + l / 16][l % 16] (times the row factor)
+// as its A value and CPL consecutive columns c .., c = CPL (l % 16), of X[t +
+// l / 16] as its B values of the CPL MFMA column tiles (tile nb, MFMA column
+// n stands for column CPL n + nb), so both loads are contiguous rows.
+//
+// Bound by its loads (fp32 MFMA floor 0.34 ms for 28 layers at T = 4096, the
+// bytes 0.4 ms): the loads of the next MG_U quads are kept as they come
+// (fp16 X, G and its factor apart) and converted where they are used --
+// converting at the load made every MFMA batch wait for the batch after it
+// (28 layers at T = 4096 1043 -> 827 us with 2 waves, T = 512 142 -> 104).
+// Splitting the tokens over a workgroup's waves instead of 256 columns over
+// 56 workgroups took one layer from 213 to 38 us at T = 4096, 28 layers from
+// 857 to 676 (T = 512 162 -> 91, T = 128 46 -> 35).
 constexpr int MG_U = 4;  // token quads a wave loads ahead
 
-template <bool F16>
-__device__ __forceinline__ void lora_grad_mfma_acc(const LoraGradJob& jb, int T, int col,
-                                                   floatx4 (&acc)[4]) {
+// Tokens [t0, t1) of one wave.
+template <int CPL>
+__device__ __forceinline__ void lora_grad_acc(const LoraGradJob& jb, int t0, int t1, int col,
+                                              floatx4 (&acc)[CPL]) {
+  typedef _Float16 xvec __attribute__((ext_vector_type(CPL)));
   const int lane = threadIdx.x & 63, kq = lane >> 4, r = lane & 15;
-  float gv[MG_U];
-  float4 xv[MG_U];
-  auto load = [&](int t0) {
+  if (t0 >= t1) return;
+  const _Float16* X = jb.X + col;
+  const float* Gc = jb.G + r;
+  float gv[MG_U], fv[MG_U];
+  xvec xv[MG_U];
+  auto load = [&](int tb) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < MG_U; ++u) {
-      const int t = t0 + 4 * u + kq;
-      const int tc = min(t, T - 1);
-      const float f = t < T ? (jb.xs ? jb.xs[tc] : 1.0f) : 0.f;
-      gv[u] = jb.G[(long long)tc * jb.ldg + r] * f;
-      xv[u] = load_x4s<F16>(jb.X, (long long)tc * jb.ldx + col);
+      const int tc = min(tb + 4 * u + kq, t1 - 1);
+      fv[u] = jb.xs ? jb.xs[tc] : 1.0f;
+      gv[u] = Gc[(long long)tc * jb.ldg];
+      xv[u] = *reinterpret_cast<const xvec*>(X + (long long)tc * jb.ldx);
     }
   };
-  load(0);
-  for (int t0 = 0; t0 < T; t0 += 4 * MG_U) {
+  load(t0);
+  for (int tb = t0; tb < t1; tb += 4 * MG_U) {
     float g_c[MG_U];
-    float4 x_c[MG_U];
+    xvec x_c[MG_U];
 #pragma unroll
     for (int u = 0; u < MG_U; ++u) {
-      g_c[u] = gv[u];
+      // tokens past t1 get a zero G value, so they add nothing
+      g_c[u] = tb + 4 * u + kq < t1 ? gv[u] * fv[u] : 0.f;
       x_c[u] = xv[u];
     }
-    if (t0 + 4 * MG_U < T) load(t0 + 4 * MG_U);
+    if (tb + 4 * MG_U < t1) load(tb + 4 * MG_U);
 #pragma unroll
-    for (int u = 0; u < MG_U; ++u) {
-      acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(g_c[u], x_c[u].x, acc[0], 0, 0, 0);
-      acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(g_c[u], x_c[u].y, acc[1], 0, 0, 0);
-      acc[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(g_c[u], x_c[u].z, acc[2], 0, 0, 0);
-      acc[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(g_c[u], x_c[u].w, acc[3], 0, 0, 0);
-    }
+    for (int u = 0; u < MG_U; ++u)
+#pragma unroll
+      for (int nb = 0; nb < CPL; ++nb)
+        acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(g_c[u], (float)x_c[u][nb], acc[nb], 0, 0, 0);
   }
 }
 
-__global__ __launch_bounds__(NTH) void lora_grad_mfma_kernel(const LoraGradJob* __restrict__ jobs,
-                                                             const LoraGradGrid G, int T,
-                                                             float lscale, int accumulate) {
+// W waves a workgroup split the tokens into contiguous ranges, all over the
+// same GC = 16 CPL columns; the W partial 16 x GC blocks are added in LDS in
+// wave order.
+template <int W, int CPL>
+__global__ __launch_bounds__(W * 64) void lora_grad_kernel(const LoraGradJob* __restrict__ jobs,
+                                                           const LoraGradGrid G, int T,
+                                                           float lscale, int accumulate) {
+  constexpr int GC = 16 * CPL;
   const int bpl = G.block_start[kLoraJobs];
   const int layer = (int)blockIdx.x / bpl, lb = (int)blockIdx.x - layer * bpl;
   int j = 0;
@@ -101,132 +101,45 @@ __global__ __launch_bounds__(NTH) void lora_grad_mfma_kernel(const LoraGradJob* 
   for (int i = 1; i < kLoraJobs; ++i)
     if (lb >= G.block_start[i]) j = i;
   const LoraGradJob jb = jobs[layer * kLoraJobs + j];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int c = (lb - G.block_start[j]) * GC + 64 * w + 4 * (lane & 15);  // this lane's columns
-  if ((lb - G.block_start[j]) * GC + 64 * w >= jb.ncols) return;           // wave-uniform
-  const int cc = c < jb.ncols ? c : 0;
-  floatx4 acc[4];
-#pragma unroll
-  for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4{0.f, 0.f, 0.f, 0.f};
-  if (jb.x_f16)
-    lora_grad_mfma_acc<true>(jb, T, cc, acc);
-  else
-    lora_grad_mfma_acc<false>(jb, T, cc, acc);
-  if (c >= jb.ncols) return;
-  // lane: ranks 4 (l / 16) + i of MFMA column l % 16, i.e. columns c .. c + 3
-  const int r0 = 4 * (lane >> 4);
-  if (jb.out_is_B) {  // out[col][16]: four consecutive ranks of each column
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      float4* o = reinterpret_cast<float4*>(jb.out + (long long)(c + nb) * R + r0);
-      const float4 prev = accumulate ? *o : make_float4(0.f, 0.f, 0.f, 0.f);
-      *o = make_float4(prev.x + lscale * acc[nb][0], prev.y + lscale * acc[nb][1],
-                       prev.z + lscale * acc[nb][2], prev.w + lscale * acc[nb][3]);
-    }
-  } else {  // out[16][ncols]: four consecutive columns of each rank
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float4* o = reinterpret_cast<float4*>(jb.out + (long long)(r0 + i) * jb.ncols + c);
-      const float4 prev = accumulate ? *o : make_float4(0.f, 0.f, 0.f, 0.f);
-      *o = make_float4(prev.x + lscale * acc[0][i], prev.y + lscale * acc[1][i],
-                       prev.z + lscale * acc[2][i], prev.w + lscale * acc[3][i]);
-    }
-  }
-}
-
-// Long token ranges: wave w of the four takes token quads w, w + 4, .. for
-// all GC columns of the block (16 MFMA tiles: column group cg of 64, tile
-// nb), loads MG2_U quads ahead, and the four partial 16 x GC blocks are added
-// in LDS in wave order.
-constexpr int MG2_U = 4;
-
-template <bool F16>
-__device__ __forceinline__ void lora_grad_mfma2_acc(const LoraGradJob& jb, int T, int cb, int w,
-                                                    floatx4 (&acc)[4][4]) {
-  const int lane = threadIdx.x & 63, kq = lane >> 4, r = lane & 15;
-  const int nq = (T + 3) / 4;
-  if (w >= nq) return;
-  int colc[4];
-#pragma unroll
-  for (int cg = 0; cg < 4; ++cg) colc[cg] = min(cb + 64 * cg + 4 * r, jb.ncols - 4);
-  float gv[MG2_U];
-  float4 xv[MG2_U][4];
-  auto load = [&](int q0) __attribute__((always_inline)) {  // quads q0, q0 + 4, ..
-#pragma unroll
-    for (int u = 0; u < MG2_U; ++u) {
-      const int t = 4 * (q0 + 4 * u) + kq;
-      const int tc = min(t, T - 1);
-      const float f = t < T ? (jb.xs ? jb.xs[tc] : 1.0f) : 0.f;
-      gv[u] = jb.G[(long long)tc * jb.ldg + r] * f;
-#pragma unroll
-      for (int cg = 0; cg < 4; ++cg) xv[u][cg] = load_x4s<F16>(jb.X, (long long)tc * jb.ldx + colc[cg]);
-    }
-  };
-  load(w);
-  for (int q0 = w; q0 < nq; q0 += 4 * MG2_U) {
-    float g_c[MG2_U];
-    float4 x_c[MG2_U][4];
-#pragma unroll
-    for (int u = 0; u < MG2_U; ++u) {
-      g_c[u] = gv[u];
-#pragma unroll
-      for (int cg = 0; cg < 4; ++cg) x_c[u][cg] = xv[u][cg];
-    }
-    if (q0 + 4 * MG2_U < nq) load(q0 + 4 * MG2_U);
-    // quads past nq carry a zero G value (t >= T), so they add nothing
-#pragma unroll
-    for (int u = 0; u < MG2_U; ++u)
-#pragma unroll
-      for (int cg = 0; cg < 4; ++cg) {
-        acc[cg][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(g_c[u], x_c[u][cg].x, acc[cg][0], 0, 0, 0);
-        acc[cg][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(g_c[u], x_c[u][cg].y, acc[cg][1], 0, 0, 0);
-        acc[cg][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(g_c[u], x_c[u][cg].z, acc[cg][2], 0, 0, 0);
-        acc[cg][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(g_c[u], x_c[u][cg].w, acc[cg][3], 0, 0, 0);
-      }
-  }
-}
-
-__global__ __launch_bounds__(NTH) void lora_grad_mfma2_kernel(const LoraGradJob* __restrict__ jobs,
-                                                              const LoraGradGrid G, int T,
-                                                              float lscale, int accumulate) {
-  const int bpl = G.block_start[kLoraJobs];
-  const int layer = (int)blockIdx.x / bpl, lb = (int)blockIdx.x - layer * bpl;
-  int j = 0;
-#pragma unroll
-  for (int i = 1; i < kLoraJobs; ++i)
-    if (lb >= G.block_start[i]) j = i;
-  const LoraGradJob jb = jobs[layer * kLoraJobs + j];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int cb = (lb - G.block_start[j]) * GC;
-  floatx4 acc[4][4];
+  const int tw = ((T + 4 * W - 1) / (4 * W)) * 4;  // tokens a wave, whole quads
+  const int cc = min(cb + CPL * (lane & 15), jb.ncols - CPL);
+  floatx4 acc[CPL];
 #pragma unroll
-  for (int cg = 0; cg < 4; ++cg)
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) acc[cg][nb] = floatx4{0.f, 0.f, 0.f, 0.f};
-  if (jb.x_f16)
-    lora_grad_mfma2_acc<true>(jb, T, cb, w, acc);
-  else
-    lora_grad_mfma2_acc<false>(jb, T, cb, w, acc);
-  // partial [16 ranks][GC columns] of each wave; column 4 n + nb of group cg
-  __shared__ float red[4][R][GC];
+  for (int nb = 0; nb < CPL; ++nb) acc[nb] = floatx4{0.f, 0.f, 0.f, 0.f};
+  lora_grad_acc<CPL>(jb, w * tw, min(T, (w + 1) * tw), cc, acc);
+  // lane: ranks 4 (l / 16) + i of its CPL columns; the block in the order it
+  // is stored in: out[col][16] (dB) or out[16][col] (dA)
+  __shared__ __attribute__((aligned(16))) float red[W][R * GC];
   const int r0 = 4 * (lane >> 4), n = lane & 15;
+  if (jb.out_is_B) {
 #pragma unroll
-  for (int cg = 0; cg < 4; ++cg)
+    for (int nb = 0; nb < CPL; ++nb)
+      *reinterpret_cast<floatx4*>(&red[w][(CPL * n + nb) * R + r0]) = acc[nb];
+  } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      *reinterpret_cast<float4*>(&red[w][r0 + i][64 * cg + 4 * n]) =
-          make_float4(acc[cg][0][i], acc[cg][1][i], acc[cg][2][i], acc[cg][3][i]);
+#pragma unroll
+      for (int nb = 0; nb < CPL; nb += 4)
+        *reinterpret_cast<float4*>(&red[w][(r0 + i) * GC + CPL * n + nb]) =
+            make_float4(acc[nb][i], acc[nb + 1][i], acc[nb + 2][i], acc[nb + 3][i]);
+  }
   __syncthreads();
-  // thread i finishes column cb + i (all 16 ranks), the waves in order
-  const int col = cb + (int)threadIdx.x;
-  if (col >= jb.ncols) return;
+  for (int e = 4 * threadIdx.x; e < R * GC; e += 4 * W * 64) {
+    float4 v = *reinterpret_cast<const float4*>(&red[0][e]);
 #pragma unroll
-  for (int rr = 0; rr < R; ++rr) {
-    float v = red[0][rr][threadIdx.x];
-#pragma unroll
-    for (int q = 1; q < 4; ++q) v += red[q][rr][threadIdx.x];
-    float* o = jb.out_is_B ? jb.out + (long long)col * R + rr : jb.out + (long long)rr * jb.ncols + col;
-    *o = (accumulate ? *o : 0.f) + lscale * v;
+    for (int q = 1; q < W; ++q) {
+      const float4 x = *reinterpret_cast<const float4*>(&red[q][e]);
+      v = make_float4(v.x + x.x, v.y + x.y, v.z + x.z, v.w + x.w);
+    }
+    const int col = cb + (jb.out_is_B ? e / R : e % GC);
+    if (col >= jb.ncols) continue;
+    float4* o = reinterpret_cast<float4*>(
+        jb.out + (jb.out_is_B ? (long long)cb * R + e : (long long)(e / GC) * jb.ncols + col));
+    const float4 prev = accumulate ? *o : make_float4(0.f, 0.f, 0.f, 0.f);
+    *o = make_float4(prev.x + lscale * v.x, prev.y + lscale * v.y, prev.z + lscale * v.z,
+                     prev.w + lscale * v.w);
   }
 }
 
@@ -500,22 +413,38 @@ hipError_t lora_grad(const LoraGradJob* jobs, const LoraGradPlan& plan, int laye
     set_error("lora_grad: %d layers, T=%d", layers, T);
     return hipErrorInvalidValue;
   }
-  for (int i = 0; i < kLoraJobs; ++i)
-    if (plan.ncols[i] % 4) {
-      set_error("lora_grad: job %d has %d columns (a multiple of 4 is required)", i, plan.ncols[i]);
+  int cols = 0;
+  for (int i = 0; i < kLoraJobs; ++i) {
+    if (plan.ncols[i] % 8) {
+      set_error("lora_grad: job %d has %d columns (a multiple of 8 is required)", i, plan.ncols[i]);
       return hipErrorInvalidValue;
     }
-  LoraGradGrid G{};
-  for (int i = 0; i < kLoraJobs; ++i)
-    G.block_start[i + 1] = G.block_start[i] + (plan.ncols[i] + GC - 1) / GC;
-  const dim3 grid(layers * G.block_start[kLoraJobs]);
-  // short token ranges: one wave a 64-column slice over every token (more
-  // waves in flight); long ones: four waves a block split the tokens
-  // (C4: 0.98 -> 0.86 ms against the fp32 VALU form; C2 57 -> 46 us)
-  if (T <= 512)
-    hipLaunchKernelGGL(lora_grad_mfma_kernel, grid, dim3(NTH), 0, st, jobs, G, T, lscale, accumulate);
-  else
-    hipLaunchKernelGGL(lora_grad_mfma2_kernel, grid, dim3(NTH), 0, st, jobs, G, T, lscale, accumulate);
+    cols += plan.ncols[i];
+  }
+  auto go = [&](auto wc, auto cc) {
+    constexpr int W = decltype(wc)::value, CPL = decltype(cc)::value;
+    LoraGradGrid G{};
+    for (int i = 0; i < kLoraJobs; ++i)
+      G.block_start[i + 1] = G.block_start[i] + (plan.ncols[i] + 16 * CPL - 1) / (16 * CPL);
+    hipLaunchKernelGGL((lora_grad_kernel<W, CPL>), dim3(layers * G.block_start[kLoraJobs]),
+                       dim3(W * 64), 0, st, jobs, G, T, lscale, accumulate);
+  };
+  // 128 columns a workgroup (16-byte X loads, half the loads per MFMA) where
+  // that still fills the CUs, 64 where it does not (one layer: 112 blocks);
+  // as many waves over the tokens as it takes to fill the chip.  28 layers at
+  // T = 4096, us: 64 columns 786 / 773 / 834 with 4 / 8 / 16 waves, 128
+  // columns 676 / 683 / 699; one layer: 49 / 40 / 38 and 70 / 59 / 57.  At T =
+  // 128 28 layers 35 with 2 or 4 waves, 41 with 8.
+  using std::integral_constant;
+  const int blocks = layers * (cols / 128);
+  auto width = [&](auto wc) {
+    if (blocks >= 192) go(wc, integral_constant<int, 8>());
+    else go(wc, integral_constant<int, 4>());
+  };
+  if (blocks < 512 && T >= 1024) width(integral_constant<int, 16>());
+  else if (blocks < 512 && T >= 64) width(integral_constant<int, 8>());
+  else if (T >= 64) width(integral_constant<int, 4>());
+  else width(integral_constant<int, 2>());
   LLMT_LAUNCH_CHECK();
   return hipSuccess;
 }

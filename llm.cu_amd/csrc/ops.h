@@ -317,8 +317,7 @@ hipError_t attn_delta(const void* dO, int dO_is_f16, long long ldd, const _Float
 
 // ---------------------------------------------------------------- LoRA / AdamW
 struct LoraGradJob {
-  const void* X;     // [T, ldx] fp16 or fp32
-  int x_f16;
+  const _Float16* X;  // [T, ldx]
   long long ldx;
   const float* xs;   // NULL, or row t of X stands for X[t] * xs[t]
   int ncols;
