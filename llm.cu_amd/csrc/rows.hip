@@ -944,23 +944,31 @@ __global__ __launch_bounds__(RT) void norm_bwd_kernel(const NormBwdArgs a) {
 // NR rows on MFMA (16 x 16 x 16 fp16: rows x ranks of one adapter times
 // ranks x 16 columns): wave w takes columns 256 w .. of the row, A operand
 // = the rows' dh values (rows past NR zero), scaled by 2^-10 into fp16 range
-// (dh is in the GEMM's scaled units), B operand = 4 consecutive ranks of one
-// column from the transposed copy at [H][48].  The 16 x 16 results go
-// through LDS (out[NR][H], H <= 4 RT) to the thread that owns the column.
+// (dh is in the GEMM's scaled units) and split into two fp16 parts, the value
+// and what its rounding left times 2^11 (22 bits of the fp32 dh, summed
+// apart in fp32), B operand = 4 consecutive ranks of one column from the
+// transposed copy at [H][48].  The 16 x 16 results go through LDS
+// (out[NR][H], H <= 4 RT) to the thread that owns the column.
 constexpr float kLoraMfmaScale = 1.0f / 1024.0f;
+constexpr float kLoraLowScale = 2048.0f;
 
 template <int NR>
 __device__ __forceinline__ void lora_rows_mfma(const NormBwdArgs& a, const float (*hs)[64],
                                                float* out) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int kq = lane >> 4, n = lane & 15;
-  half4 aop[3];
+  half4 aop[3], alo[3];
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
     const float4 h4 = n < NR ? *reinterpret_cast<const float4*>(&hs[n][a.in.term[q].hidx + 4 * kq])
                              : make_float4(0.f, 0.f, 0.f, 0.f);
-    aop[q] = half4{(_Float16)(h4.x * kLoraMfmaScale), (_Float16)(h4.y * kLoraMfmaScale),
-                   (_Float16)(h4.z * kLoraMfmaScale), (_Float16)(h4.w * kLoraMfmaScale)};
+    const float x[4] = {h4.x * kLoraMfmaScale, h4.y * kLoraMfmaScale, h4.z * kLoraMfmaScale,
+                        h4.w * kLoraMfmaScale};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      aop[q][e] = (_Float16)x[e];
+      alo[q][e] = (_Float16)((x[e] - (float)aop[q][e]) * kLoraLowScale);
+    }
   }
   const int H = a.H;
 #pragma unroll
@@ -979,9 +987,13 @@ __device__ __forceinline__ void lora_rows_mfma(const NormBwdArgs& a, const float
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
       acc[nb] = floatx4{0.f, 0.f, 0.f, 0.f};
+      floatx4 low = acc[nb];
 #pragma unroll
-      for (int q = 0; q < 3; ++q)
+      for (int q = 0; q < 3; ++q) {
         acc[nb] = __builtin_amdgcn_mfma_f32_16x16x16f16(aop[q], b[q][nb], acc[nb], 0, 0, 0);
+        low = __builtin_amdgcn_mfma_f32_16x16x16f16(alo[q], b[q][nb], low, 0, 0, 0);
+      }
+      acc[nb] += low * (1.0f / kLoraLowScale);
     }
     // lane: rows 4 kq + i of column cb + 16 nb + n
 #pragma unroll
@@ -998,7 +1010,7 @@ __device__ __forceinline__ void lora_rows_mfma(const NormBwdArgs& a, const float
 }
 
 // LM: 0 no adapter terms, 1 the q/k/v terms on VALU, 2 on MFMA
-// (lora_rows_mfma: 255 -> 229 VGPRs, C4 52.6 -> 45.9 us a layer).
+// (lora_rows_mfma: at 4096 rows 52.6 -> 45 us a layer).
 template <int NR, int LM, bool NT = false>
 __global__ __launch_bounds__(RT) void norm_bwd_rows_kernel(const NormBwdArgs a, int T) {
   constexpr bool LORA = LM > 0;
@@ -1495,15 +1507,16 @@ inline unsigned grid_elems(long long n) {
 // Token rows a workgroup of the parallel-rows epilogues (o_post, resid_norm,
 // norm_bwd with rows of one piece per thread): NR rows side by side share a
 // memory round trip, a barrier pair per reduction and (o_post, the attention
-// norm's backward) the adapter values.  At T >= 2048 each kernel takes the
-// count measured best for it (C4, 4096 rows, us at NR = 1 / 2 / 4 / 8):
-// resid_norm 37.1 / 24.2 / 24.5 / 25.6, norm_bwd 41.5 / 32.1 / 34.5 / 41.7,
-// o_post 52.8 / 32.1 / 30.5 / 35.3, norm_bwd with the three adapter terms
-// 82.3 / 76.7 / 68.0 / 58.7 (its 196 KB of adapter values per workgroup).
-// At short T (the B1 x S128 step) one row a workgroup keeps more CUs busy,
-// except for resid_norm (4.84 against 4.39 us at two rows, 128 rows) and
-// o_post (5.95 against 5.70 us; norm_bwd 5.0 / 5.9 / 9.0, with the adapter
-// terms 8.4 / 9.7 / 13.0 at 1 / 2 / 4 rows).
+// norm's backward) the adapter values.  Up to 768 rows the count that gives
+// every CU one workgroup (a second, partial round of one-row workgroups costs
+// a whole round trip): few rows for few CUs, `small` up to 256 rows, then 2
+// and 3; beyond that what each kernel measured best (us at NR = 1 / 2 / 3 /
+// 4 / 8):
+//   rows                128               624               2000
+//   resid_norm    3.2 3.7 4.5 5.1    9.0 5.9 5.5 6.0    14.6 13.6 14.5 14.0
+//   o_post        5.8 5.6 6.7 7.7    11.5 8.3 7.4 8.2   19.7 16.1 16.2 14.6
+//   norm_bwd      4.3 6.2 7.6 9.9    15.3 11.8 10.4 11.5  21.8 16.0 17.7 16.9
+//   with adapters 7.5 9.0 10 12      23.4 15.7 12.0 13.9  49.6 27.2 24.9 22.7
 // LLMT_ROWS_PER_WG (1, 2, 3, 4 or 8) overrides all of them.
 static int rows_per_wg(int T, int P, int large_t, int small_t = 1) {
   if (P != 1) return 1;
@@ -1512,7 +1525,7 @@ static int rows_per_wg(int T, int P, int large_t, int small_t = 1) {
     const int v = atoi(e);
     if (v == 1 || v == 2 || v == 3 || v == 4 || v == 8) return v;
   }
-  return T >= 2048 ? large_t : small_t;
+  return T <= 256 ? small_t : T <= 512 ? 2 : T <= 768 ? 3 : large_t;
 }
 
 // split_col_ok: the kernel reads its partials through load_row, which alone
@@ -1600,7 +1613,7 @@ hipError_t o_post(const RowIn& in, const float* x_in, const float* w, float eps,
                   float* hbuf, float* x_mid, _Float16* xn2, hipStream_t st) {
   if (!row_in_ok(in, H, "o_post")) return hipErrorInvalidValue;
   const int P = (H + 4 * RT - 1) / (4 * RT);
-  const int nr = rows_per_wg(T, P, 4, 2);
+  const int nr = rows_per_wg(T, P, T >= 1536 ? 4 : 2, 2);
   const dim3 g((T + nr - 1) / nr);
   switch (P * 10 + nr) {
     case 11: hipLaunchKernelGGL((o_post_kernel<1>), g, dim3(RT), 0, st, in, x_in, w, eps, H, hbuf, x_mid, xn2); break;
@@ -1631,7 +1644,7 @@ hipError_t resid_norm(const RowIn& in, const float* x_res, const float* w, float
                       float* x_out, _Float16* xn, hipStream_t st) {
   if (!row_in_ok(in, H, "resid_norm")) return hipErrorInvalidValue;
   const int P = (H + 4 * RT - 1) / (4 * RT);
-  const int nr = rows_per_wg(T, P, 2, 2);
+  const int nr = rows_per_wg(T, P, 2);
   const dim3 g((T + nr - 1) / nr);
   switch (P * 10 + nr) {
     case 11: hipLaunchKernelGGL(resid_norm_kernel<1>, g, dim3(RT), 0, st, in, x_res, w, eps, H, x_out, xn); break;
@@ -1723,9 +1736,9 @@ hipError_t norm_bwd(const NormBwdArgs& a, int T, hipStream_t st) {
       ok = am.in.term[q].c0 == 0 && am.in.term[q].n == a.H && am.in.term[q].hidx == q * R;
     if (!ok) am.lora_at = nullptr;
   }
-  // large T: the VALU LoRA form shares its adapter values over 8 rows; the
-  // MFMA form runs 4 (128 VGPRs, two workgroups a CU: C4 50.7 -> 49.0 us
-  // against 8 rows at 229 VGPRs; 2 rows 59 us)
+  // many rows: the VALU LoRA form shares its adapter values over 8 rows; the
+  // MFMA form runs 4 (128 VGPRs, two workgroups a CU: at 4096 rows 45 us
+  // against 46 at 8 rows and 54 at 2)
   const int nr = rows_per_wg(T, P, lora ? (am.lora_at ? 4 : 8) : 2);
   const dim3 g((T + nr - 1) / nr);
   // the stashed x and the incoming residual gradient are read once: past

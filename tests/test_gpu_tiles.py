@@ -105,3 +105,34 @@ def test_head_row_tiles(dev, T):
         assert rel_l2(dx.cpu(), dl_ref @ E.float()) < 1e-3
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("T", [16, 272, 528, 784])
+def test_layer_row_epilogues_at_row_counts(dev, T):
+    """One small layer at token counts on both sides of the row epilogues'
+    rows-a-workgroup steps (256, 512, 768 rows), adapters large enough for
+    their input-gradient term (split into two fp16 parts on the matrix cores
+    above 256 rows) to dominate dx."""
+    print(f"case: row epilogues T{T}", flush=True)
+    d = ref.Dims(**{**ref.QWEN3_1_7B.__dict__, "n_layers": 1, "vocab": 256, "hidden": 512,
+                    "intermediate": 512, "n_heads": 4, "n_kv_heads": 2})
+    g = torch.Generator().manual_seed(T)
+    lw = make_layer(g, d)
+    ad = make_adapters(g, d, b_std=0.5)[0]
+    x, dy = torch.randn(T, d.hidden, generator=g), torch.randn(T, d.hidden, generator=g)
+    f = lambda t: t.to(torch.float32).to(dev).contiguous()
+    cos, sin = ref.rope_tables(T, d.head_dim, d.theta)
+    y_ref, st = ref.layer_forward(x, lw, ad, d, 1, T, cos, sin)
+    dx_ref, grads_ref = ref.layer_backward(dy, st, lw, ad, d, 1, T, cos, sin)
+    ctx = llmt.Context(llmt.make_dims(d), 1, T)
+    try:
+        ctx.set_layer_f16(0, *(getattr(lw, n).half().to(dev).contiguous() for n in
+                               ("wq", "wk", "wv", "wo", "w_gate", "w_up", "w_down")),
+                          f(lw.attn_norm), f(lw.ffn_norm), f(lw.q_norm), f(lw.k_norm))
+        ctx.lora_set("param", llmt.flatten_adapters([ad]).to(dev))
+        assert rel_l2(ctx.layer_forward(0, x.to(dev), 1).cpu(), y_ref) < GRAD_TOL
+        assert rel_l2(ctx.layer_backward(0, dy.to(dev), 1).cpu(), dx_ref) < GRAD_TOL
+        errs = grad_errors(ctx.lora_get("grad"), [grads_ref], d)
+        assert max(errs.values()) < GRAD_TOL
+    finally:
+        ctx.close()
