@@ -1439,6 +1439,80 @@ __global__ __launch_bounds__(RT) void qk_bwd_kernel(const QkBwdArgs a) {
 }
 
 
+// The layer API's row passes for rows of up to 2048 columns: a wave a row,
+// the row in registers (eight 16-byte loads a lane, one memory round trip and
+// no barrier).  Against the general forms below (a workgroup a row, two
+// passes of 4-byte loads): copy_norm 5.3 -> 4.5 us at 128 rows, 27.7 -> 19.3 at
+// 4096 (84 MB), grad_rows 5.1 -> 4.0 and 33.4 -> 18.7.
+constexpr int WROW = 8;  // 16-byte pieces a lane
+
+__global__ __launch_bounds__(256) void copy_norm_wave_kernel(const float* x,
+                                                             const float* __restrict__ w, float eps,
+                                                             int H, int T, float* x_out,
+                                                             _Float16* __restrict__ xn) {
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (t >= T) return;
+  const float* xr = x + (long long)t * H;
+  float4 v[WROW], ww[WROW];
+#pragma unroll
+  for (int p = 0; p < WROW; ++p) {
+    const int c = min(4 * (lane + 64 * p), H - 4);
+    v[p] = ld4(xr + c);
+    ww[p] = ld4(w + c);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int p = 0; p < WROW; ++p)
+    if (4 * (lane + 64 * p) < H)
+      ss += v[p].x * v[p].x + v[p].y * v[p].y + v[p].z * v[p].z + v[p].w * v[p].w;
+  const float r = rsqrtf(wave_sum(ss) / H + eps);
+#pragma unroll
+  for (int p = 0; p < WROW; ++p) {
+    const int c = 4 * (lane + 64 * p);
+    if (c >= H) continue;
+    *reinterpret_cast<float4*>(x_out + (long long)t * H + c) = v[p];
+    st_h4(xn + (long long)t * H + c, make_float4(v[p].x * r * ww[p].x, v[p].y * r * ww[p].y,
+                                                 v[p].z * r * ww[p].z, v[p].w * r * ww[p].w));
+  }
+}
+
+__global__ __launch_bounds__(256) void grad_rows_wave_kernel(const float* dy, int H, int T,
+                                                             float* dres,
+                                                             _Float16* __restrict__ g16,
+                                                             float* __restrict__ rinv,
+                                                             const _Float16* __restrict__ ks) {
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (t >= T) return;
+  const float* dr = dy + (long long)t * H;
+  float4 v[WROW], g[WROW];
+#pragma unroll
+  for (int p = 0; p < WROW; ++p) {
+    const int c = min(4 * (lane + 64 * p), H - 4);
+    v[p] = ld4(dr + c);
+    g[p] = ks ? ldh4(ks + c) : make_float4(1.f, 1.f, 1.f, 1.f);
+  }
+  float amax = 0.f;
+#pragma unroll
+  for (int p = 0; p < WROW; ++p) {
+    g[p] = mul4v(v[p], g[p]);
+    if (4 * (lane + 64 * p) < H) amax = fmaxf(amax, amax4(g[p]));
+  }
+  amax = wave_max(amax);
+  const float sc = pow2_scale_for(amax);
+  if (lane == 0) rinv[t] = 1.0f / sc;
+#pragma unroll
+  for (int p = 0; p < WROW; ++p) {
+    const int c = 4 * (lane + 64 * p);
+    if (c >= H) continue;
+    *reinterpret_cast<float4*>(dres + (long long)t * H + c) = v[p];
+    st_h4(g16 + (long long)t * H + c, mul4(g[p], sc));
+  }
+}
+// rows the wave forms take: 16-byte pieces of rows of at most 2048 columns
+inline bool wave_rows_ok(const void* a, const void* b, const void* c, int H) {
+  return H % 4 == 0 && H <= 4 * 64 * WROW && ((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) % 16 == 0;
+}
+
 // x_out = x; xn = fp16(rmsnorm(x) * w).
 __global__ __launch_bounds__(RT) void copy_norm_kernel(const float* __restrict__ x,
                                                        const float* __restrict__ w, float eps,
@@ -1543,14 +1617,22 @@ static bool row_in_ok(const RowIn& in, int n, const char* who, bool split_col_ok
 
 hipError_t copy_norm(const float* x, const float* w, float eps, int H, int T, float* x_out,
                      _Float16* xn, hipStream_t st) {
-  hipLaunchKernelGGL(copy_norm_kernel, dim3(T), dim3(RT), 0, st, x, w, eps, H, x_out, xn);
+  if (wave_rows_ok(x, x_out, w, H) && (uintptr_t)xn % 8 == 0)
+    hipLaunchKernelGGL(copy_norm_wave_kernel, dim3((T + 3) / 4), dim3(256), 0, st, x, w, eps, H, T,
+                       x_out, xn);
+  else
+    hipLaunchKernelGGL(copy_norm_kernel, dim3(T), dim3(RT), 0, st, x, w, eps, H, x_out, xn);
   LLMT_LAUNCH_CHECK();
   return hipSuccess;
 }
 
 hipError_t grad_rows(const float* dy, int H, int T, float* dres, _Float16* g16, float* rinv,
                      const _Float16* ks, hipStream_t st) {
-  hipLaunchKernelGGL(grad_rows_kernel, dim3(T), dim3(RT), 0, st, dy, H, dres, g16, rinv, ks);
+  if (wave_rows_ok(dy, dres, dres, H) && ((uintptr_t)g16 | (uintptr_t)ks) % 8 == 0)
+    hipLaunchKernelGGL(grad_rows_wave_kernel, dim3((T + 3) / 4), dim3(256), 0, st, dy, H, T, dres,
+                       g16, rinv, ks);
+  else
+    hipLaunchKernelGGL(grad_rows_kernel, dim3(T), dim3(RT), 0, st, dy, H, dres, g16, rinv, ks);
   LLMT_LAUNCH_CHECK();
   return hipSuccess;
 }

@@ -136,3 +136,30 @@ def test_layer_row_epilogues_at_row_counts(dev, T):
         assert max(errs.values()) < GRAD_TOL
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("T,H", [(16, 512), (48, 2048), (32, 2112)])
+def test_layer_input_alignment(dev, T, H):
+    """The layer API's row passes on inputs that start off a 16-byte boundary
+    (and on rows wider than 2048 columns) against the aligned call: the same
+    values, so the fp32 outputs agree to the rounding of an fp16 operand."""
+    print(f"case: layer input alignment T{T} H{H}", flush=True)
+    d = ref.Dims(**{**ref.QWEN3_1_7B.__dict__, "n_layers": 1, "vocab": 256, "hidden": H,
+                    "intermediate": 256, "n_heads": 2, "n_kv_heads": 1})
+    g = torch.Generator().manual_seed(T + H)
+    lw = make_layer(g, d)
+    ad = make_adapters(g, d)[0]
+    f = lambda t: t.to(torch.float32).to(dev).contiguous()
+    ctx = llmt.Context(llmt.make_dims(d), 1, T)
+    try:
+        ctx.set_layer_f16(0, *(getattr(lw, n).half().to(dev).contiguous() for n in
+                               ("wq", "wk", "wv", "wo", "w_gate", "w_up", "w_down")),
+                          f(lw.attn_norm), f(lw.ffn_norm), f(lw.q_norm), f(lw.k_norm))
+        ctx.lora_set("param", llmt.flatten_adapters([ad]).to(dev))
+        x, dy = torch.randn(T, H, generator=g).to(dev), torch.randn(T, H, generator=g).to(dev)
+        off = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(T, H)
+        y, dx = ctx.layer_forward(0, x, 1), ctx.layer_backward(0, dy, 1)
+        y2, dx2 = ctx.layer_forward(0, off(x), 1), ctx.layer_backward(0, off(dy), 1)
+        assert rel_l2(y2.cpu(), y.cpu()) < 1e-3 and rel_l2(dx2.cpu(), dx.cpu()) < 1e-3
+    finally:
+        ctx.close()
