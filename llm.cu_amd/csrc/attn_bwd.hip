@@ -295,7 +295,7 @@ __device__ __forceinline__ void kv_accum(const _Float16* Qs, const _Float16* Ds,
 // each phase its own scheduling region with the LDS reads issued ahead of the
 // MFMAs.  (Interleaving one half's dS VALU with the other half's MFMAs was
 // measured slower at B4 x S2048: 277 against 255 us.)
-template <bool MASK>
+template <bool MASK, int QT = BLK>
 __device__ __forceinline__ void kv_tile(const _Float16* Qs, const _Float16* Ds,
                                         const float* lse_s, const float* del_s,
                                         const float* dsc_s, const half8 (&kf)[4],
@@ -303,7 +303,7 @@ __device__ __forceinline__ void kv_tile(const _Float16* Qs, const _Float16* Ds,
                                         floatx4 (&dvT)[8], float sl2, float gs, int qq0, int key,
                                         int S, int lane) {
 #pragma unroll
-  for (int j2 = 0; j2 < 2; ++j2) {
+  for (int j2 = 0; j2 < QT / 32; ++j2) {
     floatx4 p[2], ds[2];
     kv_scores(Qs, Ds, kf, vf, j2, p, ds, lane);
     sched_reads_ahead<16, 16, 6, 2, 2, 0>();
@@ -428,17 +428,17 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs& a, _Float16* buf0, _F
 
 // Small grids (the B1 x S128 step: 8 KV heads x 8 key blocks): the NW waves
 // of the workgroup all own the same 16 keys and split the group's
-// (query head, query tile) iterations between them (wave w takes it = w,
-// w + NW, ..), each through LDS buffers of its own (no barriers in the
-// loop); their dK/dV sums meet in LDS at the end, in wave order.  Two waves
-// keep two buffers each (the next tile lands during the current one); four
-// waves one each (4 x 33.5 KB of LDS), refilled once the wave's reads of it
-// have returned -- at B1 x S128 (2 query heads x 2 tiles) each wave then
-// has a single iteration.
-template <int NW>
-constexpr int split_bufs() { return NW >= 4 ? 1 : 2; }
+// (query head, QT-query tile) iterations between them (wave w takes it = w,
+// w + NW, ..), each through an LDS buffer of its own (no barriers in the
+// loop), refilled once the wave's reads of it have returned; their dK/dV sums
+// meet in LDS at the end, in wave order.  Tiles of 32 queries (17 KB a wave)
+// leave room for two workgroups a CU, whose waves hide each other's refills:
+// against 64-query tiles at one workgroup a CU, B1 x S512 26.8 -> 22.9 us, B3
+// x S208 20.2 -> 13.5, B1 x S128 8.5 -> 8.2.
+// halves of a wave's buffer
+constexpr int split_buf(int qt) { return 2 * qt * HD + 3 * BLK * 2; }
 
-template <int NW>
+template <int NW, int QT>
 __device__ __forceinline__ void dkdv_block_split(const AttnArgs& a, _Float16* smem, float* red,
                                                  int kb, int j, int b) {
   constexpr int NT = NW * 64;
@@ -450,23 +450,22 @@ __device__ __forceinline__ void dkdv_block_split(const AttnArgs& a, _Float16* sm
   const long long rowb = (long long)b * S;
   const int k0 = kb * 16;
   const float sl2 = a.sm_scale * LOG2E;
-  const int qb0 = k0 / BLK;
-  const int nqt = (S + BLK - 1) / BLK - qb0;
+  const int qb0 = k0 / QT;
+  const int nqt = (S + QT - 1) / QT - qb0;
   const int niter = group * nqt;
-  constexpr int NB = split_bufs<NW>();
-  _Float16* mine = smem + w * NB * KV_BUF;
-  TileDma<1> dq_, dd_;
+  _Float16* mine = smem + w * split_buf(QT);
+  TileDma<1, QT> dq_, dd_;
   dq_.init(a.ldq, 0);
   dd_.init(a.ld16, 0);
   auto issue = [&](int it, _Float16* buf) {
     const int h = j * group + it / nqt, qb = qb0 + it % nqt;
-    dq_.issue(a.q + rowb * a.ldq + h * HD, a.ldq, qb * BLK, S, buf, 0);
-    dd_.issue(a.dO16 + rowb * a.ld16 + h * HD, a.ld16, qb * BLK, S, buf + TILE, 0);
-    float* vec = reinterpret_cast<float*>(buf + 2 * TILE);
+    dq_.issue(a.q + rowb * a.ldq + h * HD, a.ldq, qb * QT, S, buf, 0);
+    dd_.issue(a.dO16 + rowb * a.ld16 + h * HD, a.ld16, qb * QT, S, buf + QT * HD, 0);
+    float* vec = reinterpret_cast<float*>(buf + 2 * QT * HD);
     const long long bh = ((long long)b * a.nq + h) * S;
-    dma_vec64(a.lse + bh, qb * BLK, S, vec);
-    dma_vec64(a.delta + bh, qb * BLK, S, vec + BLK);
-    dma_vec64(a.dsc + bh, qb * BLK, S, vec + 2 * BLK);
+    dma_vec64(a.lse + bh, qb * QT, S, vec);
+    dma_vec64(a.delta + bh, qb * QT, S, vec + BLK);
+    dma_vec64(a.dsc + bh, qb * QT, S, vec + 2 * BLK);
   };
   if (w < niter) issue(w, mine);
   const float gs = group_do_scale<NT>(a.dsc, b, a.nq, j, group, S, red);
@@ -482,37 +481,26 @@ __device__ __forceinline__ void dkdv_block_split(const AttnArgs& a, _Float16* sm
     dkT[i] = floatx4{0.f, 0.f, 0.f, 0.f};
     dvT[i] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
-  int n = 0;
-  for (int it = w; it < niter; it += NW, ++n) {
-    wait_vm<0>();  // this wave's own tile (its buffers are private)
+  for (int it = w; it < niter; it += NW) {
+    wait_vm<0>();  // this wave's own tile (its buffer is private)
     asm volatile("" ::: "memory");
-    if constexpr (NB == 2)
-      if (it + NW < niter) issue(it + NW, mine + ((n + 1) & 1) * KV_BUF);
-    const _Float16* buf = mine + (NB == 2 ? (n & 1) * KV_BUF : 0);
     const int qb = qb0 + it % nqt;
-    if (qb * BLK + BLK - 1 < k0) {
-      if constexpr (NB == 1)
-        if (it + NW < niter) issue(it + NW, mine);
-      continue;
-    }
-    const _Float16* Qs = buf;
-    const _Float16* Ds = buf + TILE;
-    const float* lse_s = reinterpret_cast<const float*>(buf + 2 * TILE);
+    const _Float16* Qs = mine;
+    const _Float16* Ds = mine + QT * HD;
+    const float* lse_s = reinterpret_cast<const float*>(mine + 2 * QT * HD);
     const float* del_s = lse_s + BLK;
     const float* dsc_s = lse_s + 2 * BLK;
-    const bool full = qb * BLK >= k0 + 15 && qb * BLK + BLK <= S;
+    const bool full = qb * QT >= k0 + 15 && qb * QT + QT <= S;
     if (full)
-      kv_tile<false>(Qs, Ds, lse_s, del_s, dsc_s, kf, vf, dkT, dvT, sl2, gs, qb * BLK, k0 + c, S,
-                     lane);
+      kv_tile<false, QT>(Qs, Ds, lse_s, del_s, dsc_s, kf, vf, dkT, dvT, sl2, gs, qb * QT, k0 + c,
+                         S, lane);
     else
-      kv_tile<true>(Qs, Ds, lse_s, del_s, dsc_s, kf, vf, dkT, dvT, sl2, gs, qb * BLK, k0 + c, S,
-                    lane);
-    if constexpr (NB == 1) {
-      if (it + NW < niter) {  // one buffer: refill it once this tile's reads returned
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-        asm volatile("" ::: "memory");
-        issue(it + NW, mine);
-      }
+      kv_tile<true, QT>(Qs, Ds, lse_s, del_s, dsc_s, kf, vf, dkT, dvT, sl2, gs, qb * QT, k0 + c, S,
+                        lane);
+    if (it + NW < niter) {  // refill the buffer once this tile's reads returned
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+      asm volatile("" ::: "memory");
+      issue(it + NW, mine);
     }
   }
   // waves 1 .. NW-1 hand their sums to wave 0, which adds them in order
@@ -545,25 +533,28 @@ __device__ __forceinline__ void dkdv_block_split(const AttnArgs& a, _Float16* sm
 // the last batches' 178 us key blocks started only once earlier ones had
 // drained, leaving a tail at half occupancy for 45% of the dK/dV launch).
 // PART 0: both kinds; 1: dK/dV only; 2: dQ only -- the one-kind forms keep
-// their own (smaller) register and LDS budgets.
+// their own (smaller) register and LDS budgets; 4: both, dK/dV blocks of 16
+// keys split over the waves in tiles of 32 queries.
 constexpr int BWD_BUF = KV_BUF > 2 * TILE ? KV_BUF : 2 * TILE;  // halves per buffer
 
 template <int NW, int RW, int PART>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void attn_bwd_kernel(const AttnArgs a, int nkvb, int nqb) {
   // PART 0-2: the two tile buffers as separate arrays (statically named
-  // buffers, see dq_block); PART 3: one array split per wave.
+  // buffers, see dq_block); 4: one array split per wave.
   constexpr int BUF = PART == 1 ? KV_BUF : PART == 2 ? 2 * TILE : BWD_BUF;
-  constexpr int SMEM3 = NW * split_bufs<NW>() * KV_BUF > 4 * TILE ? NW * split_bufs<NW>() * KV_BUF : 4 * TILE;
-  __shared__ __attribute__((aligned(1024))) _Float16 buf0[PART == 3 ? SMEM3 : BUF];
-  __shared__ __attribute__((aligned(1024))) _Float16 buf1[PART == 3 ? 8 : BUF];
+  constexpr bool SPLIT = PART == 4;
+  constexpr int QT = 32;
+  constexpr int SMEM4 = NW * split_buf(QT) > 4 * TILE ? NW * split_buf(QT) : 4 * TILE;
+  __shared__ __attribute__((aligned(1024))) _Float16 buf0[SPLIT ? SMEM4 : BUF];
+  __shared__ __attribute__((aligned(1024))) _Float16 buf1[SPLIT ? 8 : BUF];
   __shared__ float red[NW];
   const int x = blockIdx.y, b = blockIdx.x;
   const int nkvx = PART == 2 ? 0 : nkvb * a.nkv;
   if constexpr (PART != 2) {
     if (x < nkvx) {
-      if constexpr (PART == 3)
-        dkdv_block_split<NW>(a, buf0, red, x / a.nkv, x % a.nkv, b);
+      if constexpr (SPLIT)
+        dkdv_block_split<NW, QT>(a, buf0, red, x / a.nkv, x % a.nkv, b);
       else
         dkdv_block<NW, 1>(a, buf0, buf1, red, x / a.nkv, x % a.nkv, b);
       return;
@@ -571,7 +562,7 @@ void attn_bwd_kernel(const AttnArgs a, int nkvb, int nqb) {
   }
   if constexpr (PART != 1) {
     const int y = x - nkvx;
-    if constexpr (PART == 3)
+    if constexpr (SPLIT)
       dq_block<NW, RW>(a, buf0, buf0 + 2 * TILE, nqb - 1 - y / a.nq, y % a.nq, b);
     else
       dq_block<NW, RW>(a, buf0, buf1, nqb - 1 - y / a.nq, y % a.nq, b);
@@ -648,17 +639,30 @@ hipError_t attn_bwd(const AttnArgs& a, int B, hipStream_t st) {
   // a wave are (attention backward 54.4 against 58.4 us), the dQ blocks then
   // being as long as the dK/dV ones.  LLMT_ATTN_CFG still selects any shape.
   AttnShape s = attn_shape(B, a.S, a.nq);
+  int nwk = dkdv_waves(B, a.S, a.nkv);
   if (!getenv("LLMT_ATTN_CFG")) {
-    if (!bwd_one_launch(a, B, dkdv_waves(B, a.S, a.nkv), s.nw, s.rw)) s.rw = 1;
-    // tiny grids (the B1 x S128 step): dK/dV blocks of 16 keys whose four
-    // waves split the group's query tiles, beside 64-query dQ blocks
-    if (!getenv("LLMT_ATTN_DKDV_WAVES") && (long long)B * a.nq * ((a.S + 63) / 64) < 64) {
-      launch_bwd<4, 1, 3>(a, B, (a.S + 15) / 16, (a.S + 63) / 64, st);
-      LLMT_LAUNCH_CHECK();
-      return hipSuccess;
+    if (!getenv("LLMT_ATTN_DKDV_WAVES")) {
+      // Small grids are serial chains on few CUs: dK/dV blocks of 16 keys
+      // whose four waves split the group's 32-query tiles, beside 64-query dQ
+      // blocks (two workgroups a CU), while both kinds are at most 800
+      // workgroups.  Against 32-key blocks of two waves, us: B1 x S128 11.7
+      // -> 8.2, B1 x S256 18.3 -> 12.1, B3 x S208 20.8 -> 13.5, B1 x S512 31.9
+      // -> 22.9, B1 x S1024 75.5 -> 45.4; beyond (B8 x S256) 24.7 against 33.2.
+      const long long n = (long long)B * (a.nkv * (long long)((a.S + 15) / 16) +
+                                          a.nq * (long long)((a.S + 63) / 64));
+      if (n <= 800) {
+        launch_bwd<4, 1, 4>(a, B, (a.S + 15) / 16, (a.S + 63) / 64, st);
+        LLMT_LAUNCH_CHECK();
+        return hipSuccess;
+      }
+      // one launch for both kinds needs one wave count: two launches of
+      // blocks of different widths run one after the other (B3 x S512 51.5 us
+      // against 37.3, B1 x S1536 115 against 89)
+      if (nwk != s.nw && bwd_one_launch(a, B, s.nw, s.nw, s.rw)) nwk = s.nw;
     }
+    if (!bwd_one_launch(a, B, nwk, s.nw, s.rw)) s.rw = 1;
   }
-  launch_attn_bwd(a, B, dkdv_waves(B, a.S, a.nkv), s.nw, s.rw, st);
+  launch_attn_bwd(a, B, nwk, s.nw, s.rw, st);
   LLMT_LAUNCH_CHECK();
   return hipSuccess;
 }

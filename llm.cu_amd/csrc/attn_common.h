@@ -60,7 +60,7 @@ __device__ __forceinline__ void tile_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// DMA of 64-row tiles through buffer loads with an LDS destination: rows
+// DMA of 64- (or ROWS-) row tiles through buffer loads with an LDS destination: rows
 // past the end of the matrix fall outside the buffer and arrive as zeros.
 // Wave w moves the 1 KB chunks w, w + NW, ...: chunk ch holds tile rows
 // 4 ch .. 4 ch + 3; lane l fills slot l % 16 of row 4 ch + l / 16.  The
@@ -77,25 +77,26 @@ __device__ __forceinline__ void buffer_lds4(__amdgpu_buffer_rsrc_t rs, void* lds
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)lds, 4, off, 0, 0, 0);
 }
 
-template <int NW>
+template <int NW, int ROWS = BLK>
 struct TileDma {
-  unsigned off[16 / NW];
+  static constexpr int CH = ROWS / 4 / NW;  // chunks a wave
+  unsigned off[CH];
   __device__ __forceinline__ void init(long long ld, int w) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int i = 0; i < 16 / NW; ++i) {
+    for (int i = 0; i < CH; ++i) {
       const int r = 4 * (w + NW * i) + (lane >> 4);
       off[i] = (unsigned)(r * ld * 2 + (((lane & 15) ^ swz(r)) << 4));
     }
   }
-  // Rows r0 .. r0 + 63 of `src` ([nrows, ld] fp16) into `tile`.
+  // Rows r0 .. r0 + ROWS - 1 of `src` ([nrows, ld] fp16) into `tile`.
   __device__ __forceinline__ void issue(const _Float16* src, long long ld, int r0, int nrows,
                                         _Float16* tile, int w) const {
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(src + (long long)r0 * ld), (short)0, (int)((long long)(nrows - r0) * ld * 2),
         kRsrcWord3);
 #pragma unroll
-    for (int i = 0; i < 16 / NW; ++i)
+    for (int i = 0; i < CH; ++i)
       buffer_lds16(rs, tile + (w + NW * i) * 512, off[i]);
   }
 };

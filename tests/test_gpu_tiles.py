@@ -163,3 +163,39 @@ def test_layer_input_alignment(dev, T, H):
         assert rel_l2(y2.cpu(), y.cpu()) < 1e-3 and rel_l2(dx2.cpu(), dx.cpu()) < 1e-3
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("B,S,nq,nkv", [(1, 33, 16, 8), (2, 47, 8, 8), (1, 250, 32, 8),
+                                        (1, 530, 16, 8), (3, 333, 16, 8), (2, 700, 16, 8),
+                                        (1, 1100, 8, 4)])
+def test_attention_grid_sizes(dev, B, S, nq, nkv):
+    """The attention backward on both sides of its small-grid rule (16-key
+    blocks split over four waves in 32-query tiles, then one launch, then
+    two), ragged S, through the operators and the fused block."""
+    print(f"case: attention B{B} S{S} nq{nq} nkv{nkv}", flush=True)
+    g = torch.Generator().manual_seed(3 * S + nq)
+    q = torch.randn(B, S, nq, 128, generator=g).half()
+    k = torch.randn(B, S, nkv, 128, generator=g).half()
+    v = torch.randn(B, S, nkv, 128, generator=g).half()
+    do = torch.randn(B, S, nq, 128, generator=g)
+    o_ref, lse_ref = ref.attention_fwd(q.float(), k.float(), v.float())
+    qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
+    o, lse = llmt.attention_fwd(qd, kd, vd)
+    assert rel_l2(o.float().cpu(), o_ref) < 2e-3
+    assert (lse.cpu() - lse_ref).abs().max() < 1e-3
+    want = ref.attention_bwd(do, q.float(), k.float(), v.float(), o.float().cpu(), lse.cpu())
+    for a, b in zip(llmt.attention_bwd(qd, kd, vd, o, lse, do.to(dev)), want):
+        assert rel_l2(a.cpu(), b) < GRAD_TOL
+    # the block on inputs whose norm and rotation the oracle applies
+    cos, sin = ref.rope_tables(S, 128, 1e6)
+    one = torch.ones(128)
+    rot = lambda t: ref.rope_fwd(ref.rmsnorm(t.float(), one, 1e-6), cos, sin)
+    x = [t.float().requires_grad_() for t in (q, k)]
+    with torch.enable_grad():
+        qr, kr = (rot(t) for t in x)
+    od, ld = ref.attention_fwd(qr.detach(), kr.detach(), v.float())
+    dqr, dkr, dv_ref = ref.attention_bwd(do.half().float(), qr.detach(), kr.detach(), v.float(), od, ld)
+    dq_ref, dk_ref = torch.autograd.grad((qr, kr), x, (dqr, dkr))
+    got = llmt.attention_block_bwd(qd, kd, vd, one.to(dev), one.to(dev), do.half().to(dev))
+    for a, b in zip(got, (dq_ref, dk_ref, dv_ref)):
+        assert rel_l2(a.cpu(), b) < GRAD_TOL
