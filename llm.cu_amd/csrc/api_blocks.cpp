@@ -39,20 +39,30 @@ using namespace llmt;
 
 static Ctx* C_(llmt_ctx* c) { return reinterpret_cast<Ctx*>(c); }
 
-// Temporary device buffers released (stream-ordered) on scope exit.
+// Temporary device buffers of one call: sub-buffers (256-byte aligned) of a
+// single stream-ordered allocation, released on scope exit.  Every get() asks
+// for its size while `base` is NULL; alloc() then makes the one allocation
+// and the same get() calls, in the same order, return the sub-buffers.  (One
+// allocation and free a call instead of one a buffer: the attention backward
+// of B3 x S333 67 -> 49 us a forward + backward, 43 us of it kernels.)
 struct Temps {
   hipStream_t st;
-  std::vector<void*> ptrs;
+  char* base = nullptr;
+  size_t used = 0, total = 0;
   explicit Temps(hipStream_t s) : st(s) {}
   template <class T>
   T* get(size_t n) {
-    void* p = nullptr;
-    if (hipMallocAsync(&p, n * sizeof(T) + 256, st) != hipSuccess) return nullptr;
-    ptrs.push_back(p);
-    return static_cast<T*>(p);
+    char* p = base ? base + used : nullptr;
+    used += (n * sizeof(T) + 511) & ~(size_t)255;
+    return reinterpret_cast<T*>(p);
+  }
+  bool alloc() {
+    total = used;
+    used = 0;
+    return hipMallocAsync((void**)&base, total, st) == hipSuccess;
   }
   ~Temps() {
-    for (void* p : ptrs) (void)hipFreeAsync(p, st);
+    if (base) (void)hipFreeAsync(base, st);
   }
 };
 
@@ -254,17 +264,23 @@ int llmt_lm_head_ce(const void* hidden, const void* W, const int* targets, int T
           "llmt_lm_head_ce: T %% 16, T %% seq_len, H %% 32, V %% 32 must be 0");
   hipStream_t st = (hipStream_t)stream;
   Temps tmp(st);
-  _Float16* E = tmp.get<_Float16>((size_t)V * H);
-  _Float16* ET = tmp.get<_Float16>((size_t)V * H);
-  float* logits = tmp.get<float>((size_t)T * V);
-  _Float16* g16 = tmp.get<_Float16>((size_t)T * V);
-  float2* stats = tmp.get<float2>((size_t)T * ce_stats_per_row(V));
-  float* rows = tmp.get<float>(T);
-  float* lse = tmp.get<float>(T);
+  _Float16 *E, *ET, *g16;
+  float *logits, *rows, *lse, *part;
+  float2* stats;
   const size_t pe = (size_t)gemm_pick_split(T, H, V, 64, false) * T * H;
-  float* part = tmp.get<float>(pe);
-  TRY_ARG(E && ET && logits && g16 && stats && rows && lse && part,
-          "llmt_lm_head_ce: out of memory");
+  auto layout = [&]() {
+    E = tmp.get<_Float16>((size_t)V * H);
+    ET = tmp.get<_Float16>((size_t)V * H);
+    logits = tmp.get<float>((size_t)T * V);
+    g16 = tmp.get<_Float16>((size_t)T * V);
+    stats = tmp.get<float2>((size_t)T * ce_stats_per_row(V));
+    rows = tmp.get<float>(T);
+    lse = tmp.get<float>(T);
+    part = tmp.get<float>(pe);
+  };
+  layout();
+  TRY_ARG(tmp.alloc(), "llmt_lm_head_ce: out of memory");
+  layout();
   TRY_HIP(pack_f16((const _Float16*)W, H, 0, V, H, E, H, 0, 0, st));
   TRY_HIP(pack_f16((const _Float16*)W, H, 1, H, V, ET, V, 0, 0, st));
   return head_ce_packed(st, (const _Float16*)hidden, E, ET, targets, T, seq_len, H, V, logits, g16,
@@ -309,10 +325,16 @@ int llmt_attention_bwd(const void* q, const void* k, const void* v, const void* 
   hipStream_t st = (hipStream_t)stream;
   const int T = B * S;
   Temps tmp(st);
-  float* delta = tmp.get<float>((size_t)B * nq * S);
-  float* dsc = tmp.get<float>((size_t)T * nq);
-  _Float16* dO16 = tmp.get<_Float16>((size_t)T * nq * kHeadDim);
-  TRY_ARG(delta && dsc && dO16, "llmt_attention_bwd: out of memory");
+  float *delta, *dsc;
+  _Float16* dO16;
+  auto layout = [&]() {
+    delta = tmp.get<float>((size_t)B * nq * S);
+    dsc = tmp.get<float>((size_t)T * nq);
+    dO16 = tmp.get<_Float16>((size_t)T * nq * kHeadDim);
+  };
+  layout();
+  TRY_ARG(tmp.alloc(), "llmt_attention_bwd: out of memory");
+  layout();
   const long long ldq = (long long)nq * kHeadDim, ldkv = (long long)nkv * kHeadDim;
   TRY_HIP(attn_delta(dout, 0, ldq, (const _Float16*)o, ldq, nq, S, T, delta, dO16, ldq, dsc, st));
   AttnArgs a{};
