@@ -22,12 +22,12 @@ namespace {
 #define LLMT_INLINE __attribute__((always_inline))
 
 // ---------------------------------------------------------------- forward
-// One 64-key tile of the online softmax for RW 16-query tiles of a wave:
-// st holds the raw scores (rows key, column query); on return the fp32
+// One tile of 16 MT keys of the online softmax for RW 16-query tiles of a
+// wave: st holds the raw scores (rows key, column query); on return the fp32
 // probabilities relative to the running max, with m, l and the output
 // accumulators rescaled.  MASK: apply causality / sequence end.
-template <int RW, bool MASK>
-__device__ __forceinline__ void softmax_tile(floatx4 (&st)[RW][4], float (&m)[RW], float (&l)[RW],
+template <int RW, bool MASK, int MT = 4>
+__device__ __forceinline__ void softmax_tile(floatx4 (&st)[RW][MT], float (&m)[RW], float (&l)[RW],
                                              floatx4 (&ot)[RW][8], float sl2, int key0, int q0,
                                              int S, int lane) {
   const int c = lane & 15, g = lane >> 4;
@@ -36,7 +36,7 @@ __device__ __forceinline__ void softmax_tile(floatx4 (&st)[RW][4], float (&m)[RW
     const int q = q0 + 16 * r + c;
     float bm = -INFINITY;
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         float s = st[r][mt][v];
@@ -53,14 +53,17 @@ __device__ __forceinline__ void softmax_tile(floatx4 (&st)[RW][4], float (&m)[RW
     const float alpha = __builtin_amdgcn_exp2f(m[r] - mu);
     m[r] = mn;
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int v = 0; v < 4; ++v) st[r][mt][v] = __builtin_amdgcn_exp2f(fmaf(st[r][mt][v], sl2, -mu));
     // row sum as a tree (independent adds) rather than one serial chain
-    float ps4[4];
+    float ps[MT];
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) ps4[mt] = (st[r][mt][0] + st[r][mt][1]) + (st[r][mt][2] + st[r][mt][3]);
-    l[r] = l[r] * alpha + ((ps4[0] + ps4[1]) + (ps4[2] + ps4[3]));
+    for (int mt = 0; mt < MT; ++mt) ps[mt] = (st[r][mt][0] + st[r][mt][1]) + (st[r][mt][2] + st[r][mt][3]);
+    if constexpr (MT == 4)
+      l[r] = l[r] * alpha + ((ps[0] + ps[1]) + (ps[2] + ps[3]));
+    else
+      l[r] = l[r] * alpha + (ps[0] + ps[1]);
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) ot[r][dt] *= alpha;
   }
@@ -232,6 +235,201 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(const AttnArgs a) {
   }
 }
 
+// Small grids: workgroup (16 RW queries q0 .., head h, batch b), the causal
+// range of keys split over its four waves in 32-key tiles w, w + 4, ..; each
+// wave keeps its own running softmax, and the four are merged through LDS at
+// the end (in wave order).  attn_fwd_kernel's waves walk every key tile of
+// their queries, up to S / 64 in a row, each a serial chain of LDS reads,
+// MFMAs, softmax and a barrier: on a chip that is not full that chain is the
+// time (B1 x S512: 11.4 us, here 8.6; 0.5 GFLOP).  Here it is a quarter as
+// long and has no barrier: a wave's K and V tiles are its own, the next K tile
+// is fetched when the scores are done, the next V tile when the output is (16
+// KB a wave, two workgroups a CU; the register bound keeps both resident).
+constexpr int FS_KEYS = 32;
+
+template <int RW>
+__global__ __launch_bounds__(256, 2) void attn_fwd_split_kernel(const AttnArgs a) {
+  constexpr int NW = 4, FT = FS_KEYS * HD;
+  __shared__ __attribute__((aligned(1024))) _Float16 kbuf[NW * FT];
+  __shared__ __attribute__((aligned(1024))) _Float16 vbuf[NW * FT];
+  __shared__ float2 ml[NW][RW * 16];  // (max, sum) of a query's keys in each wave
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int q0 = 16 * RW * (gridDim.z - 1 - blockIdx.z), h = blockIdx.x, b = blockIdx.y;
+  const int S = a.S;
+  const int kvh = h / (a.nq / a.nkv);
+  const long long rowb = (long long)b * S;
+  const float sl2 = a.sm_scale * LOG2E;
+  const _Float16* kbase = a.k + rowb * a.ldk + kvh * HD;
+  const _Float16* vbase = a.v + rowb * a.ldv + kvh * HD;
+  const int nkt = (min(q0 + 16 * RW, S) + FS_KEYS - 1) / FS_KEYS;
+  _Float16* const Ks = kbuf + w * FT;
+  _Float16* const Vs = vbuf + w * FT;
+  using Dma = TileDma<1, FS_KEYS>;
+  Dma dk, dv;
+  dk.init(a.ldk, 0);
+  dv.init(a.ldv, 0);
+  if (w < nkt) {
+    dk.issue(kbase, a.ldk, w * FS_KEYS, S, Ks, 0);
+    dv.issue(vbase, a.ldv, w * FS_KEYS, S, Vs, 0);
+  }
+  half8 qf[RW][4];
+  if (a.qn) {  // as in attn_fwd_kernel; wave 0 stores q16w
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+      const int q = q0 + 16 * r + c, qc = min(q, S - 1);
+      norm_rope_frag(qf[r], a.qraw + (rowb + qc) * a.ldqr + h * HD, a.qn, a.cosT, a.sinT, qc,
+                     a.eps, g);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        if (q >= S)
+          qf[r][ks] = half8{};
+        else if (w == 0)
+          *reinterpret_cast<half8*>(a.q16w + (rowb + q) * a.ldq + h * HD + 32 * ks + 8 * g) =
+              qf[r][ks];
+      }
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+        qf[r][ks] = frag_global(a.q + rowb * a.ldq + h * HD, a.ldq, q0 + 16 * r + c, S, ks, lane);
+  }
+  floatx4 ot[RW][8];
+  float m[RW], l[RW];
+#pragma unroll
+  for (int r = 0; r < RW; ++r) {
+    m[r] = -INFINITY;
+    l[r] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ot[r][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  wait_vm<0>();
+  for (int kt = w; kt < nkt; kt += NW) {
+    const bool next = kt + NW < nkt;
+    if (kt != w) wait_vm<Dma::CH>();  // this K tile (the V tile may be in flight)
+    asm volatile("" ::: "memory");
+    floatx4 st[RW][2];
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+#pragma unroll
+      for (int r = 0; r < RW; ++r) st[r][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const half8 kf = frag_rm(Ks, mt * 16, ks, lane);
+#pragma unroll
+        for (int r = 0; r < RW; ++r) st[r][mt] = mfma16(kf, qf[r][ks], st[r][mt]);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the reads of the K tile have returned
+    asm volatile("" ::: "memory");
+    if (next) dk.issue(kbase, a.ldk, (kt + NW) * FS_KEYS, S, Ks, 0);
+    if (kt * FS_KEYS + FS_KEYS - 1 <= q0 && kt * FS_KEYS + FS_KEYS <= S)
+      softmax_tile<RW, false, 2>(st, m, l, ot, sl2, kt * FS_KEYS, q0, S, lane);
+    else
+      softmax_tile<RW, true, 2>(st, m, l, ot, sl2, kt * FS_KEYS, q0, S, lane);
+    half8 pb[RW];
+#pragma unroll
+    for (int r = 0; r < RW; ++r) pb[r] = pair_frag(st[r][0], st[r][1]);
+    if (next) wait_vm<Dma::CH>();  // this V tile (the next K tile may be in flight)
+    else wait_vm<0>();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) {
+      const half8 vf = frag_tr(Vs, dt * 16, 0, lane);
+#pragma unroll
+      for (int r = 0; r < RW; ++r) ot[r][dt] = mfma16(vf, pb[r], ot[r][dt]);
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    asm volatile("" ::: "memory");
+    if (next) dv.issue(vbase, a.ldv, (kt + NW) * FS_KEYS, S, Vs, 0);
+  }
+
+  // merge: a wave's output (16 queries x 128 dims fp32, 16-byte pieces
+  // swizzled by the query) goes where its own K tile was, the second sixteen
+  // queries where its V tile was; then wave w takes queries 4 w .. 4 w + 3 of
+  // each sixteen, 16 lanes a query, dims 8 j .. 8 j + 7 in lane j
+#pragma unroll
+  for (int r = 0; r < RW; ++r) {
+    float* const xo = reinterpret_cast<float*>(r ? vbuf : kbuf) + (w * 16 + c) * HD;
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt)
+      *reinterpret_cast<floatx4*>(xo + (((4 * dt + g) ^ c) << 2)) = ot[r][dt];
+    const float lw = xg_sum(l[r]);
+    if (g == 0) ml[w][16 * r + c] = make_float2(m[r], lw);
+  }
+  __syncthreads();
+  const int j = c;
+#pragma unroll
+  for (int r = 0; r < RW; ++r) {
+    const float* const xo = reinterpret_cast<const float*>(r ? vbuf : kbuf);
+    const int qi = 4 * w + g, q = q0 + 16 * r + qi;
+    float M = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) M = fmaxf(M, ml[i][16 * r + qi].x);
+    const float mu = M == -INFINITY ? 0.f : M;
+    float L = 0.f, o[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = 0.f;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      const float2 p = ml[i][16 * r + qi];
+      const float f = __builtin_amdgcn_exp2f(p.x - mu);
+      const float* row = xo + (i * 16 + qi) * HD;
+      const floatx4 x0 = *reinterpret_cast<const floatx4*>(row + (((2 * j) ^ qi) << 2));
+      const floatx4 x1 = *reinterpret_cast<const floatx4*>(row + (((2 * j + 1) ^ qi) << 2));
+      L = fmaf(p.y, f, L);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o[e] = fmaf(x0[e], f, o[e]);
+        o[4 + e] = fmaf(x1[e], f, o[4 + e]);
+      }
+    }
+    const float inv = 1.0f / L;
+    half4v ov[2];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ov[e >> 2][e & 3] = (_Float16)(o[e] * inv);
+    const long long bhq = ((long long)b * a.nq + h) * S + q;
+    if (q < S) {
+      half4v* op = reinterpret_cast<half4v*>(a.o + (rowb + q) * a.ldo + h * HD + 8 * j);
+      op[0] = ov[0];
+      op[1] = ov[1];
+      if (j == 0) a.lse[bhq] = (M + __log2f(L)) * LN2;
+    }
+    if (a.dout) {  // the backward's dO operand, as in attn_fwd_kernel
+      const half4v* dr =
+          reinterpret_cast<const half4v*>(a.dout + (rowb + min(q, S - 1)) * a.lddo + h * HD + 8 * j);
+      const half4v dx[2] = {dr[0], dr[1]};
+      float dl = 0.f, am = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        dl += (float)dx[e >> 2][e & 3] * (float)ov[e >> 2][e & 3];
+        am = fmaxf(am, fabsf((float)dx[e >> 2][e & 3]));
+      }
+      dl = sum16_dpp(dl);
+      am = max16(am);
+      if (q < S) {
+        const float sc = pow2_scale_for(am, kDoScaleExp);
+        half4v* d16 = reinterpret_cast<half4v*>(a.dO16w + (rowb + q) * a.ld16 + h * HD + 8 * j);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          half4v x;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) x[v] = (_Float16)((float)dx[i][v] * sc);
+          d16[i] = x;
+        }
+        if (j == 0) {
+          a.deltaw[bhq] = dl;
+          a.dscw[bhq] = pow2_inv_scale_for(am, kDoScaleExp);
+        }
+      }
+    }
+  }
+}
+
 // Per token row, 16 lanes per head (lane j: dims 8 j .. 8 j + 7, 16-byte
 // accesses): delta[b, h, s] = sum_d dO * O, and dO16 = fp16(dO * sc) with sc
 // the power-of-two scale of the head's max |dO|, dsc[b, h, s] = 1 / sc (0 for
@@ -299,6 +497,14 @@ void launch_fwd(const AttnArgs& a, int B, hipStream_t st) {
                      0, st, a);
 }
 
+template <int RW>
+hipError_t launch_fwd_split(const AttnArgs& a, int B, hipStream_t st) {
+  hipLaunchKernelGGL(attn_fwd_split_kernel<RW>, dim3(a.nq, B, (a.S + 16 * RW - 1) / (16 * RW)),
+                     dim3(256), 0, st, a);
+  LLMT_LAUNCH_CHECK();
+  return hipSuccess;
+}
+
 }  // namespace
 
 hipError_t attn_delta(const void* dO, int dO_is_f16, long long ldd, const _Float16* o,
@@ -332,6 +538,21 @@ hipError_t attn_fwd(const AttnArgs& a, int B, hipStream_t st) {
     set_error("attn_fwd: the fused q norm needs qraw, the RoPE tables and q16w; the dO "
               "operand needs dO16w, deltaw and dscw");
     return hipErrorInvalidValue;
+  }
+  if (!getenv("LLMT_ATTN_CFG")) {
+    // Keys split over a workgroup's waves while every workgroup is resident
+    // at once (two a CU): 16-query blocks up to 512 of them; above, 32-query
+    // blocks (half the K and V traffic) where the chain of key tiles is long
+    // against the number of heads, that is B nq ceil(S / 32) <= 16384 / (B nq)
+    // and S >= 256.  us, attn_fwd_kernel -> split (nq 16): 16 queries B1 x S128
+    // 5.6 -> 4.6, B1 x S256 7.7 -> 5.7, B2 x S208 7.6 -> 6.4, B1 x S512 11.4 ->
+    // 8.6 (above: B3 x S208 8.1 against 9.5); 32 queries B2 x S512 12.8 -> 10.9,
+    // B1 x S1024 20.0 -> 14.6, B1 x S2048 37.2 -> 35.8 (beyond: B2 x S768 17.4
+    // against 18.7, B3 x S333 10.7 against 12.0; short: B3 x S208 8.1 against 8.5).
+    const long long heads = (long long)B * a.nq;
+    if (heads * ((a.S + 15) / 16) <= 512) return launch_fwd_split<1>(a, B, st);
+    if (a.S >= 256 && heads * heads * ((a.S + 31) / 32) <= 16384)
+      return launch_fwd_split<2>(a, B, st);
   }
   const AttnShape s = attn_shape(B, a.S, a.nq);
   switch (s.nw * 10 + s.rw) {

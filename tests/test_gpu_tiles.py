@@ -199,3 +199,28 @@ def test_attention_grid_sizes(dev, B, S, nq, nkv):
     got = llmt.attention_block_bwd(qd, kd, vd, one.to(dev), one.to(dev), do.half().to(dev))
     for a, b in zip(got, (dq_ref, dk_ref, dv_ref)):
         assert rel_l2(a.cpu(), b) < GRAD_TOL
+
+
+@pytest.mark.parametrize("B,S,nq,nkv", [(1, 1, 16, 8), (1, 17, 4, 1), (2, 31, 16, 8), (1, 129, 16, 8),
+                                        (1, 512, 16, 8), (1, 513, 16, 8), (2, 272, 16, 8),
+                                        (3, 257, 8, 8), (2, 530, 16, 8), (1, 1061, 16, 8)])
+def test_attention_forward_key_split(dev, B, S, nq, nkv):
+    """The attention forward on both sides of its rule: keys split over the
+    waves of 16- and of 32-query workgroups, then one sweep a wave; ragged S,
+    fewer key tiles than waves.  A NaN query row stays in its own row."""
+    print(f"case: attention forward B{B} S{S} nq{nq} nkv{nkv}", flush=True)
+    g = torch.Generator().manual_seed(5 * S + nq)
+    q = torch.randn(B, S, nq, 128, generator=g).half()
+    k = torch.randn(B, S, nkv, 128, generator=g).half()
+    v = torch.randn(B, S, nkv, 128, generator=g).half()
+    o_ref, lse_ref = ref.attention_fwd(q.float(), k.float(), v.float())
+    o, lse = llmt.attention_fwd(q.to(dev), k.to(dev), v.to(dev))
+    # fp16 probabilities and output: 2^-11 each, at most a few of them a row
+    assert rel_l2(o.float().cpu(), o_ref) < 2e-3
+    assert (lse.cpu() - lse_ref).abs().max() < 1e-3
+    r = S // 2
+    q[:, r, 0] = float("nan")
+    o2, lse2 = llmt.attention_fwd(q.to(dev), k.to(dev), v.to(dev))
+    assert torch.isnan(o2[:, r, 0]).all() and torch.isnan(lse2[:, 0, r]).all()
+    o2[:, r, 0], lse2[:, 0, r] = o[:, r, 0], lse[:, 0, r]
+    assert torch.equal(o2, o) and torch.equal(lse2, lse)
