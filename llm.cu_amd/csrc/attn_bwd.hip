@@ -28,9 +28,9 @@ namespace llmt {
 namespace {
 
 // ---------------------------------------------------------------- dQ
-// dS^T for one 64-key tile: dp (rows key, column query) = dP^T in, dS^T out.
-template <int RW, bool MASK>
-__device__ __forceinline__ void ds_tile_q(const floatx4 (&pt)[RW][4], floatx4 (&dp)[RW][4],
+// dS^T for one tile of 16 MT keys: dp (rows key, column query) = dP^T in, dS^T out.
+template <int RW, bool MASK, int MT>
+__device__ __forceinline__ void ds_tile_q(const floatx4 (&pt)[RW][MT], floatx4 (&dp)[RW][MT],
                                           const float (&lse2)[RW], const float (&del)[RW],
                                           float sl2, int key0, int q0, int S, int lane) {
   const int c = lane & 15, g = lane >> 4;
@@ -38,7 +38,7 @@ __device__ __forceinline__ void ds_tile_q(const floatx4 (&pt)[RW][4], floatx4 (&
   for (int r = 0; r < RW; ++r) {
     const int q = q0 + 16 * r + c;
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         float pv = __builtin_amdgcn_exp2f(fmaf(pt[r][mt][v], sl2, -lse2[r]));
@@ -48,6 +48,53 @@ __device__ __forceinline__ void ds_tile_q(const floatx4 (&pt)[RW][4], floatx4 (&
         }
         dp[r][mt][v] = pv * (dp[r][mt][v] - del[r]);
       }
+  }
+}
+
+// A wave's query rows q0 + 16 r + lane % 16 as dQ operands: Q and dO
+// fragments, the log2 LSE, delta in the row's dO scale, dQ's factor.
+template <int RW>
+__device__ __forceinline__ void load_dq_rows(const AttnArgs& a, long long rowb, int q0, int h,
+                                             int b, int lane, half8 (&qf)[RW][4],
+                                             half8 (&df)[RW][4], float (&lse2)[RW],
+                                             float (&del)[RW], float (&fq)[RW]) {
+  const int S = a.S, c = lane & 15;
+#pragma unroll
+  for (int r = 0; r < RW; ++r) {
+    const int q = q0 + 16 * r + c;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      qf[r][ks] = frag_global(a.q + rowb * a.ldq + h * HD, a.ldq, q, S, ks, lane);
+      df[r][ks] = frag_global(a.dO16 + rowb * a.ld16 + h * HD, a.ld16, q, S, ks, lane);
+    }
+    const bool ok = q < S;
+    lse2[r] = ok ? a.lse[((long long)b * a.nq + h) * S + q] * LOG2E : 0.f;
+    const float dsc = ok ? a.dsc[((long long)b * a.nq + h) * S + q] : 0.f;
+    del[r] = dsc > 0.f ? a.delta[((long long)b * a.nq + h) * S + q] / dsc : 0.f;
+    fq[r] = a.sm_scale * dsc;
+  }
+}
+
+// dQ row q of head h from its accumulators (factor f).
+__device__ __forceinline__ void store_dq(const AttnArgs& a, const floatx4 (&dqT)[8], float f,
+                                         long long rowb, int q, int h, int g) {
+  const int S = a.S;
+  float dy[8][4];
+#pragma unroll
+  for (int d = 0; d < 8; ++d)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) dy[d][v] = dqT[d][v] * f;
+  if (a.qn) {  // the block API: through q's RoPE and norm to d qraw
+    const int qc = min(q, S - 1);
+    norm_rope_bwd_row(dy, a.qraw + (rowb + qc) * a.ldqr + h * HD, a.qn, a.cosT, a.sinT, qc, a.eps,
+                      g);
+  }
+  if (q < S) {
+    float* dq = a.dq + (rowb + q) * a.ldgq + h * HD;
+#pragma unroll
+    for (int d = 0; d < 8; ++d)
+      *reinterpret_cast<float4*>(dq + d * 16 + 4 * g) =
+          make_float4(dy[d][0], dy[d][1], dy[d][2], dy[d][3]);
   }
 }
 
@@ -77,20 +124,7 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, _Float16* buf0, _Flo
   dv.issue(vbase, a.ldv, 0, S, buf0 + TILE, w);
   half8 qf[RW][4], df[RW][4];
   float lse2[RW], del[RW], fq[RW];
-#pragma unroll
-  for (int r = 0; r < RW; ++r) {
-    const int q = q0 + 16 * r + c;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      qf[r][ks] = frag_global(a.q + rowb * a.ldq + h * HD, a.ldq, q, S, ks, lane);
-      df[r][ks] = frag_global(a.dO16 + rowb * a.ld16 + h * HD, a.ld16, q, S, ks, lane);
-    }
-    const bool ok = q < S;
-    lse2[r] = ok ? a.lse[((long long)b * a.nq + h) * S + q] * LOG2E : 0.f;
-    const float dsc = ok ? a.dsc[((long long)b * a.nq + h) * S + q] : 0.f;
-    del[r] = dsc > 0.f ? a.delta[((long long)b * a.nq + h) * S + q] / dsc : 0.f;
-    fq[r] = a.sm_scale * dsc;
-  }
+  load_dq_rows<RW>(a, rowb, q0, h, b, lane, qf, df, lse2, del, fq);
   floatx4 dqT[RW][8];
 #pragma unroll
   for (int r = 0; r < RW; ++r)
@@ -134,7 +168,7 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, _Float16* buf0, _Flo
     }
     sched_reads_ahead<32, 32 * RW, 8, 2 * RW, 2, 0>();
     __builtin_amdgcn_sched_barrier(0);
-    ds_tile_q<RW, MASK>(pt, dp, lse2, del, sl2, kb * BLK, q0, S, lane);
+    ds_tile_q<RW, MASK, 4>(pt, dp, lse2, del, sl2, kb * BLK, q0, S, lane);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -162,27 +196,107 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, _Float16* buf0, _Flo
   for (int kb = nfull; kb < nkb; ++kb)
     tile_step(kb, std::true_type{}, (kb & 1) ? buf1 : buf0, (kb & 1) ? buf0 : buf1);
 #pragma unroll
-  for (int r = 0; r < RW; ++r) {
-    const int q = q0 + 16 * r + c;
-    const float f = fq[r];
-    float dy[8][4];
+  for (int r = 0; r < RW; ++r) store_dq(a, dqT[r], fq[r], rowb, q0 + 16 * r + c, h, g);
+}
+
+// Small grids: 16 RW queries a workgroup, the causal key range split over its
+// waves in 32-key tiles w, w + NW, .., each through an LDS buffer of its own
+// (no barriers in the loop); the dQ sums meet in LDS, wave r adding those of
+// the r-th sixteen queries in wave order.  dq_block's chain of up to S / 64
+// tiles a wave, each waiting for its own loads, is what a small grid waits
+// for (B1 x S512: attention backward 23.4 us, with these blocks 19.6).
+template <int NW, int RW>
+__device__ __forceinline__ void dq_block_split(const AttnArgs& a, _Float16* smem, int qb, int h,
+                                               int b) {
+  constexpr int KT = 32;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int S = a.S;
+  const int kvh = h / (a.nq / a.nkv);
+  const long long rowb = (long long)b * S;
+  const int q0 = qb * RW * 16;
+  const int nkt = (min(q0 + RW * 16, S) + KT - 1) / KT;
+  const float sl2 = a.sm_scale * LOG2E;
+  _Float16* const Ks = smem + w * (2 * KT * HD);
+  _Float16* const Vs = Ks + KT * HD;
+  TileDma<1, KT> dk, dv;
+  dk.init(a.ldk, 0);
+  dv.init(a.ldv, 0);
+  auto issue = [&](int kt) {
+    dk.issue(a.k + rowb * a.ldk + kvh * HD, a.ldk, kt * KT, S, Ks, 0);
+    dv.issue(a.v + rowb * a.ldv + kvh * HD, a.ldv, kt * KT, S, Vs, 0);
+  };
+  if (w < nkt) issue(w);
+  half8 qf[RW][4], df[RW][4];
+  float lse2[RW], del[RW], fq[RW];
+  load_dq_rows<RW>(a, rowb, q0, h, b, lane, qf, df, lse2, del, fq);
+  floatx4 dqT[RW][8];
 #pragma unroll
-    for (int d = 0; d < 8; ++d)
+  for (int r = 0; r < RW; ++r)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) dy[d][v] = dqT[r][d][v] * f;
-    if (a.qn) {  // the block API: through q's RoPE and norm to d qraw
-      const int qc = min(q, S - 1);
-      norm_rope_bwd_row(dy, a.qraw + (rowb + qc) * a.ldqr + h * HD, a.qn, a.cosT, a.sinT, qc,
-                        a.eps, g);
+    for (int i = 0; i < 8; ++i) dqT[r][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int kt = w; kt < nkt; kt += NW) {
+    wait_vm<0>();  // this wave's own tile (its buffer is private)
+    asm volatile("" ::: "memory");
+    floatx4 pt[RW][2], dp[RW][2];
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+#pragma unroll
+      for (int r = 0; r < RW; ++r) {
+        pt[r][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        dp[r][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const half8 kf = frag_rm(Ks, mt * 16, ks, lane);
+        const half8 vf = frag_rm(Vs, mt * 16, ks, lane);
+#pragma unroll
+        for (int r = 0; r < RW; ++r) {
+          pt[r][mt] = mfma16(kf, qf[r][ks], pt[r][mt]);
+          dp[r][mt] = mfma16(vf, df[r][ks], dp[r][mt]);
+        }
+      }
     }
-    if (q < S) {
-      float* dq = a.dq + (rowb + q) * a.ldgq + h * HD;
+    if (kt * KT + KT <= q0 + 1 && q0 + RW * 16 <= S)
+      ds_tile_q<RW, false, 2>(pt, dp, lse2, del, sl2, kt * KT, q0, S, lane);
+    else
+      ds_tile_q<RW, true, 2>(pt, dp, lse2, del, sl2, kt * KT, q0, S, lane);
+    half8 db[RW];
 #pragma unroll
-      for (int d = 0; d < 8; ++d)
-        *reinterpret_cast<float4*>(dq + d * 16 + 4 * g) =
-            make_float4(dy[d][0], dy[d][1], dy[d][2], dy[d][3]);
+    for (int r = 0; r < RW; ++r) db[r] = pair_frag(dp[r][0], dp[r][1]);
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      const half8 kc = frag_tr(Ks, d * 16, 0, lane);
+#pragma unroll
+      for (int r = 0; r < RW; ++r) dqT[r][d] = mfma16(kc, db[r], dqT[r][d]);
+    }
+    if (kt + NW < nkt) {  // refill the buffer once this tile's reads returned
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+      asm volatile("" ::: "memory");
+      issue(kt + NW);
     }
   }
+  // a wave's sums go where its own tile was ([r][register][lane] floatx4)
+  floatx4* const xch = reinterpret_cast<floatx4*>(smem);
+#pragma unroll
+  for (int r = 0; r < RW; ++r)
+    if (w != r) {
+#pragma unroll
+      for (int d = 0; d < 8; ++d) xch[((w * 2 + r) * 8 + d) * 64 + lane] = dqT[r][d];
+    }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < RW; ++r)
+    if (w == r) {
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww)
+        if (ww != r) {
+#pragma unroll
+          for (int d = 0; d < 8; ++d) dqT[r][d] += xch[((ww * 2 + r) * 8 + d) * 64 + lane];
+        }
+      store_dq(a, dqT[r], fq[r], rowb, q0 + 16 * r + c, h, g);
+    }
 }
 
 // dK and dV rows of one key (dkT / dvT in the group's dO scale gs): dK
@@ -534,16 +648,17 @@ __device__ __forceinline__ void dkdv_block_split(const AttnArgs& a, _Float16* sm
 // drained, leaving a tail at half occupancy for 45% of the dK/dV launch).
 // PART 0: both kinds; 1: dK/dV only; 2: dQ only -- the one-kind forms keep
 // their own (smaller) register and LDS budgets; 4: both, dK/dV blocks of 16
-// keys split over the waves in tiles of 32 queries.
+// keys split over the waves in tiles of 32 queries; 5: as 4, dQ
+// blocks split over the waves in tiles of 32 keys as well.
 constexpr int BWD_BUF = KV_BUF > 2 * TILE ? KV_BUF : 2 * TILE;  // halves per buffer
 
 template <int NW, int RW, int PART>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void attn_bwd_kernel(const AttnArgs a, int nkvb, int nqb) {
   // PART 0-2: the two tile buffers as separate arrays (statically named
-  // buffers, see dq_block); 4: one array split per wave.
+  // buffers, see dq_block); 4, 5: one array split per wave.
   constexpr int BUF = PART == 1 ? KV_BUF : PART == 2 ? 2 * TILE : BWD_BUF;
-  constexpr bool SPLIT = PART == 4;
+  constexpr bool SPLIT = PART == 4 || PART == 5;
   constexpr int QT = 32;
   constexpr int SMEM4 = NW * split_buf(QT) > 4 * TILE ? NW * split_buf(QT) : 4 * TILE;
   __shared__ __attribute__((aligned(1024))) _Float16 buf0[SPLIT ? SMEM4 : BUF];
@@ -562,7 +677,9 @@ void attn_bwd_kernel(const AttnArgs a, int nkvb, int nqb) {
   }
   if constexpr (PART != 1) {
     const int y = x - nkvx;
-    if constexpr (SPLIT)
+    if constexpr (PART == 5)
+      dq_block_split<NW, RW>(a, buf0, nqb - 1 - y / a.nq, y % a.nq, b);
+    else if constexpr (SPLIT)
       dq_block<NW, RW>(a, buf0, buf0 + 2 * TILE, nqb - 1 - y / a.nq, y % a.nq, b);
     else
       dq_block<NW, RW>(a, buf0, buf1, nqb - 1 - y / a.nq, y % a.nq, b);
@@ -646,10 +763,21 @@ hipError_t attn_bwd(const AttnArgs& a, int B, hipStream_t st) {
       // whose four waves split the group's 32-query tiles, beside 64-query dQ
       // blocks (two workgroups a CU), while both kinds are at most 800
       // workgroups.  Against 32-key blocks of two waves, us: B1 x S128 11.7
-      // -> 8.2, B1 x S256 18.3 -> 12.1, B3 x S208 20.8 -> 13.5, B1 x S512 31.9
-      // -> 22.9, B1 x S1024 75.5 -> 45.4; beyond (B8 x S256) 24.7 against 33.2.
+      // -> 8.2, B1 x S256 18.3 -> 12.1, B3 x S208 20.8 -> 13.5, B2 x S400 20.7;
+      // beyond (B8 x S256) 24.7 against 33.2.
       const long long n = (long long)B * (a.nkv * (long long)((a.S + 15) / 16) +
                                           a.nq * (long long)((a.S + 63) / 64));
+      // With few heads the dQ blocks are the longest chains once dK/dV blocks
+      // take most CUs: they then split their keys too (up to 16 heads, 320 to
+      // 1536 workgroups by the count above).  us: B1 x S432 17.6 -> 17.5, B1 x
+      // S512 23.4 -> 19.6, B1 x S1024 46.0 -> 36.8, B1 x S1100 65.9 -> 43.7, B1
+      // x S2048 117 -> 107 (outside: B1 x S320 14.2 against 14.4, B1 x S3000
+      // 179 against 208, B2 x S400 20.7 against 23.6, B3 x S208 14.0 against 18.3).
+      if (n > 320 && n <= 1536 && (long long)B * a.nq <= 16) {
+        launch_bwd<4, 2, 5>(a, B, (a.S + 15) / 16, (a.S + 31) / 32, st);
+        LLMT_LAUNCH_CHECK();
+        return hipSuccess;
+      }
       if (n <= 800) {
         launch_bwd<4, 1, 4>(a, B, (a.S + 15) / 16, (a.S + 63) / 64, st);
         LLMT_LAUNCH_CHECK();

@@ -224,3 +224,11 @@ def test_attention_forward_key_split(dev, B, S, nq, nkv):
     assert torch.isnan(o2[:, r, 0]).all() and torch.isnan(lse2[:, 0, r]).all()
     o2[:, r, 0], lse2[:, 0, r] = o[:, r, 0], lse[:, 0, r]
     assert torch.equal(o2, o) and torch.equal(lse2, lse)
+
+
+@pytest.mark.parametrize("B,S,nq,nkv", [(1, 431, 16, 8), (1, 450, 16, 8), (2, 799, 8, 4),
+                                        (1, 1063, 8, 1), (4, 1030, 4, 4)])
+def test_attention_backward_key_split(dev, B, S, nq, nkv):
+    """The dQ blocks whose keys are split over the waves (few heads, grids of
+    320 to 1536 workgroups), both edges of that rule, ragged last blocks."""
+    test_attention_grid_sizes(dev, B, S, nq, nkv)
