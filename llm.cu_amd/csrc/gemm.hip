@@ -1,4 +1,4 @@
-// gemm.hip — skinny "NT" GEMM on fp16 MFMA (v_mfma_f32_16x16x32_f16) for
+// gemm.hip — "NT" GEMMs on fp16 MFMA (v_mfma_f32_16x16x32_f16) for
 // gfx950, plus the layout kernels (fragment packing, transposes,
 // conversions, the bit-exact int8 quantizer) and the split-K reduction used
 // by the standalone GEMM entry points.
