@@ -941,33 +941,73 @@ __global__ __launch_bounds__(RT) void norm_bwd_kernel(const NormBwdArgs a) {
 // (LORA: the attention norm's q, k, v terms, each over all H columns, whose
 // 48 x 4 values a thread loads once for all its rows).
 // The attention norm's LoRA dx term s (dh_q A_q + dh_k A_k + dh_v A_v) of
-// NR rows on MFMA (16 x 16 x 16 fp16: rows x ranks of one adapter times
-// ranks x 16 columns): wave w takes columns 256 w .. of the row, A operand
-// = the rows' dh values (rows past NR zero), scaled by 2^-10 into fp16 range
-// (dh is in the GEMM's scaled units) and split into two fp16 parts, the value
-// and what its rounding left times 2^11 (22 bits of the fp32 dh, summed
-// apart in fp32), B operand = 4 consecutive ranks of one column from the
-// transposed copy at [H][48].  The 16 x 16 results go through LDS
-// (out[NR][H], H <= 4 RT) to the thread that owns the column.
-constexpr float kLoraMfmaScale = 1.0f / 1024.0f;
-constexpr float kLoraLowScale = 2048.0f;
+// NR rows on MFMA (16 x 16 x 16 fp16: four rows' dh parts x ranks of one
+// adapter, times ranks x 16 columns): wave w takes columns 256 w .. of the row,
+// B operand = 4 consecutive ranks of one column from the transposed copy at
+// [H][48].  dh keeps its fp32 value: each row is scaled by a power of two to
+// [2^14, 2^15) and split into three fp16 parts (the value, then what is left
+// times 2^11, twice), which hold all 24 bits of every element down to 2^-38
+// of the row's largest; the parts of a row are operand rows 4 i .. 4 i + 2 (a
+// fourth is zero), so one product of 16 operand rows does all three and the
+// lane that owns a row and column gets them as one register quad.  The results
+// go through LDS (row i at out + i kLoraLd, the pad keeping the four rows of a
+// store in different banks) to the thread that owns the column.  The kernel
+// alone, H = 2048, us at 512 / 2000 / 4096 rows: 9.5 / 21.7 / 41.3 (one row a
+// workgroup on VALU 12.9 / 49.0 / 94.2; fp32 products 16 x 16 x 4, a quarter of
+// the rate, 14.9 / 32.0 / 60.1; two fp16 parts under a fixed scale, one product
+// each, 9.0 / 22.8 / 40.0, but dh below 2^-4 lost bits, 1.4e-4 at 1e-4, and
+// above 2^26 overflowed).
+constexpr float kLoraPart = 2048.0f;  // 2^11: one fp16 part
+constexpr int kLoraLd = 4 * RT + 16;
 
+// B operands of the 64 columns from 256 wave + 64 cg.
+__device__ __forceinline__ void lora_mfma_load(const NormBwdArgs& a, int cg, half4 (&b)[3][4]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb) {
+    const int col = min(256 * wave + 64 * cg + 16 * nb + (lane & 15), a.H - 1);
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      b[q][nb] = *reinterpret_cast<const half4*>(a.lora_at + (long long)col * (3 * R) + q * R +
+                                                 4 * (lane >> 4));
+  }
+}
+
+// b: the first 64 columns' operands, loaded by the caller before hs was ready.
 template <int NR>
 __device__ __forceinline__ void lora_rows_mfma(const NormBwdArgs& a, const float (*hs)[64],
-                                               float* out) {
+                                               half4 (&b)[3][4], float* out) {
+  constexpr int NG = (NR + 3) / 4;  // groups of four rows
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int kq = lane >> 4, n = lane & 15;
-  half4 aop[3], alo[3];
+  const int kq = lane >> 4, n = lane & 15, part = n & 3;
+  half4 aop[NG][3];
+  int ex[NG];  // row 4 i + kq, which this lane stores, is scaled by 2^ex
 #pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    const float4 h4 = n < NR ? *reinterpret_cast<const float4*>(&hs[n][a.in.term[q].hidx + 4 * kq])
-                             : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float x[4] = {h4.x * kLoraMfmaScale, h4.y * kLoraMfmaScale, h4.z * kLoraMfmaScale,
-                        h4.w * kLoraMfmaScale};
+  for (int i = 0; i < NG; ++i) {
+    const int row = 4 * i + (n >> 2);
+    float4 h[3];
+    float amax = 0.f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      aop[q][e] = (_Float16)x[e];
-      alo[q][e] = (_Float16)((x[e] - (float)aop[q][e]) * kLoraLowScale);
+    for (int q = 0; q < 3; ++q) {
+      h[q] = row < NR ? *reinterpret_cast<const float4*>(&hs[row][a.in.term[q].hidx + 4 * kq])
+                      : make_float4(0.f, 0.f, 0.f, 0.f);
+      amax = fmaxf(amax, amax4(h[q]));
+    }
+    amax = fmaxf(amax, __shfl_xor(amax, 16));
+    amax = fmaxf(amax, __shfl_xor(amax, 32));
+    const int k = 15 - __builtin_amdgcn_frexp_expf(amax);
+    ex[i] = __shfl(k, 4 * kq);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const float x[4] = {ldexpf(h[q].x, k), ldexpf(h[q].y, k), ldexpf(h[q].z, k), ldexpf(h[q].w, k)};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const _Float16 p0 = (_Float16)x[e];
+        const float r1 = (x[e] - (float)p0) * kLoraPart;
+        const _Float16 p1 = (_Float16)r1;
+        const _Float16 p2 = (_Float16)((r1 - (float)p1) * kLoraPart);
+        aop[i][q][e] = part == 0 ? p0 : part == 1 ? p1 : part == 2 ? p2 : (_Float16)0.f;
+      }
     }
   }
   const int H = a.H;
@@ -975,42 +1015,32 @@ __device__ __forceinline__ void lora_rows_mfma(const NormBwdArgs& a, const float
   for (int cg = 0; cg < 4; ++cg) {
     const int cb = 256 * wave + 64 * cg;
     if (cb >= H) break;  // wave-uniform
-    half4 b[3][4];
+    if (cg > 0) lora_mfma_load(a, cg, b);
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      const int col = min(cb + 16 * nb + n, H - 1);
+    for (int i = 0; i < NG; ++i) {
+      floatx4 acc[4];
 #pragma unroll
-      for (int q = 0; q < 3; ++q)
-        b[q][nb] = *reinterpret_cast<const half4*>(a.lora_at + (long long)col * (3 * R) + q * R + 4 * kq);
-    }
-    floatx4 acc[4];
+      for (int nb = 0; nb < 4; ++nb) {
+        acc[nb] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      acc[nb] = floatx4{0.f, 0.f, 0.f, 0.f};
-      floatx4 low = acc[nb];
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        acc[nb] = __builtin_amdgcn_mfma_f32_16x16x16f16(aop[q], b[q][nb], acc[nb], 0, 0, 0);
-        low = __builtin_amdgcn_mfma_f32_16x16x16f16(alo[q], b[q][nb], low, 0, 0, 0);
+        for (int q = 0; q < 3; ++q)
+          acc[nb] = __builtin_amdgcn_mfma_f32_16x16x16f16(aop[i][q], b[q][nb], acc[nb], 0, 0, 0);
       }
-      acc[nb] += low * (1.0f / kLoraLowScale);
-    }
-    // lane: rows 4 kq + i of column cb + 16 nb + n
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 4 * kq + i;
-      if (row >= NR) continue;
+      // lane: the parts of row 4 i + kq, column cb + 16 nb + n
+      if (4 * i + kq >= NR) continue;
 #pragma unroll
       for (int nb = 0; nb < 4; ++nb) {
         const int col = cb + 16 * nb + n;
-        if (col < H) out[row * H + col] = acc[nb][i];
+        if (col < H)
+          out[(4 * i + kq) * kLoraLd + col] = ldexpf(
+              acc[nb][0] + (acc[nb][1] + acc[nb][2] * (1.0f / kLoraPart)) * (1.0f / kLoraPart), -ex[i]);
       }
     }
   }
 }
 
 // LM: 0 no adapter terms, 1 the q/k/v terms on VALU, 2 on MFMA
-// (lora_rows_mfma: at 4096 rows 52.6 -> 45 us a layer).
+// (lora_rows_mfma).
 template <int NR, int LM, bool NT = false>
 __global__ __launch_bounds__(RT) void norm_bwd_rows_kernel(const NormBwdArgs a, int T) {
   constexpr bool LORA = LM > 0;
@@ -1032,6 +1062,8 @@ __global__ __launch_bounds__(RT) void norm_bwd_rows_kernel(const NormBwdArgs a, 
   }
   float4 v[NR], hv[NR];
   load_rows<NR, true>(a.in, t0, T, H, v, hv);
+  half4 lb[3][4];
+  if constexpr (LM == 2) lora_mfma_load(a, 0, lb);
   const float4 ww = ld4(a.w + cc);
   const float4 ks4 = a.g16_ks ? ldh4(a.g16_ks + cc) : make_float4(1.f, 1.f, 1.f, 1.f);
 #pragma unroll
@@ -1042,14 +1074,13 @@ __global__ __launch_bounds__(RT) void norm_bwd_rows_kernel(const NormBwdArgs a, 
           mul4(hv[i], rs[i]);
   }
   if constexpr (LM == 2) {
-    __shared__ __attribute__((aligned(16))) float lora_out[NR * 4 * RT];  // [NR][H]
+    __shared__ __attribute__((aligned(16))) float lora_out[NR * kLoraLd];
     __syncthreads();
-    lora_rows_mfma<NR>(a, hs, lora_out);
+    lora_rows_mfma<NR>(a, hs, lb, lora_out);
     __syncthreads();
-    const float ls = a.in.lscale / kLoraMfmaScale;
 #pragma unroll
     for (int i = 0; i < NR; ++i)
-      v[i] = add4(v[i], mul4(*reinterpret_cast<const float4*>(&lora_out[i * H + cc]), ls));
+      v[i] = add4(v[i], mul4(*reinterpret_cast<const float4*>(&lora_out[i * kLoraLd + cc]), a.in.lscale));
   } else if constexpr (LM == 1) {
     LoraRegs<1, 3> L;
     lora_load<1, 3>(a.in, H, L);
@@ -1819,8 +1850,8 @@ hipError_t norm_bwd(const NormBwdArgs& a, int T, hipStream_t st) {
     if (!ok) am.lora_at = nullptr;
   }
   // many rows: the VALU LoRA form shares its adapter values over 8 rows; the
-  // MFMA form runs 4 (128 VGPRs, two workgroups a CU: at 4096 rows 45 us
-  // against 46 at 8 rows and 54 at 2)
+  // MFMA form runs 4, one product's worth (the kernel alone at 4096 rows 41.3
+  // us, 54.5 at 2 rows, 48.4 at 3, 43.5 at 8)
   const int nr = rows_per_wg(T, P, lora ? (am.lora_at ? 4 : 8) : 2);
   const dim3 g((T + nr - 1) / nr);
   // the stashed x and the incoming residual gradient are read once: past

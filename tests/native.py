@@ -1,0 +1,41 @@
+"""ctypes mirrors of the library's internal launch arguments (csrc/ops.h) and
+its exported C++ entry points, for tests of one kernel or of a host-side rule
+that no C entry point reaches alone."""
+import ctypes as C
+
+vp, i32, i64, f32 = C.c_void_p, C.c_int, C.c_longlong, C.c_float
+
+
+def _struct(name, fields):
+    return type(name, (C.Structure,), {"_fields_": fields})
+
+
+BSeg = _struct("BSeg", [("ptr", vp), ("colscale", vp), ("kscale", vp), ("rows", i32), ("ld", i32),
+                        ("is_i8", i32)])
+GemmArgs = _struct("GemmArgs", [
+    ("A", vp), ("lda", i32), ("seg", BSeg * 4), ("seg_start", i32 * 5), ("nseg", i32), ("C", vp),
+    ("ldc", i32), ("split_stride", i64), ("M", i32), ("N", i32), ("K", i32), ("split", i32),
+    ("split_col", i32), ("glu", i32), ("glu16", vp), ("ldglu", i32), ("gu16", vp),
+    ("rowstats", vp)])
+LoraTerm = _struct("LoraTerm", [("shr", vp), ("row0", i32), ("kp", i32), ("c0", i32), ("n", i32),
+                                ("hidx", i32)])
+RowIn = _struct("RowIn", [
+    ("part", vp), ("split", i32), ("ss", i64), ("ldp", i32), ("split_col", i32), ("hcol", i32),
+    ("nh", i32), ("nterm", i32), ("term", LoraTerm * 3), ("lscale", f32)])
+NormBwdArgs = _struct("NormBwdArgs", [
+    ("inp", RowIn), ("rinv_in", vp), ("gscale", f32), ("dh_out", vp), ("dh_col", i32), ("x", vp),
+    ("w", vp), ("eps", f32), ("H", i32), ("dres_in", vp), ("dres_out", vp), ("dmid_out", vp),
+    ("g16", vp), ("rinv_out", vp), ("g16_ks", vp), ("lora_at", vp)])
+
+
+def fn(L, symbol, restype, *argtypes):
+    f = getattr(L, symbol)
+    f.restype, f.argtypes = restype, list(argtypes)
+    return f
+
+
+def norm_bwd(L, args, T, stream=None):
+    """hipError_t of llmt::norm_bwd(const NormBwdArgs&, int, hipStream_t)."""
+    f = fn(L, "_ZN4llmt8norm_bwdERKNS_11NormBwdArgsEiP12ihipStream_t", i32,
+           C.POINTER(NormBwdArgs), i32, vp)
+    return f(C.byref(args), T, stream)

@@ -111,7 +111,7 @@ def test_head_row_tiles(dev, T):
 def test_layer_row_epilogues_at_row_counts(dev, T):
     """One small layer at token counts on both sides of the row epilogues'
     rows-a-workgroup steps (256, 512, 768 rows), adapters large enough for
-    their input-gradient term (split into two fp16 parts on the matrix cores
+    their input-gradient term (three fp16 parts of dh on the matrix cores
     above 256 rows) to dominate dx."""
     print(f"case: row epilogues T{T}", flush=True)
     d = ref.Dims(**{**ref.QWEN3_1_7B.__dict__, "n_layers": 1, "vocab": 256, "hidden": 512,
