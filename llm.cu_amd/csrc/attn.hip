@@ -528,6 +528,31 @@ hipError_t attn_delta(const void* dO, int dO_is_f16, long long ldd, const _Float
   return hipSuccess;
 }
 
+// Keys split over a workgroup's waves: 16-query blocks while every workgroup
+// is resident at once (two a CU, 512); above, 32-query blocks (half the K and V
+// traffic) where the chain of key tiles is long against the number of heads,
+// that is B nq ceil(S / 32) <= 16384 / (B nq) and S >= 256, up to 1280
+// workgroups: beyond that the chip is full and attn_fwd_kernel's larger blocks
+// read less.  us, attn_fwd_kernel -> split:
+//   16 queries, nq 16  B1 x S128 5.6 -> 4.6, B1 x S256 7.7 -> 5.7, B2 x S208 7.6
+//                      -> 6.4, B1 x S512 11.4 -> 8.6 (above: B3 x S208 8.1
+//                      against 9.5)
+//   32 queries, B nq   2: S8192 119 -> 68, S16384 (1024 workgroups) 255 -> 200
+//                      4: S4096 62 -> 37, S8192 (1024) 130 -> 105
+//                         (S12288, 1536: 213 against 215)
+//                      8: S4096 (1024) 68 -> 57, S5120 (1280) 88 -> 82
+//                         (S6144, 1536: 109 against 113)
+//                      16: S1024 20.0 -> 14.6, S2048 (1024) 37.2 -> 35.8
+//                         (S2560, 1280: 46.7 against 48.4)
+//                      32: S512 12.8 -> 10.9 (S768 16.9 against 18.1)
+// (short: B3 x S208 8.1 against 8.5).  Returns the 16-query tiles a workgroup,
+// 0 for attn_fwd_kernel.
+int attn_fwd_split_tiles(int B, int S, int nq) {
+  const long long heads = (long long)B * nq, b32 = heads * ((S + 31) / 32);
+  if (heads * ((S + 15) / 16) <= 512) return 1;
+  return S >= 256 && b32 <= 1280 && heads * b32 <= 16384 ? 2 : 0;
+}
+
 hipError_t attn_fwd(const AttnArgs& a, int B, hipStream_t st) {
   if (a.nq % a.nkv || a.S <= 0) {
     set_error("attn_fwd: nq=%d nkv=%d S=%d", a.nq, a.nkv, a.S);
@@ -540,19 +565,9 @@ hipError_t attn_fwd(const AttnArgs& a, int B, hipStream_t st) {
     return hipErrorInvalidValue;
   }
   if (!getenv("LLMT_ATTN_CFG")) {
-    // Keys split over a workgroup's waves while every workgroup is resident
-    // at once (two a CU): 16-query blocks up to 512 of them; above, 32-query
-    // blocks (half the K and V traffic) where the chain of key tiles is long
-    // against the number of heads, that is B nq ceil(S / 32) <= 16384 / (B nq)
-    // and S >= 256.  us, attn_fwd_kernel -> split (nq 16): 16 queries B1 x S128
-    // 5.6 -> 4.6, B1 x S256 7.7 -> 5.7, B2 x S208 7.6 -> 6.4, B1 x S512 11.4 ->
-    // 8.6 (above: B3 x S208 8.1 against 9.5); 32 queries B2 x S512 12.8 -> 10.9,
-    // B1 x S1024 20.0 -> 14.6, B1 x S2048 37.2 -> 35.8 (beyond: B2 x S768 17.4
-    // against 18.7, B3 x S333 10.7 against 12.0; short: B3 x S208 8.1 against 8.5).
-    const long long heads = (long long)B * a.nq;
-    if (heads * ((a.S + 15) / 16) <= 512) return launch_fwd_split<1>(a, B, st);
-    if (a.S >= 256 && heads * heads * ((a.S + 31) / 32) <= 16384)
-      return launch_fwd_split<2>(a, B, st);
+    const int rw = attn_fwd_split_tiles(B, a.S, a.nq);
+    if (rw == 1) return launch_fwd_split<1>(a, B, st);
+    if (rw == 2) return launch_fwd_split<2>(a, B, st);
   }
   const AttnShape s = attn_shape(B, a.S, a.nq);
   switch (s.nw * 10 + s.rw) {

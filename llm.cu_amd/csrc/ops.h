@@ -306,6 +306,9 @@ struct AttnArgs {
   float* deltaw;
   float* dscw;
 };
+// 16-query tiles a workgroup (1 or 2) where the forward splits a workgroup's
+// keys over its waves, 0 where each wave walks all of them.
+int attn_fwd_split_tiles(int B, int S, int nq);
 hipError_t attn_fwd(const AttnArgs& a, int B, hipStream_t st);
 hipError_t attn_bwd(const AttnArgs& a, int B, hipStream_t st);
 // Operands of a standalone attention backward from dO [T, ldd] (fp32, or

@@ -203,7 +203,8 @@ def test_attention_grid_sizes(dev, B, S, nq, nkv):
 
 @pytest.mark.parametrize("B,S,nq,nkv", [(1, 1, 16, 8), (1, 17, 4, 1), (2, 31, 16, 8), (1, 129, 16, 8),
                                         (1, 512, 16, 8), (1, 513, 16, 8), (2, 272, 16, 8),
-                                        (3, 257, 8, 8), (2, 530, 16, 8), (1, 1061, 16, 8)])
+                                        (3, 257, 8, 8), (2, 530, 16, 8), (1, 1061, 16, 8),
+                                        (1, 2061, 4, 2), (1, 2061, 24, 3)])
 def test_attention_forward_key_split(dev, B, S, nq, nkv):
     """The attention forward on both sides of its rule: keys split over the
     waves of 16- and of 32-query workgroups, then one sweep a wave; ragged S,
