@@ -736,6 +736,31 @@ void launch_attn_bwd(const AttnArgs& a, int B, int nwk, int nwq, int rw, hipStre
 
 }  // namespace
 
+// Small grids are serial chains on few CUs: dK/dV blocks of 16 keys whose four
+// waves split the group's 32-query tiles, beside 64-query dQ blocks (two
+// workgroups a CU), while both kinds are at most 800 workgroups (1).  Against
+// 32-key blocks of two waves, us: B1 x S128 11.7 -> 8.2, B1 x S256 18.3 -> 12.1,
+// B3 x S208 20.8 -> 13.5, B2 x S400 20.7; beyond (B8 x S256) 24.7 against 33.2.
+//
+// With few heads the dQ blocks are the longest chains once dK/dV blocks take
+// most CUs: they then split their keys too (2), up to 16 heads, 320 to 1536
+// workgroups by the count above.  us: B1 x S432 17.6 -> 17.5, B1 x S512 23.4 ->
+// 19.6, B1 x S1024 46.0 -> 36.8, B1 x S1100 65.9 -> 43.7, B1 x S2048 117 -> 107
+// (outside: B1 x S320 14.2 against 14.4, B1 x S3000 179 against 208, B2 x S400
+// 20.7 against 23.6, B3 x S208 14.0 against 18.3).  Up to two query heads a KV
+// head the dK/dV chain is the shorter one at any workgroup count (S / 128 tiles
+// of 32 queries a head against S / 64 of 64 keys), so from S = 768 they do so
+// below 320 as well; the operator, us, (1) -> (2) at nq / nkv: 1 / 1 S1024 37 ->
+// 28, S4096 130 -> 58 (114 in general form); 2 / 1 S2048 67 -> 50; 4 / 2 S1024
+// 38 -> 33; 4 / 4 S1024 42 -> 28; 8 / 4 S768 33 -> 31.  With more query heads
+// the form above stays: 6 / 2 S1024 42 against 46, 4 / 1 S2048 93 against 96.
+int attn_bwd_split(int B, int S, int nq, int nkv) {
+  const long long n =
+      (long long)B * (nkv * (long long)((S + 15) / 16) + nq * (long long)((S + 63) / 64));
+  if ((n > 320 || (S >= 768 && nq <= 2 * nkv)) && n <= 1536 && (long long)B * nq <= 16) return 2;
+  return n <= 800 ? 1 : 0;
+}
+
 hipError_t attn_bwd(const AttnArgs& a, int B, hipStream_t st) {
   if (a.nq % a.nkv || a.S <= 0 || !a.dO16 || !a.dsc || !a.dk || !a.dv) {
     set_error("attn_bwd: nq=%d nkv=%d S=%d (fp16 dO, its scales and dK/dV outputs required)",
@@ -759,27 +784,10 @@ hipError_t attn_bwd(const AttnArgs& a, int B, hipStream_t st) {
   int nwk = dkdv_waves(B, a.S, a.nkv);
   if (!getenv("LLMT_ATTN_CFG")) {
     if (!getenv("LLMT_ATTN_DKDV_WAVES")) {
-      // Small grids are serial chains on few CUs: dK/dV blocks of 16 keys
-      // whose four waves split the group's 32-query tiles, beside 64-query dQ
-      // blocks (two workgroups a CU), while both kinds are at most 800
-      // workgroups.  Against 32-key blocks of two waves, us: B1 x S128 11.7
-      // -> 8.2, B1 x S256 18.3 -> 12.1, B3 x S208 20.8 -> 13.5, B2 x S400 20.7;
-      // beyond (B8 x S256) 24.7 against 33.2.
-      const long long n = (long long)B * (a.nkv * (long long)((a.S + 15) / 16) +
-                                          a.nq * (long long)((a.S + 63) / 64));
-      // With few heads the dQ blocks are the longest chains once dK/dV blocks
-      // take most CUs: they then split their keys too (up to 16 heads, 320 to
-      // 1536 workgroups by the count above).  us: B1 x S432 17.6 -> 17.5, B1 x
-      // S512 23.4 -> 19.6, B1 x S1024 46.0 -> 36.8, B1 x S1100 65.9 -> 43.7, B1
-      // x S2048 117 -> 107 (outside: B1 x S320 14.2 against 14.4, B1 x S3000
-      // 179 against 208, B2 x S400 20.7 against 23.6, B3 x S208 14.0 against 18.3).
-      if (n > 320 && n <= 1536 && (long long)B * a.nq <= 16) {
-        launch_bwd<4, 2, 5>(a, B, (a.S + 15) / 16, (a.S + 31) / 32, st);
-        LLMT_LAUNCH_CHECK();
-        return hipSuccess;
-      }
-      if (n <= 800) {
-        launch_bwd<4, 1, 4>(a, B, (a.S + 15) / 16, (a.S + 63) / 64, st);
+      const int sp = attn_bwd_split(B, a.S, a.nq, a.nkv);
+      if (sp == 2) launch_bwd<4, 2, 5>(a, B, (a.S + 15) / 16, (a.S + 31) / 32, st);
+      if (sp == 1) launch_bwd<4, 1, 4>(a, B, (a.S + 15) / 16, (a.S + 63) / 64, st);
+      if (sp) {
         LLMT_LAUNCH_CHECK();
         return hipSuccess;
       }

@@ -310,6 +310,9 @@ struct AttnArgs {
 // keys over its waves, 0 where each wave walks all of them.
 int attn_fwd_split_tiles(int B, int S, int nq);
 hipError_t attn_fwd(const AttnArgs& a, int B, hipStream_t st);
+// 0, or the split forms of the backward's blocks: 1 dK/dV over a workgroup's
+// waves, 2 dK/dV and dQ.
+int attn_bwd_split(int B, int S, int nq, int nkv);
 hipError_t attn_bwd(const AttnArgs& a, int B, hipStream_t st);
 // Operands of a standalone attention backward from dO [T, ldd] (fp32, or
 // fp16 with dO_is_f16) and O fp16 [T, ldo]: delta[b, h, s] = sum_d dO * O,

@@ -228,8 +228,12 @@ def test_attention_forward_key_split(dev, B, S, nq, nkv):
 
 
 @pytest.mark.parametrize("B,S,nq,nkv", [(1, 431, 16, 8), (1, 450, 16, 8), (2, 799, 8, 4),
-                                        (1, 1063, 8, 1), (4, 1030, 4, 4)])
+                                        (1, 1063, 8, 1), (4, 1030, 4, 4), (1, 770, 1, 1),
+                                        (1, 2033, 2, 1), (1, 767, 4, 4), (4, 1217, 4, 4)])
 def test_attention_backward_key_split(dev, B, S, nq, nkv):
-    """The dQ blocks whose keys are split over the waves (few heads, grids of
-    320 to 1536 workgroups), both edges of that rule, ragged last blocks."""
+    """The dQ blocks whose keys are split over the waves (few heads), ragged
+    last blocks: 328 to 1312 workgroups by the rule's count; below 320 from S =
+    768 with at most two query heads a KV head (62 and 192).  Beside them what
+    the rule leaves to the other forms: 203 workgroups at 8 / 1, S = 767, and
+    1552 workgroups."""
     test_attention_grid_sizes(dev, B, S, nq, nkv)

@@ -23,3 +23,15 @@ def test_attention_forward_split_is_bounded_by_its_workgroups():
     assert [f(1, s, 8) for s in (4096, 5120, 5121, 8192)] == [2, 2, 0, 0]
     assert [f(1, s, 16) for s in (512, 513, 2048, 2049)] == [1, 2, 2, 0]
     assert [f(2, s, 16) for s in (256, 257, 512, 513)] == [1, 2, 2, 0]
+
+
+def test_attention_backward_split_lines():
+    """dQ blocks split their keys with up to 16 heads and 1536 workgroups: past
+    320 of them, and from S = 768 at any count with at most two query heads a
+    KV head (one head at S = 4096 counts exactly 320); dK/dV blocks alone up
+    to 800."""
+    f = native.fn(llmt.lib(), "_ZN4llmt14attn_bwd_splitEiiii", native.i32, *[native.i32] * 4)
+    assert [f(1, s, 1, 1) for s in (767, 768, 4095, 4096, 4097, 19648, 19649)] == [1, 2, 2, 2, 2, 2, 0]
+    assert [f(1, s, 6, 2) for s in (768, 1456, 1457, 7008, 7009)] == [1, 1, 2, 2, 0]
+    assert [f(1, s, 16, 8) for s in (16, 416, 417, 2048, 2049)] == [1, 1, 2, 2, 0]
+    assert [f(1, s, 32, 8) for s in (128, 768, 769)] == [1, 1, 0]
