@@ -1607,7 +1607,6 @@ static hipError_t launch_big(const GemmArgs& g, hipStream_t st) {
   using BF = std::integral_constant<bool, false>;
   if (gm.glu) {
     if (!i8) go(BF(), BF(), BT(), BF());
-    else if (ks) go(BT(), BT(), BT(), BF());
     else go(BT(), BF(), BT(), BF());
   } else if (fold) {
     if (!i8) go(BF(), BF(), BF(), BT());
@@ -1634,11 +1633,21 @@ hipError_t gemm_nt(const GemmArgs& g, hipStream_t st) {
     set_error("gemm_nt: unsupported shape M=%d N=%d K=%d split=%d", g.M, g.N, g.K, g.split);
     return hipErrorInvalidValue;
   }
-  for (int i = 0; i < g.nseg; ++i)
+  for (int i = 0; i < g.nseg; ++i) {
     if (g.seg[i].rows % 16) {
       set_error("gemm_nt: segment rows must be a multiple of 16 (%d)", g.seg[i].rows);
       return hipErrorInvalidValue;
     }
+    // scales that the kernels do not apply
+    if (g.seg[i].kscale && (g.glu || !g.seg[i].is_i8)) {
+      set_error("gemm_nt: a per-k scale needs an int8 segment and no SwiGLU epilogue");
+      return hipErrorInvalidValue;
+    }
+    if (g.seg[i].colscale && !g.seg[i].is_i8) {
+      set_error("gemm_nt: a column scale needs an int8 segment");
+      return hipErrorInvalidValue;
+    }
+  }
   const GemmPlan p = plan_of(g);
   if (g.glu && !(g.N == 2 * g.glu && g.glu % 16 == 0 && g.nseg == 1 && g.split == 1 && g.glu16 &&
                  g.gu16 && p.kind != GK_NT)) {

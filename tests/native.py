@@ -4,6 +4,7 @@ that no C entry point reaches alone."""
 import ctypes as C
 
 vp, i32, i64, f32 = C.c_void_p, C.c_int, C.c_longlong, C.c_float
+HIP_ERROR_INVALID_VALUE = 1
 
 
 def _struct(name, fields):
@@ -39,3 +40,9 @@ def norm_bwd(L, args, T, stream=None):
     f = fn(L, "_ZN4llmt8norm_bwdERKNS_11NormBwdArgsEiP12ihipStream_t", i32,
            C.POINTER(NormBwdArgs), i32, vp)
     return f(C.byref(args), T, stream)
+
+
+def gemm_nt(L, args, stream=None):
+    """hipError_t of llmt::gemm_nt(const GemmArgs&, hipStream_t)."""
+    f = fn(L, "_ZN4llmt7gemm_ntERKNS_8GemmArgsEP12ihipStream_t", i32, C.POINTER(GemmArgs), vp)
+    return f(C.byref(args), stream)

@@ -1,9 +1,16 @@
 """CPU: the host-side rules that choose a kernel, through the library's
 exported functions (no GPU work)."""
+import ctypes as C
+
 import pytest
+import torch
 
 import llmt
 import native
+
+# calls that must be refused, with addresses that are never read: only where
+# a call that is not refused has no device to launch on
+no_gpu = pytest.mark.skipif(torch.cuda.is_available(), reason="runs without a GPU only")
 
 
 def test_attention_forward_split_is_bounded_by_its_workgroups():
@@ -35,3 +42,41 @@ def test_attention_backward_split_lines():
     assert [f(1, s, 6, 2) for s in (768, 1456, 1457, 7008, 7009)] == [1, 1, 2, 2, 0]
     assert [f(1, s, 16, 8) for s in (16, 416, 417, 2048, 2049)] == [1, 1, 2, 2, 0]
     assert [f(1, s, 32, 8) for s in (128, 768, 769)] == [1, 1, 0]
+
+
+def _gemm(M, N, K, i8=False, split=1, A=0x10000, **kw):
+    """Arguments of a GEMM of one segment (addresses that are never read)."""
+    g = native.GemmArgs()
+    g.A, g.lda, g.nseg, g.M, g.N, g.K, g.split = A, K, 1, M, N, K, split
+    g.seg[0].ptr, g.seg[0].rows, g.seg[0].ld, g.seg[0].is_i8 = 0x20000, N, K, i8
+    for i in range(1, 5):
+        g.seg_start[i] = N
+    g.C, g.ldc = 0x30000, N
+    for k, v in kw.items():
+        setattr(g, k, v)
+    return g
+
+
+@no_gpu
+@pytest.mark.parametrize("i8", [False, True])
+@pytest.mark.parametrize("M", [16, 128, 512, 1040, 4096])
+def test_swiglu_gemm_refuses_a_per_k_scale(M, i8):
+    """No SwiGLU epilogue applies a per-k scale, whatever tile the plan takes:
+    such a GEMM is refused before any launch, not computed without the scale."""
+    L = llmt.lib()
+    g = _gemm(M, 12288, 2048, i8, glu=6144, glu16=0x40000, ldglu=6144, gu16=0x50000)
+    g.seg[0].kscale = 0x60000
+    assert native.gemm_nt(L, g) == native.HIP_ERROR_INVALID_VALUE
+    assert "per-k scale" in L.llmt_last_error().decode()
+
+
+@no_gpu
+@pytest.mark.parametrize("M", [16, 128, 512, 4096])
+@pytest.mark.parametrize("field", ["kscale", "colscale"])
+def test_gemm_refuses_a_scale_on_fp16_rows(M, field):
+    """The scales are int8 rows': on fp16 rows no kernel but one applied them."""
+    L = llmt.lib()
+    g = _gemm(M, 2048, 2048)
+    setattr(g.seg[0], field, 0x60000)
+    assert native.gemm_nt(L, g) == native.HIP_ERROR_INVALID_VALUE
+    assert "scale" in L.llmt_last_error().decode()
