@@ -1429,11 +1429,11 @@ static bool ring_segments(const GemmArgs& g) {
 static GemmPlan plan_of(const GemmArgs& g) {
   const GemmPlan nt{GK_NT, 0, 0, g.split};
   if (g.K % 64 || g.split > g.K / 64) return nt;
+  if (g.split_col) return {GK_BIG, 16, 16, g.split};  // planned as 256 x 256 tiles, unsplit
   const bool i8 = g.seg[0].is_i8;
   if (!i8 && g.M % 128 == 0 && skinny_stages() == 0 && !g.glu) return nt;
   const int need = g.glu ? GN_GLU : g.rowstats ? GN_STATS : GN_PLAIN;
   GemmPlan p = gemm_plan(g.M, g.N, g.K, i8, need, g.split, g.split);
-  if (g.split_col) p = {GK_BIG, 16, 16, g.split};  // planned as 256 x 256 tiles, unsplit
   if (p.kind == GK_BIG && !big_segments(g)) p = {GK_RING, 8, 8, g.split};
   if (p.kind == GK_RING && !ring_segments(g)) return nt;
   return p;
@@ -1452,8 +1452,11 @@ int gemm_rowstats_tiles(const GemmArgs& g) {
 // The last wave of an unsplit 256 x 256-tile GEMM: with tiles = full waves of
 // the 256 CUs plus r more (r <= 128, whole column tiles), the last r tiles
 // run as 2 r half-K workgroups, so the launch takes 1 + 1/2 wave-times of a
-// tile instead of 2 (the down-projection dX of 4096 rows: 384 tiles).  Their
-// partial is an extra fp32 [M, r/ntm x 256] the consumer reads back.
+// tile instead of 2.  Their partial is an extra fp32 [M, r/ntm x 256] the
+// consumer reads back.  (The plan takes 128 x 256 ring tiles for the
+// down-projection dX of hidden 2048, intermediate 6144; the split is reached
+// at other widths, for instance hidden 512, intermediate 4352, 8192 rows: 544
+// tiles.)
 int gemm_split_col(int M, int N, int K, bool i8) {
   if (N % 256 || K % 64 || K / 64 < 8) return 0;
   const GemmPlan p = gemm_plan(M, N, K, i8, GN_PLAIN, 0, 64);

@@ -46,3 +46,14 @@ def gemm_nt(L, args, stream=None):
     """hipError_t of llmt::gemm_nt(const GemmArgs&, hipStream_t)."""
     f = fn(L, "_ZN4llmt7gemm_ntERKNS_8GemmArgsEP12ihipStream_t", i32, C.POINTER(GemmArgs), vp)
     return f(C.byref(args), stream)
+
+
+def gemm_kernel_name(L, args):
+    """Name of the kernel gemm_nt launches for these arguments."""
+    f = fn(L, "_ZN4llmt16gemm_kernel_nameERKNS_8GemmArgsE", C.c_char_p, C.POINTER(GemmArgs))
+    return f(C.byref(args)).decode()
+
+
+def gemm_split_col(L, M, N, K, i8):
+    f = fn(L, "_ZN4llmt14gemm_split_colEiiib", i32, i32, i32, i32, C.c_bool)
+    return f(M, N, K, i8)

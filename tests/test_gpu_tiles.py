@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import llmt
+import native
 from helpers import grad_errors, rel_l2
 from oracle import lora_step as ref
 from oracle.configs import make_adapters, make_layer
@@ -107,6 +108,31 @@ def test_head_row_tiles(dev, T):
         ctx.close()
 
 
+def _small_layer_matches_oracle(dev, d, B, S, **adapter_kw):
+    """Forward, dx and adapter gradients of one fp16 layer."""
+    T = B * S
+    g = torch.Generator().manual_seed(T)
+    lw = make_layer(g, d)
+    ad = make_adapters(g, d, **adapter_kw)[0]
+    x, dy = torch.randn(T, d.hidden, generator=g), torch.randn(T, d.hidden, generator=g)
+    f = lambda t: t.to(torch.float32).to(dev).contiguous()
+    cos, sin = ref.rope_tables(S, d.head_dim, d.theta)
+    y_ref, st = ref.layer_forward(x, lw, ad, d, B, S, cos, sin)
+    dx_ref, grads_ref = ref.layer_backward(dy, st, lw, ad, d, B, S, cos, sin)
+    ctx = llmt.Context(llmt.make_dims(d), B, S)
+    try:
+        ctx.set_layer_f16(0, *(getattr(lw, n).half().to(dev).contiguous() for n in
+                               ("wq", "wk", "wv", "wo", "w_gate", "w_up", "w_down")),
+                          f(lw.attn_norm), f(lw.ffn_norm), f(lw.q_norm), f(lw.k_norm))
+        ctx.lora_set("param", llmt.flatten_adapters([ad]).to(dev))
+        assert rel_l2(ctx.layer_forward(0, x.to(dev), B).cpu(), y_ref) < GRAD_TOL
+        assert rel_l2(ctx.layer_backward(0, dy.to(dev), B).cpu(), dx_ref) < GRAD_TOL
+        errs = grad_errors(ctx.lora_get("grad"), [grads_ref], d)
+        assert max(errs.values()) < GRAD_TOL
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("T", [16, 272, 528, 784])
 def test_layer_row_epilogues_at_row_counts(dev, T):
     """One small layer at token counts on both sides of the row epilogues'
@@ -116,26 +142,19 @@ def test_layer_row_epilogues_at_row_counts(dev, T):
     print(f"case: row epilogues T{T}", flush=True)
     d = ref.Dims(**{**ref.QWEN3_1_7B.__dict__, "n_layers": 1, "vocab": 256, "hidden": 512,
                     "intermediate": 512, "n_heads": 4, "n_kv_heads": 2})
-    g = torch.Generator().manual_seed(T)
-    lw = make_layer(g, d)
-    ad = make_adapters(g, d, b_std=0.5)[0]
-    x, dy = torch.randn(T, d.hidden, generator=g), torch.randn(T, d.hidden, generator=g)
-    f = lambda t: t.to(torch.float32).to(dev).contiguous()
-    cos, sin = ref.rope_tables(T, d.head_dim, d.theta)
-    y_ref, st = ref.layer_forward(x, lw, ad, d, 1, T, cos, sin)
-    dx_ref, grads_ref = ref.layer_backward(dy, st, lw, ad, d, 1, T, cos, sin)
-    ctx = llmt.Context(llmt.make_dims(d), 1, T)
-    try:
-        ctx.set_layer_f16(0, *(getattr(lw, n).half().to(dev).contiguous() for n in
-                               ("wq", "wk", "wv", "wo", "w_gate", "w_up", "w_down")),
-                          f(lw.attn_norm), f(lw.ffn_norm), f(lw.q_norm), f(lw.k_norm))
-        ctx.lora_set("param", llmt.flatten_adapters([ad]).to(dev))
-        assert rel_l2(ctx.layer_forward(0, x.to(dev), 1).cpu(), y_ref) < GRAD_TOL
-        assert rel_l2(ctx.layer_backward(0, dy.to(dev), 1).cpu(), dx_ref) < GRAD_TOL
-        errs = grad_errors(ctx.lora_get("grad"), [grads_ref], d)
-        assert max(errs.values()) < GRAD_TOL
-    finally:
-        ctx.close()
+    _small_layer_matches_oracle(dev, d, 1, T, b_std=0.5)
+
+
+@pytest.mark.parametrize("S", [500, 512])
+def test_layer_last_wave_split(dev, L, S):
+    """A layer whose down-projection dX (N = intermediate, K = hidden) ends in a
+    partial wave of 256 x 256 tiles, which the plan then splits over K: whole
+    and ragged row blocks, read by the SwiGLU backward."""
+    print(f"case: last-wave split B16 S{S}", flush=True)
+    d = ref.Dims(**{**ref.QWEN3_1_7B.__dict__, "n_layers": 1, "vocab": 256, "hidden": 512,
+                    "intermediate": 4352, "n_heads": 2, "n_kv_heads": 1})
+    assert 0 < native.gemm_split_col(L, 16 * S, d.intermediate, d.hidden, False) < d.intermediate
+    _small_layer_matches_oracle(dev, d, 16, S)
 
 
 @pytest.mark.parametrize("T,H", [(16, 512), (48, 2048), (32, 2112)])

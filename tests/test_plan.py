@@ -80,3 +80,17 @@ def test_gemm_refuses_a_scale_on_fp16_rows(M, field):
     setattr(g.seg[0], field, 0x60000)
     assert native.gemm_nt(L, g) == native.HIP_ERROR_INVALID_VALUE
     assert "scale" in L.llmt_last_error().decode()
+
+
+@pytest.mark.parametrize("stages", ["", "0"])
+def test_split_col_gemm_keeps_its_kernel(monkeypatch, stages):
+    """A GEMM whose last tiles are split runs on the 256 x 256 tiles, also where
+    the override takes other fp16 GEMMs of M % 128 == 0 to the register-staged
+    kernel (which cannot split single tiles: the GEMM would be refused)."""
+    monkeypatch.setenv("LLMT_GEMM_SKINNY_STAGES", stages)
+    L = llmt.lib()
+    M, N, K = 4096, 8448, 512
+    col = native.gemm_split_col(L, M, N, K, False)
+    assert 0 < col < N
+    g = _gemm(M, N, K, split=2, split_col=col, split_stride=M * N)
+    assert native.gemm_kernel_name(L, g) == "gemm_dma"
