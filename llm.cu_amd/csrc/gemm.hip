@@ -64,6 +64,9 @@ __device__ __forceinline__ half8 i8x8_to_h8(u32x2 raw) {
   return h - (_Float16)1152.0f;
 }
 
+// Four dwords at any fp16 element (one load all the same).
+typedef u32x4 u32x4_h __attribute__((aligned(2)));
+
 // Register-staged kernel.  One workgroup: output tile (MF*16) x (NW*NF*16)
 // over k-steps [s0, s1) of its split.  The A tile goes through LDS in chunks
 // of CHS k-steps (two LDS buffers); chunk c + ADIST is loaded into registers
@@ -147,7 +150,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(const GemmArgs g) {
         const int q = fr / MF, mi = fr % MF;
         const int r = mi * 16 + (l & 15);
         const int k = min(kb + q * KSTEP + (l >> 4) * 8, g.K - 8);
-        ra[set][i] = *reinterpret_cast<const u32x4*>(g.A + (long long)(m0 + r) * g.lda + k);
+        ra[set][i] = *reinterpret_cast<const u32x4_h*>(g.A + (long long)(m0 + r) * g.lda + k);
       }
     }
   };
@@ -1430,6 +1433,10 @@ static GemmPlan plan_of(const GemmArgs& g) {
   const GemmPlan nt{GK_NT, 0, 0, g.split};
   if (g.K % 64 || g.split > g.K / 64) return nt;
   if (g.split_col) return {GK_BIG, 16, 16, g.split};  // planned as 256 x 256 tiles, unsplit
+  // the LDS-DMA kernels move 16-byte pieces of A's rows; a caller's rows that
+  // start elsewhere (the standalone GEMMs, the head's hidden states) are read
+  // by register loads, which have no such requirement
+  if (((uintptr_t)g.A | (uintptr_t)g.lda * sizeof(_Float16)) % 16 && !g.glu) return nt;
   const bool i8 = g.seg[0].is_i8;
   if (!i8 && g.M % 128 == 0 && skinny_stages() == 0 && !g.glu) return nt;
   const int need = g.glu ? GN_GLU : g.rowstats ? GN_STATS : GN_PLAIN;

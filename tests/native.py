@@ -57,3 +57,8 @@ def gemm_kernel_name(L, args):
 def gemm_split_col(L, M, N, K, i8):
     f = fn(L, "_ZN4llmt14gemm_split_colEiiib", i32, i32, i32, i32, C.c_bool)
     return f(M, N, K, i8)
+
+
+def gemm_rowstats_tiles(L, args):
+    f = fn(L, "_ZN4llmt19gemm_rowstats_tilesERKNS_8GemmArgsE", i32, C.POINTER(GemmArgs))
+    return f(C.byref(args))

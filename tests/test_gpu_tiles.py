@@ -43,6 +43,59 @@ def test_gemm_row_tiles(dev, L, i8, M, N, K):
     assert torch.isfinite(got).all()
 
 
+def _off(t, n=1):
+    """t's values in memory that starts n elements past a 16-byte boundary."""
+    return torch.cat([t.new_zeros(n), t.reshape(-1)])[n:].view(t.shape)
+
+
+@pytest.mark.parametrize("i8", [False, True])
+@pytest.mark.parametrize("M", [16, 48, 96, 128, 1040])
+def test_gemm_unaligned_rows(dev, L, i8, M):
+    """A that does not start on a 16-byte boundary (2, 4 and 8 bytes past it):
+    the register-staged kernel, every row form of it, fp32 sums in its own
+    order against the aligned call."""
+    print(f"case: gemm unaligned i8={i8} M{M}", flush=True)
+    N, K = 176, 320
+    g = torch.Generator().manual_seed(M)
+    A = torch.randn(M, K, generator=g).half().to(dev)
+    if i8:
+        q, sc = quantize_rows((torch.randn(N, K, generator=g) * 0.02).numpy())
+        q, sc = torch.from_numpy(q).to(dev), torch.from_numpy(sc.astype(np.float16)).to(dev)
+        run = lambda a: llmt.gemm_i8(a, q, sc)
+    else:
+        B = (torch.randn(N, K, generator=g) * 0.02).half().to(dev)
+        run = lambda a: llmt.gemm_f16(a, B)
+    want = run(A).cpu()
+    for n in (1, 2, 4):
+        a = _off(A, n)
+        assert a.data_ptr() % 16 == 2 * n
+        assert rel_l2(run(a).cpu(), want) < 1e-5
+
+
+@pytest.mark.parametrize("T", [16, 48, 128, 1040])
+def test_head_unaligned_rows(dev, T):
+    """The head on hidden states off a 16-byte boundary against the aligned
+    call: the same logits up to the order of their sums."""
+    print(f"case: head unaligned T{T}", flush=True)
+    H, V = 512, 2496
+    g = torch.Generator().manual_seed(T)
+    E = (torch.randn(V, H, generator=g) * 0.05).half().to(dev)
+    x = torch.randn(T, H, generator=g).half().to(dev)
+    tgt = torch.randint(0, V, (1, T), generator=g, dtype=torch.int32).to(dev)
+    d = ref.Dims(**{**ref.QWEN3_1_7B.__dict__, "n_layers": 1, "vocab": V, "hidden": H,
+                    "intermediate": 512, "n_heads": 2, "n_kv_heads": 1})
+    ctx = llmt.Context(llmt.make_dims(d), 1, T)
+    try:
+        ctx.set_embed_f16(E, torch.ones(H, device=dev))
+        loss, dl, dx = (t.cpu() if torch.is_tensor(t) else t
+                        for t in ctx.head_ce(x, tgt, want_dlogits=True))
+        loss2, dl2, dx2 = ctx.head_ce(_off(x), tgt, want_dlogits=True)
+        assert abs(loss2 - loss) < 1e-4
+        assert rel_l2(dl2.cpu(), dl) < 1e-4 and rel_l2(dx2.cpu(), dx) < 1e-3
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("int8,B,S", [(False, 1, 16), (False, 1, 80), (False, 3, 208),
                                       (False, 5, 400), (True, 1, 48), (True, 1, 208),
                                       (True, 1, 336), (True, 5, 400)])
@@ -176,9 +229,8 @@ def test_layer_input_alignment(dev, T, H):
                           f(lw.attn_norm), f(lw.ffn_norm), f(lw.q_norm), f(lw.k_norm))
         ctx.lora_set("param", llmt.flatten_adapters([ad]).to(dev))
         x, dy = torch.randn(T, H, generator=g).to(dev), torch.randn(T, H, generator=g).to(dev)
-        off = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(T, H)
         y, dx = ctx.layer_forward(0, x, 1), ctx.layer_backward(0, dy, 1)
-        y2, dx2 = ctx.layer_forward(0, off(x), 1), ctx.layer_backward(0, off(dy), 1)
+        y2, dx2 = ctx.layer_forward(0, _off(x), 1), ctx.layer_backward(0, _off(dy), 1)
         assert rel_l2(y2.cpu(), y.cpu()) < 1e-3 and rel_l2(dx2.cpu(), dx.cpu()) < 1e-3
     finally:
         ctx.close()

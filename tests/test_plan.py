@@ -94,3 +94,21 @@ def test_split_col_gemm_keeps_its_kernel(monkeypatch, stages):
     assert 0 < col < N
     g = _gemm(M, N, K, split=2, split_col=col, split_stride=M * N)
     assert native.gemm_kernel_name(L, g) == "gemm_dma"
+
+
+@pytest.mark.parametrize("i8", [False, True])
+@pytest.mark.parametrize("M", [16, 48, 128, 144, 336, 1024, 1040, 4096])
+@pytest.mark.parametrize("offset", [0, 2, 4, 8, 14])
+def test_gemm_with_unaligned_rows_takes_the_register_kernel(M, offset, i8):
+    """The LDS-DMA kernels move A in 16-byte pieces; rows that are not aligned to
+    them go through the register-staged kernel, with or without statistics."""
+    L = llmt.lib()
+    g = _gemm(M, 4096, 2048, i8, A=0x10000 + offset)
+    assert (native.gemm_kernel_name(L, g) == "gemm_nt") == (offset != 0)
+    if not i8:
+        n = native.gemm_rowstats_tiles(L, g)
+        g.rowstats = 0x70000
+        assert (native.gemm_kernel_name(L, g) == "gemm_nt") == (offset != 0)
+        assert n == native.gemm_rowstats_tiles(L, g) and 0 < n <= 4096 // 128
+    g = _gemm(M, 4096, 2048, i8, lda=2052)
+    assert native.gemm_kernel_name(L, g) == "gemm_nt"
