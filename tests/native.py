@@ -62,3 +62,40 @@ def gemm_split_col(L, M, N, K, i8):
 def gemm_rowstats_tiles(L, args):
     f = fn(L, "_ZN4llmt19gemm_rowstats_tilesERKNS_8GemmArgsE", i32, C.POINTER(GemmArgs))
     return f(C.byref(args))
+
+
+def gemm_plan(L, M, segs, K, glu=0):
+    """(kernel name, split) of a GEMM of the given (rows, int8) segments, planned
+    as the step plans it: the library's own split, or the SwiGLU epilogue.  No
+    address is read."""
+    g = GemmArgs()
+    g.A, g.lda, g.M, g.K, g.nseg, g.split = 0x10000, K, M, K, len(segs), 1
+    n = 0
+    for i, (rows, i8) in enumerate(segs):
+        g.seg[i].ptr, g.seg[i].rows, g.seg[i].ld, g.seg[i].is_i8 = 0x20000, rows, K, i8
+        g.seg_start[i] = n
+        n += rows
+    for i in range(len(segs), 5):
+        g.seg_start[i] = n
+    g.N = g.ldc = n
+    g.C = 0x30000
+    if glu:
+        g.glu = g.ldglu = glu
+        g.glu16, g.gu16 = 0x40000, 0x50000
+    else:
+        pick = fn(L, "_ZN4llmt15gemm_pick_splitEiiiib", i32, i32, i32, i32, i32, C.c_bool)
+        g.split = pick(M, n, K, 64, bool(segs[0][1]))
+    return gemm_kernel_name(L, g), g.split
+
+
+def layer_plan(L, d, T, i8):
+    """The kernels of one layer's eight GEMMs on T tokens, by name: forward qkv,
+    o, gu (gate/up), down; backward dX ddx, gudx, odx, qkvdx."""
+    H, I, r = d.hidden, d.intermediate, 16
+    Q, KV = d.n_heads * 128, d.n_kv_heads * 128
+    NT = Q + 2 * KV
+    shapes = {"qkv": ([(NT, i8), (3 * r, 0)], H, 0), "o": ([(H, i8), (r, 0)], Q, 0),
+              "gu": ([(2 * I, i8)], H, I), "down": ([(H, i8)], I, 0), "ddx": ([(I, i8)], H, 0),
+              "gudx": ([(H, i8)], 2 * I, 0), "odx": ([(Q, i8), (r, 0)], H, 0),
+              "qkvdx": ([(H, i8), (3 * r, 0)], NT, 0)}
+    return {n: gemm_plan(L, T, segs, K, glu)[0] for n, (segs, K, glu) in shapes.items()}

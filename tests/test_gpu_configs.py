@@ -531,6 +531,10 @@ def test_c4_int8_large_tile_full_width_matches_oracle(dev):
     (gemm_dma_kernel with per-row and per-k int8 scales, the fused SwiGLU
     epilogue at N = 2 x 6144, LoRA tail columns, the fp16 logits GEMM) at full
     width with 2 layers; vocabulary 8192 keeps the CPU oracle to seconds."""
+    import native
+    plan = native.layer_plan(llmt.lib(), Q3, 4096, True)
+    assert {n for n, k in plan.items() if k.startswith("gemm_dma")} >= {"qkv", "o", "gu", "odx",
+                                                                       "qkvdx"}, plan
     print("case: C4 T=4096 full width, 2 layers, V 8192, int8", flush=True)
     torch.set_num_threads(16)
     d = ref.Dims(n_layers=2, vocab=8192)
@@ -613,27 +617,40 @@ def test_c4_full_size_properties(dev):
 
 
 # ------------------------------------------------------------------ large-T path
-# T = B x S >= 1024 runs every frozen-weight GEMM on the 256 x 256 tile kernel
-# (fp16 and int8 B operands, LoRA rows in the column tiles, per-row int8
-# scales, the dX GEMMs' per-k scales carried by their operands); checked
-# against the oracle on the small model.
+# The small model at T = 1024 runs its frozen-weight GEMMs on stage-ring tiles.
+# A wider one at T = 4096 runs the Q/K/V, gate/up, down dX and O dX GEMMs on the
+# 256 x 256 tile kernel (fp16 and int8 B operands, LoRA rows in the column
+# tiles, the SwiGLU epilogue, per-row int8 scales, the O dX GEMM's per-k scales
+# in the kernel); both are checked against the oracle.
 
 def _small_dims():
     from helpers import SMALL
     return SMALL
 
 
-@pytest.mark.parametrize("batch,seq", [(2, 64), (4, 256)])
+def _dims_at(batch, seq, int8):
+    """The small model, or past T = 1024 the wider one with its plan checked."""
+    if batch * seq <= 1024:
+        return _small_dims()
+    import native
+    d = ref.Dims(hidden=512, n_layers=2, n_heads=16, n_kv_heads=8, head_dim=128,
+                 intermediate=4096, vocab=2048)
+    plan = native.layer_plan(llmt.lib(), d, batch * seq, int8)
+    assert {n for n, k in plan.items() if k.startswith("gemm_dma")} == {"qkv", "gu", "ddx", "odx"}
+    return d
+
+
+@pytest.mark.parametrize("batch,seq", [(2, 64), (4, 256), (16, 256)])
 def test_int8_zero_scale_channels_match_oracle(dev, batch, seq):
     """int8 weights with output channels whose fp16 scale is 0, in every
     projection: an all-zero row, and (q, k, v, o) a row below 4e-6 whose scale
     rounds to 0 in fp16 while its int8 values do not.  The forward applies the
     scale per output row, the Q/K/V and O dX GEMMs per k, and the down and
     gate/up dX operands carry it per column; the step matches the oracle on
-    the dequantised weights at T = 128 (small-M GEMMs) and T = 1024 (large
-    tiles)."""
+    the dequantised weights at T = 128 and T = 1024 (stage-ring tiles) and T =
+    4096 (256 x 256 tiles)."""
     from oracle.configs import quantize_model_int8
-    d = _small_dims()
+    d = _dims_at(batch, seq, True)
     print(f"case: int8 zero-scale channels, B{batch} S{seq}", flush=True)
     W, ad, tok, tgt, _ = config_model(d, batch=batch, seq_len=seq, seed=1013)
     chans = {"wq": (5, 130), "wk": (3, 70), "wv": (7, 100), "wo": (11, 200),
@@ -688,13 +705,14 @@ def test_int8_wide_qkv_rows_match_oracle(dev):
         ctx.close()
 
 
+@pytest.mark.parametrize("batch", [4, 16])
 @pytest.mark.parametrize("int8", [False, True])
-def test_large_tile_step_matches_oracle(dev, int8):
-    d = _small_dims()
-    print(f"case: small model, B4 S256 (T=1024), int8={int8}", flush=True)
-    W, ad, tok, tgt, qs = config_model(d, batch=4, seq_len=256, seed=1011, int8=int8)
+def test_large_tile_step_matches_oracle(dev, int8, batch):
+    d = _dims_at(batch, 256, int8)
+    print(f"case: hidden {d.hidden}, B{batch} S256 (T={256 * batch}), int8={int8}", flush=True)
+    W, ad, tok, tgt, qs = config_model(d, batch=batch, seq_len=256, seed=1011, int8=int8)
     loss_ref, grads_ref, _ = oracle_grads(W, ad, tok, tgt, d)
-    ctx = llmt.Context(llmt.make_dims(d), 4, 256, int8=int8)
+    ctx = llmt.Context(llmt.make_dims(d), batch, 256, int8=int8)
     try:
         if int8:
             _upload_i8(ctx, W, qs, dev)

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import llmt
+import native
 from helpers import rel_l2
 from oracle import lora_step as ref
 from oracle.quant import quantize_rows
@@ -16,13 +17,16 @@ def _seed(s):
     return torch.Generator().manual_seed(s)
 
 
-# M >= 1024 (a multiple of 256) takes the 256 x 128 tile kernel, including
-# partial last column tiles (2064, 4144 = 4096 + 48).
+# Stage-ring tiles up to 1024 rows; the last three run on the 256 x 256 tiles
+# (asserted below), with partial last column tiles (2064, 4144 = 4096 + 48) and
+# a ragged last row block (2032).
 @pytest.mark.parametrize("M,N,K", [(16, 64, 64), (32, 2064, 2048), (128, 4096 + 48, 2048),
                                    (128, 2048, 6144), (64, 12288, 2048), (256, 1024, 2048),
                                    (128, 2048, 12288), (48, 160, 320), (1024, 2064, 2048),
-                                   (2048, 4096 + 48, 512), (1024, 384, 4096)])
+                                   (1024, 384, 4096), (2048, 4096 + 48, 512),
+                                   (2032, 4096 + 48, 2048), (4096, 2064, 2048)])
 def test_gemm_f16_matches_fp32(dev, L, M, N, K):
+    assert native.gemm_plan(L, M, [(N, 0)], K)[0] == ("gemm_dma" if M >= 2000 else "gemm_ring")
     g = _seed(M * 7 + N + K)
     A = torch.randn(M, K, generator=g).half()
     B = (torch.randn(N, K, generator=g) * 0.02).half()
@@ -76,10 +80,12 @@ def test_gemm_strided_operands(dev, L):
     assert (out[:, 48:] == -7.0).all()
 
 
-@pytest.mark.parametrize("M", [128, 1024])
-def test_gemm_i8_matches_dequant(dev, L, M):
+@pytest.mark.parametrize("M,N,kernel", [(128, 1024, "gemm_ring"), (1024, 1024, "gemm_ring"),
+                                        (4096, 2064, "gemm_dma"), (4080, 2064, "gemm_dma")])
+def test_gemm_i8_matches_dequant(dev, L, M, N, kernel):
     g = _seed(13)
-    N, K = 1024, 2048
+    K = 2048
+    assert native.gemm_plan(L, M, [(N, 1)], K)[0] == kernel
     A = torch.randn(M, K, generator=g).half()
     w = torch.randn(N, K, generator=g) * 0.02
     q, sc = quantize_rows(w.numpy())

@@ -96,12 +96,26 @@ def test_head_unaligned_rows(dev, T):
         ctx.close()
 
 
+DMA_KINDS = {(False, 1040): {"gu"}, (True, 1040): {"gu"}, (True, 1424): {"gudx"},
+             (False, 2000): {"qkv"}, (True, 2000): {"qkv"},
+             (False, 4080): {"qkv", "o", "gu", "gudx", "odx", "qkvdx"},
+             (True, 4080): {"qkv", "o", "gu", "odx", "qkvdx"}}
+
+
 @pytest.mark.parametrize("int8,B,S", [(False, 1, 16), (False, 1, 80), (False, 3, 208),
                                       (False, 5, 400), (True, 1, 48), (True, 1, 208),
-                                      (True, 1, 336), (True, 5, 400)])
-def test_layer_row_tiles_match_oracle(dev, int8, B, S):
+                                      (True, 1, 336), (True, 5, 400), (True, 1, 16),
+                                      (True, 1, 80), (False, 2, 520), (True, 2, 520),
+                                      (True, 2, 712), (False, 8, 510), (True, 8, 510)])
+def test_layer_row_tiles_match_oracle(dev, L, int8, B, S):
+    """From 1040 rows the plan takes 256-row tiles for some of the GEMMs, with
+    ragged last row blocks here; DMA_KINDS says which, so that a case does not
+    quietly come to test another kernel."""
     print(f"case: full-width layer int8={int8} B{B} S{S}", flush=True)
     d = ref.Dims(**{**ref.QWEN3_1_7B.__dict__, "n_layers": 1, "vocab": 256})
+    plan = native.layer_plan(L, d, B * S, int8)
+    assert {n for n, k in plan.items() if k.startswith("gemm_dma")} == DMA_KINDS.get(
+        (int8, B * S), set()), plan
     g = torch.Generator().manual_seed(B * 1000 + S)
     lw = make_layer(g, d)
     ad = make_adapters(g, d)[0]
