@@ -1507,7 +1507,8 @@ int gemm_pick_split(int M, int N, int K, int max_split, bool i8) {
   return split;
 }
 
-template <class C>
+// GLU false: a tile that only plain GEMMs are launched on (the forced ones).
+template <class C, bool GLU = true>
 static hipError_t launch_ring(const GemmArgs& g, hipStream_t st) {
   const int nrb = (g.M + C::MR * 16 - 1) / (C::MR * 16);
   int nct;
@@ -1521,7 +1522,7 @@ static hipError_t launch_ring(const GemmArgs& g, hipStream_t st) {
   }
   const dim3 grid = nrb == 1 ? dim3(g.split, nct) : dim3(nrb * nct * g.split);
   if (g.glu) {
-    if constexpr (C::FC % 2 == 0) {
+    if constexpr (GLU && C::FC % 2 == 0) {
       hipLaunchKernelGGL((gemm_ring_kernel<C, false, true>), grid, dim3(512), 0, st, g, nrb, nct);
       return hipGetLastError();
     }
@@ -1570,13 +1571,13 @@ static hipError_t launch_plan(const GemmArgs& g, const GemmPlan& p, hipStream_t 
 template <int S>
 static hipError_t launch_forced(const GemmArgs& g, int nb, hipStream_t st) {
   switch (nb) {
-    case 2: return launch_ring<RingCfg<S, 8, 2, 4, false>>(g, st);
-    case 3: return launch_ring<RingCfg<S, 8, 3, 4, false>>(g, st);
-    case 4: return launch_ring<RingCfg<S, 8, 4, 4, false>>(g, st);
+    case 2: return launch_ring<RingCfg<S, 8, 2, 4, false>, false>(g, st);
+    case 3: return launch_ring<RingCfg<S, 8, 3, 4, false>, false>(g, st);
+    case 4: return launch_ring<RingCfg<S, 8, 4, 4, false>, false>(g, st);
   }
   if constexpr (S <= 5) {
-    if (nb == 6) return launch_ring<RingCfg<S, 8, 6, 4, false>>(g, st);
-    if (nb == 8) return launch_ring<RingCfg<S, 8, 8, 4, false>>(g, st);
+    if (nb == 6) return launch_ring<RingCfg<S, 8, 6, 4, false>, false>(g, st);
+    if (nb == 8) return launch_ring<RingCfg<S, 8, 8, 4, false>, false>(g, st);
   }
   set_error("gemm_nt: no %d-stage ring of %d fragments", S, nb);
   return hipErrorInvalidValue;

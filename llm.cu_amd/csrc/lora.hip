@@ -443,7 +443,7 @@ hipError_t lora_grad(const LoraGradJob* jobs, const LoraGradPlan& plan, int laye
   };
   if (blocks < 512 && T >= 1024) width(integral_constant<int, 16>());
   else if (blocks < 512 && T >= 64) width(integral_constant<int, 8>());
-  else if (T >= 64) width(integral_constant<int, 4>());
+  else if (T >= 64) go(integral_constant<int, 4>(), integral_constant<int, 8>());
   else width(integral_constant<int, 2>());
   LLMT_LAUNCH_CHECK();
   return hipSuccess;

@@ -936,10 +936,6 @@ __global__ __launch_bounds__(RT) void norm_bwd_kernel(const NormBwdArgs a) {
   }
 }
 
-// norm_bwd for rows of one piece per thread at large T, NR rows a workgroup
-// side by side (as o_post_rows_kernel), with no adapter terms or with three
-// (LORA: the attention norm's q, k, v terms, each over all H columns, whose
-// 48 x 4 values a thread loads once for all its rows).
 // The attention norm's LoRA dx term s (dh_q A_q + dh_k A_k + dh_v A_v) of
 // NR rows on MFMA (16 x 16 x 16 fp16: four rows' dh parts x ranks of one
 // adapter, times ranks x 16 columns): wave w takes columns 256 w .. of the row,
@@ -1039,11 +1035,11 @@ __device__ __forceinline__ void lora_rows_mfma(const NormBwdArgs& a, const float
   }
 }
 
-// LM: 0 no adapter terms, 1 the q/k/v terms on VALU, 2 on MFMA
-// (lora_rows_mfma).
-template <int NR, int LM, bool NT = false>
+// norm_bwd for rows of one piece per thread, NR rows a workgroup side by side
+// (as o_post_rows_kernel), with no adapter terms or (LORA) the attention norm's
+// q, k and v terms, each over all H columns, on MFMA.
+template <int NR, bool LORA, bool NT = false>
 __global__ __launch_bounds__(RT) void norm_bwd_rows_kernel(const NormBwdArgs a, int T) {
-  constexpr bool LORA = LM > 0;
   __shared__ float red[2 * NR * RW];
   __shared__ __attribute__((aligned(16))) float hs[NR][64];
   const int H = a.H;
@@ -1063,7 +1059,7 @@ __global__ __launch_bounds__(RT) void norm_bwd_rows_kernel(const NormBwdArgs a, 
   float4 v[NR], hv[NR];
   load_rows<NR, true>(a.in, t0, T, H, v, hv);
   half4 lb[3][4];
-  if constexpr (LM == 2) lora_mfma_load(a, 0, lb);
+  if constexpr (LORA) lora_mfma_load(a, 0, lb);
   const float4 ww = ld4(a.w + cc);
   const float4 ks4 = a.g16_ks ? ldh4(a.g16_ks + cc) : make_float4(1.f, 1.f, 1.f, 1.f);
 #pragma unroll
@@ -1073,7 +1069,7 @@ __global__ __launch_bounds__(RT) void norm_bwd_rows_kernel(const NormBwdArgs a, 
       *reinterpret_cast<float4*>(a.dh_out + (long long)(t0 + i) * 64 + a.dh_col + 4 * threadIdx.x) =
           mul4(hv[i], rs[i]);
   }
-  if constexpr (LM == 2) {
+  if constexpr (LORA) {
     __shared__ __attribute__((aligned(16))) float lora_out[NR * kLoraLd];
     __syncthreads();
     lora_rows_mfma<NR>(a, hs, lb, lora_out);
@@ -1081,11 +1077,6 @@ __global__ __launch_bounds__(RT) void norm_bwd_rows_kernel(const NormBwdArgs a, 
 #pragma unroll
     for (int i = 0; i < NR; ++i)
       v[i] = add4(v[i], mul4(*reinterpret_cast<const float4*>(&lora_out[i * kLoraLd + cc]), a.in.lscale));
-  } else if constexpr (LM == 1) {
-    LoraRegs<1, 3> L;
-    lora_load<1, 3>(a.in, H, L);
-    __syncthreads();
-    lora_apply_rows<NR, 3>(a.in, hs, L, v);
   }
   float s2[2 * NR];  // dot(d w, x), then sum x^2, of each row
 #pragma unroll
@@ -1849,10 +1840,10 @@ hipError_t norm_bwd(const NormBwdArgs& a, int T, hipStream_t st) {
       ok = am.in.term[q].c0 == 0 && am.in.term[q].n == a.H && am.in.term[q].hidx == q * R;
     if (!ok) am.lora_at = nullptr;
   }
-  // many rows: the VALU LoRA form shares its adapter values over 8 rows; the
-  // MFMA form runs 4, one product's worth (the kernel alone at 4096 rows 41.3
-  // us, 54.5 at 2 rows, 48.4 at 3, 43.5 at 8)
-  const int nr = rows_per_wg(T, P, lora ? (am.lora_at ? 4 : 8) : 2);
+  // many rows: the LoRA form runs 4, one product's worth (the kernel alone at
+  // 4096 rows 41.3 us, 54.5 at 2 rows, 48.4 at 3, 43.5 at 8); terms of another
+  // shape take the one-row kernel
+  const int nr = lora && !am.lora_at ? 1 : rows_per_wg(T, P, lora ? 4 : 2);
   const dim3 g((T + nr - 1) / nr);
   // the stashed x and the incoming residual gradient are read once: past
   // 32 MB a launch (C4: 33.5 MB each) nontemporal (C4 LoRA form 58.4 ->
@@ -1861,16 +1852,10 @@ hipError_t norm_bwd(const NormBwdArgs& a, int T, hipStream_t st) {
   auto rows = [&](auto nr_, auto lora_) {
     constexpr int NR = decltype(nr_)::value;
     constexpr bool LO = decltype(lora_)::value;
-    if (LO && am.lora_at) {
-      if (nt)
-        hipLaunchKernelGGL((norm_bwd_rows_kernel<NR, 2, true>), g, dim3(RT), 0, st, am, T);
-      else
-        hipLaunchKernelGGL((norm_bwd_rows_kernel<NR, 2, false>), g, dim3(RT), 0, st, am, T);
-    } else if (nt) {
-      hipLaunchKernelGGL((norm_bwd_rows_kernel<NR, LO ? 1 : 0, true>), g, dim3(RT), 0, st, am, T);
-    } else {
-      hipLaunchKernelGGL((norm_bwd_rows_kernel<NR, LO ? 1 : 0, false>), g, dim3(RT), 0, st, am, T);
-    }
+    if (nt)
+      hipLaunchKernelGGL((norm_bwd_rows_kernel<NR, LO, true>), g, dim3(RT), 0, st, am, T);
+    else
+      hipLaunchKernelGGL((norm_bwd_rows_kernel<NR, LO, false>), g, dim3(RT), 0, st, am, T);
   };
   using std::integral_constant;
   using T1 = integral_constant<bool, true>;

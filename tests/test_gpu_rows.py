@@ -8,7 +8,7 @@ import native
 pytestmark = pytest.mark.gpu
 
 
-def _norm_bwd_lora(L, dev, T, H, hscale):
+def _norm_bwd_lora(L, dev, T, H, hscale, transposed=True):
     """The attention norm's backward on the LoRA input-gradient term alone (a
     zero GEMM row), (got, want): dh values of size hscale, in the GEMM's units."""
     g = torch.Generator().manual_seed(T + H)
@@ -28,7 +28,8 @@ def _norm_bwd_lora(L, dev, T, H, hscale):
         t = r.term[q]
         t.shr, t.row0, t.kp, t.c0, t.n, t.hidx = p(Ad), 16 * q, H, 0, H, 16 * q
     a.rinv_in, a.gscale, a.dh_out, a.x, a.w, a.eps, a.H = p(rd), 1.0, p(dh), p(xd), p(wd), 1e-6, H
-    a.dres_out, a.g16, a.rinv_out, a.lora_at = p(out), p(g16), p(ro), p(At)
+    a.dres_out, a.g16, a.rinv_out = p(out), p(g16), p(ro)
+    a.lora_at = p(At) if transposed else None
     assert native.norm_bwd(L, a, T) == 0, L.llmt_last_error()
     torch.cuda.synchronize()
     d = 2.0 * (h.double() @ A.double()) * rinv.double()[:, None]
@@ -40,14 +41,16 @@ def _norm_bwd_lora(L, dev, T, H, hscale):
 
 @pytest.mark.parametrize("hscale", [1e-4, 3e3, 1e9])
 @pytest.mark.parametrize("T,H,rows", [(200, 512, ""), (272, 512, ""), (520, 2048, ""),
-                                      (784, 512, ""), (2064, 2048, ""), (49, 528, "8")])
+                                      (784, 512, ""), (2064, 2048, ""), (49, 528, "8"),
+                                      (784, 512, "no copy")])
 def test_norm_bwd_lora_term_is_fp32(dev, L, monkeypatch, T, H, rows, hscale):
     """The LoRA input-gradient term at every rows-a-workgroup count (1, 2, 3
-    and 4 by the token count, 8 by the override), for dh values of any size.  Bound: the 48 products and their sum, the row factor
+    and 4 by the token count, 8 by the override; one without the transposed
+    adapter copy), for dh values of any size.  Bound: the 48 products and their sum, the row factor
     and the few operations after it, each 2^-24: 60 * 2^-24 = 3.6e-6, row by
     row (the rows' factors differ by 2^20)."""
     print(f"case: norm_bwd LoRA term T{T} H{H} rows {rows or 'by T'} dh {hscale:g}", flush=True)
-    monkeypatch.setenv("LLMT_ROWS_PER_WG", rows)
-    got, want = _norm_bwd_lora(L, dev, T, H, hscale)
+    monkeypatch.setenv("LLMT_ROWS_PER_WG", rows if rows.isdigit() else "")
+    got, want = _norm_bwd_lora(L, dev, T, H, hscale, rows != "no copy")
     err = ((got.double() - want).norm(dim=1) / want.norm(dim=1)).max()
     assert float(err) < 3.6e-6
