@@ -559,6 +559,35 @@ __device__ __forceinline__ void load_rows(const RowIn& in, int t0, int T, int n,
   }
 }
 
+// load_rows without h, and with it four h columns of one row: thread 16 i + j
+// (i < NR, j < nh / 4) takes group j of row t0 + i, other threads hold a copy of
+// some group.
+template <int NR>
+__device__ __forceinline__ void load_rows_h(const RowIn& in, int t0, int T, int n, float4 (&v)[NR],
+                                            float4& h) {
+  const int c = 4 * (int)threadIdx.x;
+  const int off = c < n ? c : 0;
+  const int hi = min((int)threadIdx.x >> 4, NR - 1), hj = (int)threadIdx.x & 15;
+  const float* const hrow = in.part + (long long)min(t0 + hi, T - 1) * in.ldp + in.hcol +
+                            4 * (hj < in.nh / 4 ? hj : 0);
+  const float* prow[NR];
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    prow[i] = in.part + (long long)min(t0 + i, T - 1) * in.ldp;
+    v[i] = ld4(prow[i] + off);
+  }
+  h = ld4(hrow);
+  for (int k = 1; k < in.split; ++k) {
+    float4 x[NR];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) x[i] = ld4(prow[i] + (long long)k * in.ss + off);
+    const float4 y = ld4(hrow + (long long)k * in.ss);
+#pragma unroll
+    for (int i = 0; i < NR; ++i) v[i] = add4(v[i], x[i]);
+    h = add4(h, y);
+  }
+}
+
 // load_rows then mid() as one memory round trip, as load_row_then (NR <= 2
 // rows, 4 or 8 splits; load_rows waits for each split before issuing the
 // next).  C2: o_dx_post 6.1 -> 4.6 us (one row, load_row_then), o_post at
@@ -945,14 +974,16 @@ __global__ __launch_bounds__(RT) void norm_bwd_kernel(const NormBwdArgs a) {
 // times 2^11, twice), which hold all 24 bits of every element down to 2^-38
 // of the row's largest; the parts of a row are operand rows 4 i .. 4 i + 2 (a
 // fourth is zero), so one product of 16 operand rows does all three and the
-// lane that owns a row and column gets them as one register quad.  The results
-// go through LDS (row i at out + i kLoraLd, the pad keeping the four rows of a
-// store in different banks) to the thread that owns the column.  The kernel
-// alone, H = 2048, us at 512 / 2000 / 4096 rows: 9.5 / 21.7 / 41.3 (one row a
-// workgroup on VALU 12.9 / 49.0 / 94.2; fp32 products 16 x 16 x 4, a quarter of
-// the rate, 14.9 / 32.0 / 60.1; two fp16 parts under a fixed scale, one product
-// each, 9.0 / 22.8 / 40.0, but dh below 2^-4 lost bits, 1.4e-4 at 1e-4, and
-// above 2^26 overflowed).
+// lane that owns a row and column gets them as one register quad.  The first
+// 16 NR threads split a row's 48 values once for all waves, through LDS.  The
+// results go through LDS (row i at out + i kLoraLd, the pad keeping the four
+// rows of a store in different banks) to the thread that owns the column.  The
+// kernel alone, H = 2048, us at 512 / 2000 / 4096 rows: 8.6 / 20.9 / 38.6 (one
+// row a workgroup on VALU 12.9 / 49.0 / 93.9; every wave splitting for itself
+// 9.5 / 22.0 / 41.7; fp32 products 16 x 16 x 4, a quarter of the rate, 14.9 /
+// 32.0 / 60.1; two fp16 parts under a fixed scale, one product each, 9.0 / 22.6
+// / 41.1, but dh below 2^-4 lost bits, 1.4e-4 at 1e-4, and above 2^26
+// overflowed).
 constexpr float kLoraPart = 2048.0f;  // 2^11: one fp16 part
 constexpr int kLoraLd = 4 * RT + 16;
 
@@ -969,42 +1000,53 @@ __device__ __forceinline__ void lora_mfma_load(const NormBwdArgs& a, int cg, hal
   }
 }
 
-// b: the first 64 columns' operands, loaded by the caller before hs was ready.
+// The parts of NR rows, in LDS: part p of h column c of row i at
+// part[(p * NR + i) * 48 + c], the row's exponent in ex[i].
 template <int NR>
-__device__ __forceinline__ void lora_rows_mfma(const NormBwdArgs& a, const float (*hs)[64],
+struct LoraParts {
+  __attribute__((aligned(16))) _Float16 part[3 * NR * 48];
+  int ex[NR];
+};
+
+// Thread 16 i + j (i < NR, j < 12) splits its four h columns 4 j .. of row i.
+template <int NR>
+__device__ __forceinline__ void lora_split(float4 h, LoraParts<NR>& lp) {
+  const int i = (int)threadIdx.x >> 4, j = (int)threadIdx.x & 15;
+  if (i >= NR) return;  // whole 16-lane groups
+  const int k = 15 - __builtin_amdgcn_frexp_expf(max16(j < 12 ? amax4(h) : 0.f));
+  if (j == 0) lp.ex[i] = k;
+  if (j >= 12) return;
+  const float x[4] = {ldexpf(h.x, k), ldexpf(h.y, k), ldexpf(h.z, k), ldexpf(h.w, k)};
+  half4 p[3];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    p[0][e] = (_Float16)x[e];
+    const float r = (x[e] - (float)p[0][e]) * kLoraPart;
+    p[1][e] = (_Float16)r;
+    p[2][e] = (_Float16)((r - (float)p[1][e]) * kLoraPart);
+  }
+#pragma unroll
+  for (int q = 0; q < 3; ++q) *reinterpret_cast<half4*>(&lp.part[(q * NR + i) * 48 + 4 * j]) = p[q];
+}
+
+// b: the first 64 columns' operands, loaded by the caller before lp was ready.
+template <int NR>
+__device__ __forceinline__ void lora_rows_mfma(const NormBwdArgs& a, const LoraParts<NR>& lp,
                                                half4 (&b)[3][4], float* out) {
   constexpr int NG = (NR + 3) / 4;  // groups of four rows
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int kq = lane >> 4, n = lane & 15, part = n & 3;
   half4 aop[NG][3];
-  int ex[NG];  // row 4 i + kq, which this lane stores, is scaled by 2^ex
+  int ex[NG];  // of row 4 i + kq, which this lane stores
 #pragma unroll
   for (int i = 0; i < NG; ++i) {
     const int row = 4 * i + (n >> 2);
-    float4 h[3];
-    float amax = 0.f;
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      h[q] = row < NR ? *reinterpret_cast<const float4*>(&hs[row][a.in.term[q].hidx + 4 * kq])
-                      : make_float4(0.f, 0.f, 0.f, 0.f);
-      amax = fmaxf(amax, amax4(h[q]));
-    }
-    amax = fmaxf(amax, __shfl_xor(amax, 16));
-    amax = fmaxf(amax, __shfl_xor(amax, 32));
-    const int k = 15 - __builtin_amdgcn_frexp_expf(amax);
-    ex[i] = __shfl(k, 4 * kq);
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const float x[4] = {ldexpf(h[q].x, k), ldexpf(h[q].y, k), ldexpf(h[q].z, k), ldexpf(h[q].w, k)};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const _Float16 p0 = (_Float16)x[e];
-        const float r1 = (x[e] - (float)p0) * kLoraPart;
-        const _Float16 p1 = (_Float16)r1;
-        const _Float16 p2 = (_Float16)((r1 - (float)p1) * kLoraPart);
-        aop[i][q][e] = part == 0 ? p0 : part == 1 ? p1 : part == 2 ? p2 : (_Float16)0.f;
-      }
-    }
+    for (int q = 0; q < 3; ++q)
+      aop[i][q] = part < 3 && row < NR ? *reinterpret_cast<const half4*>(
+                                             &lp.part[(part * NR + row) * 48 + 16 * q + 4 * kq])
+                                       : half4{};
+    ex[i] = lp.ex[min(4 * i + kq, NR - 1)];
   }
   const int H = a.H;
 #pragma unroll
@@ -1041,7 +1083,6 @@ __device__ __forceinline__ void lora_rows_mfma(const NormBwdArgs& a, const float
 template <int NR, bool LORA, bool NT = false>
 __global__ __launch_bounds__(RT) void norm_bwd_rows_kernel(const NormBwdArgs a, int T) {
   __shared__ float red[2 * NR * RW];
-  __shared__ __attribute__((aligned(16))) float hs[NR][64];
   const int H = a.H;
   const int t0 = blockIdx.x * NR;
   const int c = 4 * (int)threadIdx.x;
@@ -1056,28 +1097,37 @@ __global__ __launch_bounds__(RT) void norm_bwd_rows_kernel(const NormBwdArgs a, 
     dr[i] = a.dres_in ? ld4s<NT>(a.dres_in + (long long)t * H + cc) : make_float4(0.f, 0.f, 0.f, 0.f);
     rs[i] = (a.rinv_in ? a.rinv_in[t] : 1.0f) * a.gscale;
   }
-  float4 v[NR], hv[NR];
-  load_rows<NR, true>(a.in, t0, T, H, v, hv);
-  half4 lb[3][4];
-  if constexpr (LORA) lora_mfma_load(a, 0, lb);
-  const float4 ww = ld4(a.w + cc);
-  const float4 ks4 = a.g16_ks ? ldh4(a.g16_ks + cc) : make_float4(1.f, 1.f, 1.f, 1.f);
-#pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    if (LORA) store_h(a.in, hv[i], hs[i]);
-    if ((int)threadIdx.x < a.in.nh / 4 && t0 + i < T)
-      *reinterpret_cast<float4*>(a.dh_out + (long long)(t0 + i) * 64 + a.dh_col + 4 * threadIdx.x) =
-          mul4(hv[i], rs[i]);
-  }
+  float4 v[NR];
   if constexpr (LORA) {
+    __shared__ LoraParts<NR> lp;
     __shared__ __attribute__((aligned(16))) float lora_out[NR * kLoraLd];
+    const int hi = min((int)threadIdx.x >> 4, NR - 1), hj = (int)threadIdx.x & 15;
+    const int ht = min(t0 + hi, T - 1);
+    const float hr = (a.rinv_in ? a.rinv_in[ht] : 1.0f) * a.gscale;
+    float4 h;
+    half4 lb[3][4];
+    load_rows_h<NR>(a.in, t0, T, H, v, h);
+    lora_mfma_load(a, 0, lb);
+    lora_split<NR>(h, lp);
+    if ((int)threadIdx.x < 16 * NR && hj < a.in.nh / 4 && t0 + hi < T)
+      *reinterpret_cast<float4*>(a.dh_out + (long long)ht * 64 + a.dh_col + 4 * hj) = mul4(h, hr);
     __syncthreads();
-    lora_rows_mfma<NR>(a, hs, lb, lora_out);
+    lora_rows_mfma<NR>(a, lp, lb, lora_out);
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < NR; ++i)
       v[i] = add4(v[i], mul4(*reinterpret_cast<const float4*>(&lora_out[i * kLoraLd + cc]), a.in.lscale));
+  } else {
+    float4 hv[NR];
+    load_rows<NR, true>(a.in, t0, T, H, v, hv);
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+      if ((int)threadIdx.x < a.in.nh / 4 && t0 + i < T)
+        *reinterpret_cast<float4*>(a.dh_out + (long long)(t0 + i) * 64 + a.dh_col + 4 * threadIdx.x) =
+            mul4(hv[i], rs[i]);
   }
+  const float4 ww = ld4(a.w + cc);
+  const float4 ks4 = a.g16_ks ? ldh4(a.g16_ks + cc) : make_float4(1.f, 1.f, 1.f, 1.f);
   float s2[2 * NR];  // dot(d w, x), then sum x^2, of each row
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
@@ -1606,13 +1656,13 @@ inline unsigned grid_elems(long long n) {
 // norm's backward) the adapter values.  Up to 768 rows the count that gives
 // every CU one workgroup (a second, partial round of one-row workgroups costs
 // a whole round trip): few rows for few CUs, `small` up to 256 rows, then 2
-// and 3; beyond that what each kernel measured best (us at NR = 1 / 2 / 3 /
-// 4 / 8):
+// and 3; beyond that what each kernel measured best (us at NR = 1, 2, 3, 4; the
+// form with adapters alone, the others in the step):
 //   rows                128               624               2000
 //   resid_norm    3.2 3.7 4.5 5.1    9.0 5.9 5.5 6.0    14.6 13.6 14.5 14.0
 //   o_post        5.8 5.6 6.7 7.7    11.5 8.3 7.4 8.2   19.7 16.1 16.2 14.6
 //   norm_bwd      4.3 6.2 7.6 9.9    15.3 11.8 10.4 11.5  21.8 16.0 17.7 16.9
-//   with adapters 7.5 9.0 10 12      23.4 15.7 12.0 13.9  49.6 27.2 24.9 22.7
+//   with adapters 6.9 7.9 8.7 9.5    18.2 12.6 9.6 10.5   49.0 25.0 23.7 20.8
 // LLMT_ROWS_PER_WG (1, 2, 3, 4 or 8) overrides all of them.
 static int rows_per_wg(int T, int P, int large_t, int small_t = 1) {
   if (P != 1) return 1;
@@ -1835,13 +1885,13 @@ hipError_t norm_bwd(const NormBwdArgs& a, int T, hipStream_t st) {
   // adapter rows 16 q, one piece a thread (H <= 4 RT), [NR][H] fp32 of LDS
   NormBwdArgs am = a;
   if (am.lora_at) {
-    bool ok = lora && am.in.nterm == 3 && a.H <= 4 * RT && a.H % 16 == 0;
+    bool ok = lora && am.in.nterm == 3 && am.in.nh == 3 * R && a.H <= 4 * RT && a.H % 16 == 0;
     for (int q = 0; q < am.in.nterm && ok; ++q)
       ok = am.in.term[q].c0 == 0 && am.in.term[q].n == a.H && am.in.term[q].hidx == q * R;
     if (!ok) am.lora_at = nullptr;
   }
   // many rows: the LoRA form runs 4, one product's worth (the kernel alone at
-  // 4096 rows 41.3 us, 54.5 at 2 rows, 48.4 at 3, 43.5 at 8); terms of another
+  // 4096 rows 38.6 us, 49.4 at 2 rows, 44.4 at 3, 40.5 at 8); terms of another
   // shape take the one-row kernel
   const int nr = lora && !am.lora_at ? 1 : rows_per_wg(T, P, lora ? 4 : 2);
   const dim3 g((T + nr - 1) / nr);

@@ -464,8 +464,7 @@ hipError_t Ctx::layer_bwd(int l, int B) {
   // O projection dX (+ dh_o through the B_o^T rows)
   // (int8: this GEMM and the Q/K/V dX apply the per-k weight scale in the
   // kernel; folded into their operands, the LoRA B^T rows riding in the same
-  // A stream would need B^T / s, and dh, in the operands' units, would grow
-  // by ~1 / s past the fp16 range of the LoRA norm backward's MFMA operand)
+  // A stream would need B^T / s in fp16)
   BSeg so[2] = {wseg(w.woT), hseg(shadow_ptr(l, sh_bt_o), kRank, H)};
   const LoraTerm tbo[1] = {{shadow_rm + (size_t)l * shadow_per_layer + sh_a_o, 0, Q, 0, Q, 0}};
   LLMT_HIP_TRY(gemm(CAT_GEMM_BWD, og16, H, so, 2, T, H, nullptr, 0, &go_));
