@@ -77,7 +77,7 @@ static int gemm_common(const void* A, int lda, const void* B, int ldb, int is_i8
   gemm_finalize_segments(g);
   g.M = M;
   g.K = K;
-  g.split = gemm_pick_split(M, N, K, 64, is_i8 != 0);
+  g.split = gemm_pick_split(M, N, K, 64, is_i8 != 0, true);
   float* part = nullptr;
   if (g.split > 1) {
     API_TRY(hipMallocAsync((void**)&part, (size_t)g.split * M * N * sizeof(float), st));

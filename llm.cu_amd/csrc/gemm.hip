@@ -1365,10 +1365,17 @@ enum { GN_PLAIN = 0, GN_GLU = 1, GN_STATS = 2 };
 
 // The cheapest tile and split (fixed > 0: with that split) of a GEMM.  A
 // consumer reads every partial back (at 5.5 TB/s), and the row epilogues
-// issue 2, 4 or 8 partials as one round trip, other counts as several.
+// issue 2, 4 or 8 partials as one round trip, other counts as several.  In the
+// step that consumer runs anyway; `reduce` says that the sum is a pass of its
+// own that an unsplit GEMM does without (the standalone products): a launch,
+// about 4 us with its gap, and the output written again.  (Planned as in the
+// step, the standalone fp16 product M256 N4096 K2048 took 12.8 + 5.0 us in two
+// parts against 13.2 unsplit, M384 15.1 + 6.6 against 15.4, M128 N14336 K4096
+// 29.1 + 6.7 against 30.7.)
 // N counts a trailing LoRA segment (N % 64 rows); on 256 x 256 tiles it
 // rides along, with int8 weights it has column tiles of its own.
-static GemmPlan gemm_plan(int M, int N, int K, bool i8, int need, int fixed, int max_split) {
+static GemmPlan gemm_plan(int M, int N, int K, bool i8, int need, int fixed, int max_split,
+                          bool reduce = false) {
   GemmPlan best{GK_NT, 0, 0, 0};
   if (K % 64) return best;
   double best_t = 1e300;
@@ -1393,6 +1400,7 @@ static GemmPlan gemm_plan(int M, int N, int K, bool i8, int need, int fixed, int
       const double pm = (double)split * M * N * 1e-6, fill = wg / (256.0 * waves);
       double t = c.launch + waves * (c.wave + st * (c.stage + c.fill * fill)) + c.part * pm;
       t += pm * (4 / 5.5) + (split == 1 || split == 2 || split == 4 || split == 8 ? 0.0 : 0.8);
+      if (reduce && split > 1) t += 4.0 + (double)M * N * 1e-6 * (4 / 5.5);
       if (t < best_t) {
         best_t = t;
         best = {c.kind, c.mr, c.nb, split};
@@ -1487,12 +1495,12 @@ static int forced_nb(int M, int K, bool i8) {
   return env_int("LLMT_GEMM_SKINNY_NB", 0);
 }
 
-int gemm_pick_split(int M, int N, int K, int max_split, bool i8) {
+int gemm_pick_split(int M, int N, int K, int max_split, bool i8, bool reduce) {
   if (const int nb = forced_nb(M, K, i8)) {
     const int s = forced_split(M, N, K, nb);
     return s > max_split ? max_split : s;
   }
-  const GemmPlan p = gemm_plan(M, N, K, i8, GN_PLAIN, 0, max_split);
+  const GemmPlan p = gemm_plan(M, N, K, i8, GN_PLAIN, 0, max_split, reduce);
   if (p.kind != GK_NT) return p.split;
   // the register-staged kernel: about 3/4 of the CUs, four k-steps or more a
   // split

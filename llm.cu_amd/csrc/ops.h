@@ -60,8 +60,9 @@ int gemm_rowstats_tiles(const GemmArgs& g);
 // Fills seg_start/N from seg[0..nseg).
 void gemm_finalize_segments(GemmArgs& g);
 // Split factor for a GEMM of this shape and weight type on this device (>=1,
-// bounded by K); N counts a trailing LoRA segment.
-int gemm_pick_split(int M, int N, int K, int max_split, bool i8);
+// bounded by K); N counts a trailing LoRA segment.  reduce: the split partials
+// are summed by a pass that an unsplit GEMM does without.
+int gemm_pick_split(int M, int N, int K, int max_split, bool i8, bool reduce = false);
 // For a large-tile GEMM planned unsplit whose 256 x 256 tiles end in a
 // partial wave of the CUs: the column where tiles start to be split in two
 // so that the last wave is full (GemmArgs::split_col, with split 2); 0 when

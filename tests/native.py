@@ -64,10 +64,10 @@ def gemm_rowstats_tiles(L, args):
     return f(C.byref(args))
 
 
-def gemm_plan(L, M, segs, K, glu=0):
+def gemm_plan(L, M, segs, K, glu=0, reduce=False):
     """(kernel name, split) of a GEMM of the given (rows, int8) segments, planned
-    as the step plans it: the library's own split, or the SwiGLU epilogue.  No
-    address is read."""
+    as the step plans it (reduce: as the standalone products are): the library's
+    own split, or the SwiGLU epilogue.  No address is read."""
     g = GemmArgs()
     g.A, g.lda, g.M, g.K, g.nseg, g.split = 0x10000, K, M, K, len(segs), 1
     n = 0
@@ -83,8 +83,8 @@ def gemm_plan(L, M, segs, K, glu=0):
         g.glu = g.ldglu = glu
         g.glu16, g.gu16 = 0x40000, 0x50000
     else:
-        pick = fn(L, "_ZN4llmt15gemm_pick_splitEiiiib", i32, i32, i32, i32, i32, C.c_bool)
-        g.split = pick(M, n, K, 64, bool(segs[0][1]))
+        pick = fn(L, "_ZN4llmt15gemm_pick_splitEiiiibb", i32, i32, i32, i32, i32, C.c_bool, C.c_bool)
+        g.split = pick(M, n, K, 64, bool(segs[0][1]), reduce)
     return gemm_kernel_name(L, g), g.split
 
 

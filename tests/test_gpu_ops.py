@@ -18,15 +18,16 @@ def _seed(s):
 
 
 # Stage-ring tiles up to 1024 rows; the last three run on the 256 x 256 tiles
-# (asserted below), with partial last column tiles (2064, 4144 = 4096 + 48) and
-# a ragged last row block (2032).
+# (asserted below), with partial last column tiles (4144 = 4096 + 48) and a
+# ragged last row block (4080).
 @pytest.mark.parametrize("M,N,K", [(16, 64, 64), (32, 2064, 2048), (128, 4096 + 48, 2048),
                                    (128, 2048, 6144), (64, 12288, 2048), (256, 1024, 2048),
                                    (128, 2048, 12288), (48, 160, 320), (1024, 2064, 2048),
                                    (1024, 384, 4096), (2048, 4096 + 48, 512),
-                                   (2032, 4096 + 48, 2048), (4096, 2064, 2048)])
+                                   (4080, 4096 + 48, 1024), (4096, 4096 + 48, 1024)])
 def test_gemm_f16_matches_fp32(dev, L, M, N, K):
-    assert native.gemm_plan(L, M, [(N, 0)], K)[0] == ("gemm_dma" if M >= 2000 else "gemm_ring")
+    assert native.gemm_plan(L, M, [(N, 0)], K, reduce=True)[0] == (
+        "gemm_dma" if M >= 2000 else "gemm_ring")
     g = _seed(M * 7 + N + K)
     A = torch.randn(M, K, generator=g).half()
     B = (torch.randn(N, K, generator=g) * 0.02).half()
@@ -80,12 +81,13 @@ def test_gemm_strided_operands(dev, L):
     assert (out[:, 48:] == -7.0).all()
 
 
-@pytest.mark.parametrize("M,N,kernel", [(128, 1024, "gemm_ring"), (1024, 1024, "gemm_ring"),
-                                        (4096, 2064, "gemm_dma"), (4080, 2064, "gemm_dma")])
-def test_gemm_i8_matches_dequant(dev, L, M, N, kernel):
+@pytest.mark.parametrize("M,N,K,kernel", [(128, 1024, 2048, "gemm_ring"),
+                                          (1024, 1024, 2048, "gemm_ring"),
+                                          (4096, 4144, 1024, "gemm_dma"),
+                                          (4080, 4144, 1024, "gemm_dma")])
+def test_gemm_i8_matches_dequant(dev, L, M, N, K, kernel):
     g = _seed(13)
-    K = 2048
-    assert native.gemm_plan(L, M, [(N, 1)], K)[0] == kernel
+    assert native.gemm_plan(L, M, [(N, 1)], K, reduce=True)[0] == kernel
     A = torch.randn(M, K, generator=g).half()
     w = torch.randn(N, K, generator=g) * 0.02
     q, sc = quantize_rows(w.numpy())

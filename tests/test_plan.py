@@ -112,3 +112,18 @@ def test_gemm_with_unaligned_rows_takes_the_register_kernel(M, offset, i8):
         assert n == native.gemm_rowstats_tiles(L, g) and 0 < n <= 4096 // 128
     g = _gemm(M, 4096, 2048, i8, lda=2052)
     assert native.gemm_kernel_name(L, g) == "gemm_nt"
+
+
+def test_standalone_products_count_their_reduction():
+    """A standalone product split over K pays a second launch that sums the
+    parts, so it is split only where the split saves more than that; in the step
+    the sum is part of a row pass that runs anyway."""
+    L = llmt.lib()
+    split = lambda M, N, K, reduce: native.gemm_plan(L, M, [(N, 0)], K, reduce=reduce)[1]
+    for M, N, K in ((256, 4096, 2048), (384, 4096, 2048), (512, 3072, 3072), (128, 14336, 4096)):
+        assert split(M, N, K, False) > 1 and split(M, N, K, True) == 1, (M, N, K)
+    for M, N, K in ((16, 2048, 6144), (128, 2048, 6144), (128, 1024, 4096), (128, 256, 151936)):
+        assert split(M, N, K, True) > 1, (M, N, K)
+    for M in (16, 48, 128, 512, 1024, 4096):
+        for N, K in ((16, 64), (2048, 2048), (12288, 2048), (4096, 192)):
+            assert split(M, N, K, True) <= split(M, N, K, False)
