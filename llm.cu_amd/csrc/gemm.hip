@@ -14,15 +14,17 @@
 // Kernels.  B operands are stored fragment-packed (packed_index in common.h),
 // so an MFMA fragment of B is one contiguous 1 KB (int8: 512 B) wherever it
 // is read from.
-//   gemm_ring_kernel  M up to about a thousand rows, any M % 16 == 0: 16 MR x
-//                     16 NB tiles fed by LDS DMA, K split over workgroups so
+//   gemm_ring_kernel  any M % 16 == 0, all row counts where the plan finds it
+//                     cheaper (below 512 always): 16 MR x 16 NB tiles fed by
+//                     LDS DMA, K split over workgroups so
 //                     that a launch fills the CUs; the fp32 split partials
 //                     are summed in split order by the consuming row
 //                     epilogue (deterministic), and the standalone GEMM entry
 //                     points reduce them with reduce_lora
 //   gemm_dma_kernel   many rows: 256 x 256 tiles
 //   gemm_nt_kernel    what the two do not take (K % 64 != 0, several int8
-//                     segments): B streamed into registers, A through LDS
+//                     segments, rows of A off a 16-byte boundary): B streamed
+//                     into registers, A through LDS
 // gemm_plan picks the kernel, the tile and the split from a cost model.
 #include <math.h>
 #include <stdlib.h>
@@ -638,9 +640,10 @@ __global__ __launch_bounds__(WNN * 128) void gemm_dma_kernel(const GemmArgs g, i
   }
 }
 
-// Stage-ring kernel: M up to about a thousand rows (a training step of one to
-// a few sequences), fp16 or int8 weights, any M % 16 == 0.  A workgroup of
-// eight waves owns 16 MR rows x 16 NB columns, K split over workgroups.
+// Stage-ring kernel: fp16 or int8 weights, any M % 16 == 0 (every GEMM of a
+// step of one to a few sequences; of 4096 rows those whose last round of 256 x
+// 256 tiles is badly filled).  A workgroup of eight waves owns 16 MR rows x
+// 16 NB columns, K split over workgroups.
 //
 // What bounds it: up to M = 128 the weight stream and the fixed costs of a
 // launch (about 5 us: the first round trip, the partial stores), above that
@@ -1331,7 +1334,9 @@ static int skinny_stages() { return env_int("LLMT_GEMM_SKINNY_STAGES", 4); }
 // workgroup.  Fitted on MI355X to 4,800 timings of the layer GEMMs of
 // Qwen3-1.7B (M = 16 .. 4096, cold random operands): mean error 4%, and the
 // tile and split picked from the model cost 0.6% over the best measured ones
-// on average, 7% at worst.
+// on average, 7% at worst.  The logits GEMM is outside of that: several rounds
+// of column tiles that do not run in step, and the statistics (128 rows: 112 us
+// modelled, 162-170 measured; the pick is within 1% of the best in the head).
 enum { GK_NT = 0, GK_RING = 1, GK_BIG = 2 };
 struct TileCost {
   int kind, i8, mr, nb;
