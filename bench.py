@@ -1,6 +1,6 @@
 """Benchmark: LoRA fwd + fused CE + bwd + AdamW tokens/s on one MI355X.
 
-Default workload is config C2 of BASELINE.json: Qwen3-1.7B (28 layers, random
+Default workload is C2: a LoRA training step of Qwen3-1.7B (28 layers, random
 fp16 frozen weights N(0, 0.02), norms 1), rank-16 LoRA on Q/K/V/O, batch 1,
 seq 128, token ids uniform over the vocabulary, next-token targets.  The step
 runs as one captured HIP graph of libllmt.so kernels (llmt_step); inputs are
@@ -491,7 +491,7 @@ BANDWIDTH_KINDS = ("adamw", "swiglu_bwd", "norm_bwd", "cross_entropy")
 
 
 def bandwidth_kernels(kinds):
-    """The bandwidth-bound kernels of the step (north star: >= 70% of HBM):
+    """The bandwidth-bound kernels of the step (the bar: >= 70% of HBM):
     each kernel's bytes per launch as the library records them
     (llmt_profile_kernels: what the kernel's interface reads and writes in
     the dtypes it uses, split-K partials included), divided by its average

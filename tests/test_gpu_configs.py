@@ -1,7 +1,7 @@
-"""GPU parity of the benchmark configurations C0-C4 (BASELINE.json) against the
+"""GPU parity of the benchmark configurations C0-C4 against the
 exact fp32 CPU oracle, through the C ABI.
 
-Tolerances (north star): loss within 1e-3 absolute; every gradient tensor
+Tolerances: loss within 1e-3 absolute; every gradient tensor
 within 1e-2 relative L2; integer work bit-exact.  C2 is checked at full size
 (28 layers, vocabulary 151936, batch 1 x seq 128); C4 at full width with
 2 layers and B2 x S256 against the oracle, and at full size through

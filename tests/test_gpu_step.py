@@ -1,7 +1,7 @@
 """GPU parity of the whole LoRA training step (llmt_forward_backward /
 llmt_step through the C ABI) against the exact fp32 CPU oracle.
 
-Bars (north star): loss within 1e-3 absolute; every adapter-gradient tensor
+Bars: loss within 1e-3 absolute; every adapter-gradient tensor
 within 1e-2 relative L2 of the fp32 reference; integer work bit-exact."""
 import pytest
 import torch
